@@ -108,6 +108,13 @@ HKX_DEV uint32_t f32_to_e4m3(float x) {
   return sign | code;
 }
 
+// Four floats within +-448 to packed e4m3 bytes, round to nearest even (v_cvt_pk_fp8_f32, the
+// OCP format on gfx950; two values an instruction against about 15 to build a code by hand).
+HKX_DEV uint32_t cvt_e4m3x4(float a, float b, float c, float d) {
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
+}
+
 HKX_DEV uint32_t f32_to_i8(float x) {
   float r = __builtin_rintf(x);
   r = __builtin_fminf(__builtin_fmaxf(r, -128.0f), 127.0f);

@@ -120,3 +120,24 @@ def _vllm_op(V, m, n, k):
     assert V.PATCH.stats["hk"] == before + 1
     xq, xs = O.mx_quant(x)
     assert O.rel_to_max(out.cpu(), O.mx_gemm(xq, w, xs, rows)) < 5e-3
+
+
+def test_mx_quant_every_code_and_the_special_values():
+    """Every bf16 value against a block whose largest is 448 (so each rounds to its own e4m3
+    code, ties and subnormals included), and infinities and NaN, whose codes are +-448."""
+    v = torch.arange(1 << 16, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    v = v[(v.float().abs() <= 448)].float()
+    v = torch.cat([v, v.new_zeros(-len(v) % 31)]).reshape(-1, 31)
+    x = torch.cat([v, torch.full((len(v), 1), 448.0)], 1).bfloat16()
+    q, s = mxfp8.quant(x.to(DEV))
+    rq, rs = O.mx_quant(x)
+    assert torch.equal(q.cpu().view(torch.uint8), rq.view(torch.uint8)) and torch.equal(s.cpu(), rs)
+    x = torch.zeros(3, 32)
+    x[0, :2] = torch.tensor([float("inf"), -1.0])
+    x[1, :2] = torch.tensor([float("-inf"), 1.0])
+    x[2, :3] = torch.tensor([float("nan"), 448.0, -2.0])
+    q, _ = mxfp8.quant(x.bfloat16().to(DEV))
+    q = q.cpu().view(torch.uint8)
+    # inf / 2^121 clamps to 448; a NaN is left out of the largest value and clamps to -448
+    assert q[0, :2].tolist() == [0x7e, 0x80] and q[1, :2].tolist() == [0xfe, 0x00]
+    assert q[2, :3].tolist() == [0xfe, 0x7e, 0xc0]
