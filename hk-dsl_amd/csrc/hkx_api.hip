@@ -415,6 +415,19 @@ int wave_cut(int m, int n, int outw) {
   return (n / outw / per) * per * outw;
 }
 
+// Whether a paired decode call the stream kernel can take also runs on it. Up to K = 4096
+// (X held in registers) it always does: 1.06-2.4x the blocked kernel at 1536 to 28672 rows of
+// W, M = 1 to 32. Past that X is streamed with every 16-row block, and where those blocks are
+// more than the CUs but at most two a CU, the blocked kernel's 32-row workgroups are one wave
+// and read X half as often: it stays there above M = 16 (8192 x 6144 at M = 24: 24.6 against
+// 27.6 us) or where the last blocks leave CUs idle (6144 x 5120 at M = 8: 16.5 against 17.4);
+// on either side the stream kernel wins (4096 x 8192 at M = 16: 24.3 -> 16.1 us, 12288 x 5120
+// at M = 16: 34.5 -> 26.6, 28672 x 8192 at M = 1: 95.3 -> 78.5).
+bool pair_streams(int m, int n, int k) {
+  const int blocks = (n + 7) / 8, cus = cu_count();
+  return k <= 4096 || blocks <= cus || blocks > 2 * cus || (m <= 16 && blocks > cus * 7 / 4);
+}
+
 hipError_t tile_dispatch(const Plan& p, const hkx::TileArgs& t, bool fp8, int mode, dim3 grid,
                          hipStream_t s) {
   const int bm = p.tile_m, bn = p.tile_n;
@@ -718,14 +731,17 @@ int hkx_gemm(const HkxGemmArgs* args, void* stream) {
       mode = p.pair ? hkx::kDecPair : hkx::kDecOut;
     }
     const int gw = std::min((a.n + 7) / 8, cu_count());
-    if ((p.variant & HKX_DEC_STREAM) && hkx::stream_takes(d, p.splits, p.pair) && hkx::roww_takes(d, gw)) {
+    const bool stream = (p.variant & HKX_DEC_STREAM) && hkx::stream_takes(d, p.splits) &&
+                        (!p.pair || pair_streams(a.m, a.n, a.k));
+    if (stream && !p.pair && hkx::roww_takes(d, gw)) {
       rc = launched(hkx::launch_roww(d, dim3(gw), s), "decode GEMM");
-    } else if ((p.variant & HKX_DEC_STREAM) && hkx::stream_takes(d, p.splits, p.pair) && hkx::rows_takes(d)) {
+    } else if (stream && hkx::rows_takes(d, p.pair)) {
       const dim3 g(std::min((a.n + 3) / 4, cu_count()));
-      rc = launched(hkx::launch_rows(d, g, s), "decode GEMM");
-    } else if ((p.variant & HKX_DEC_STREAM) && hkx::stream_takes(d, p.splits, p.pair)) {
-      const dim3 g(std::min((a.n + 15) / 16, cu_count()));
-      rc = launched(hkx::launch_stream(d, g, s), "decode GEMM");
+      rc = launched(hkx::launch_rows(d, p.pair, g, s), "decode GEMM");
+    } else if (stream) {
+      const int bc = p.pair ? 8 : 16;  // C columns of a 16-row block
+      const dim3 g(std::min((a.n + bc - 1) / bc, cu_count()));
+      rc = launched(hkx::launch_stream(d, p.pair, g, s), "decode GEMM");
     } else {
       rc = launched(hkx::launch_decode(d, p.waves, p.fn, p.mf, mode, grid, s), "decode GEMM");
     }

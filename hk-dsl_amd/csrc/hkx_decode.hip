@@ -58,7 +58,7 @@ static bool stream_fast(const DecodeArgs& a) {
   return true;
 }
 
-bool stream_takes(const DecodeArgs& a, int splits, bool pair) {
+bool stream_takes(const DecodeArgs& a, int splits) {
   const int groups = a.g_total;  // 128-element K groups
   // a tile operand reaches LDS by 4-byte DMA: bf16, fp16 or fp32, rows 4-byte aligned, byte
   // offsets within 32 bits
@@ -71,21 +71,22 @@ bool stream_takes(const DecodeArgs& a, int splits, bool pair) {
   }
   // two 16-token fragments (M 17-32) keep one buffer of partial sums, which needs two chunks
   // a block (K of 2048 and up)
-  return splits == 1 && !pair && groups % 8 == 0 && groups <= 256 &&
+  // (the paired form's two halves of W take the place of one; it has no tile operand)
+  return splits == 1 && groups % 8 == 0 && groups <= 256 &&
          (a.M <= 16 || (a.M <= 32 && groups >= 16));
 }
 
-template <int EPF, int MF>
+template <int EPF, int MF, bool PAIR = false>
 static hipError_t launch_stream_ep(const DecodeArgs& a, dim3 grid, hipStream_t s) {
   const dim3 block(512);
   switch (a.g_total / 8) {
     case 1:
-      if constexpr (MF == 1) { hipLaunchKernelGGL((stream_kernel<1, EPF, MF>), grid, block, 0, s, a); break; }
+      if constexpr (MF == 1) { hipLaunchKernelGGL((stream_kernel<1, EPF, MF, PAIR>), grid, block, 0, s, a); break; }
       return hipErrorInvalidValue;  // (stream_takes sends no such call)
-    case 2: hipLaunchKernelGGL((stream_kernel<2, EPF, MF>), grid, block, 0, s, a); break;
-    case 3: hipLaunchKernelGGL((stream_kernel<3, EPF, MF>), grid, block, 0, s, a); break;
-    case 4: hipLaunchKernelGGL((stream_kernel<4, EPF, MF>), grid, block, 0, s, a); break;
-    default: hipLaunchKernelGGL((stream_kernel<0, EPF, MF>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((stream_kernel<2, EPF, MF, PAIR>), grid, block, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((stream_kernel<3, EPF, MF, PAIR>), grid, block, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((stream_kernel<4, EPF, MF, PAIR>), grid, block, 0, s, a); break;
+    default: hipLaunchKernelGGL((stream_kernel<0, EPF, MF, PAIR>), grid, block, 0, s, a); break;
   }
   return hipGetLastError();
 }
@@ -304,7 +305,11 @@ __global__ void __launch_bounds__(512) rows_kernel(const DecodeArgs p) {
 // workgroup's fills are issued at its start (X, then on wave 0 the bias values, then the
 // chunks in order), chunk j is multiplied once its fills land, and wave 0 sums the waves'
 // quad sums, applies the epilogue and stores after the last.
-template <int CPW>
+//
+// The paired form (PAIR): a chunk's 4 rows are 2 gate rows and the 2 up rows of the same C
+// columns, and wave 0's lanes read both sums of a column: 24576 x 4096 at M = 1 37.6 -> 30.5 us
+// against the blocked kernel it replaced (6.6 TB/s), 4096 x 4096 at M = 3 11.0 -> 7.4.
+template <int CPW, bool PAIR>
 __global__ void __launch_bounds__(512) rowsq_kernel(const DecodeArgs p) {
   constexpr int NW = 8;
   constexpr int CH = 32768;  // a chunk: 4 rows x 8 KB
@@ -314,7 +319,8 @@ __global__ void __launch_bounds__(512) rowsq_kernel(const DecodeArgs p) {
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nck = (p.N + 3) / 4;
+  constexpr int CC = PAIR ? 2 : 4;  // C columns of a chunk
+  const int nck = (p.N + CC - 1) / CC;
   const int c0 = blockIdx.x * CPW;  // this workgroup's first chunk
   if (c0 >= nck) return;
 
@@ -324,12 +330,13 @@ __global__ void __launch_bounds__(512) rowsq_kernel(const DecodeArgs p) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = wave >> 1, P = (wave & 1) * 256 + i * 64 + lane;
-    fv[i] = (uint32_t)r * p.ldb_b + (uint32_t)((P ^ (4 * r + (P >> 7))) << 4);
+    const int wr = PAIR ? (r & 1) + (r >> 1) * p.pair_off : r;  // its row of W past the chunk's first
+    fv[i] = (uint32_t)wr * p.ldb_b + (uint32_t)((P ^ (4 * r + (P >> 7))) << 4);
   }
   // chunks past N (the last workgroup's second) are filled out of range: they read zeros
   // and are never stored, and every wave issues the same loads
   auto fill = [&](int j) {
-    const uint32_t base = c0 + j < nck ? (uint32_t)(c0 + j) * 4u * p.ldb_b : 0x80000000u;
+    const uint32_t base = c0 + j < nck ? (uint32_t)(c0 + j) * CC * p.ldb_b : 0x80000000u;
     uint8_t* slot = ring + j * CH + (wave >> 1) * 8192 + (wave & 1) * 4096;
 #pragma unroll
     for (int i = 0; i < 4; ++i) buf_load16_lds<kNonTemporal>(rw, slot + i * 1024, fv[i] + base, 0);
@@ -355,8 +362,8 @@ __global__ void __launch_bounds__(512) rowsq_kernel(const DecodeArgs p) {
   }
   // wave 0, lane l: the bias of chunk l / 16's row (l / 4) % 4 (bf16, unit stride)
   const int fc = lane >> 4, fr = (lane >> 2) & 3, ftl = lane & 3;
-  const int fn = 4 * (c0 + fc) + fr;
-  const bool f_ok = fc < CPW && c0 + fc < nck && fn < p.N;
+  const int fn = CC * (c0 + fc) + fr;
+  const bool f_ok = fc < CPW && c0 + fc < nck && fn < p.N && (!PAIR || fr < 2);
   // (one buffer load on every lane of every wave, out of range where unused: a load under
   // a branch gets a wait of its own at the branch's end, before the fills)
   const uint16_t bias_w = __builtin_amdgcn_raw_buffer_load_b16(
@@ -416,7 +423,12 @@ __global__ void __launch_bounds__(512) rowsq_kernel(const DecodeArgs p) {
   float v = 0.f;
 #pragma unroll
   for (int w2 = 0; w2 < NW; ++w2) v += *(const float*)(ring + RED + (w2 * CPW + fc) * 64 + (lane & 15) * 4);
-  if (fused) v = act4(e.act, f32x4{v * sc + (ra_vec ? bf16_to_f32(bias_w) + e.cadd : add0), 0.f, 0.f, 0.f}).x;
+  if constexpr (PAIR) {  // rows 2 and 3 of the chunk hold the up sums of rows 0 and 1
+    float u = 0.f;
+#pragma unroll
+    for (int w2 = 0; w2 < NW; ++w2) u += *(const float*)(ring + RED + (w2 * CPW + fc) * 64 + ((lane & 7) + 8) * 4);
+    v = silu(v) * u;
+  } else if (fused) v = act4(e.act, f32x4{v * sc + (ra_vec ? bf16_to_f32(bias_w) + e.cadd : add0), 0.f, 0.f, 0.f}).x;
   if (f_ok && ftl < p.M) {
     const int64_t idx = (int64_t)ftl * p.ldc + fn;
     if (p.c_dt == HKX_BF16) ((uint16_t*)p.c)[idx] = (uint16_t)(pack_bf16x2(v, 0.f) & 0xffffu);
@@ -618,8 +630,17 @@ hipError_t launch_roww(const DecodeArgs& a, dim3 grid, hipStream_t s) {
 // against 156.4; 65536: 75.3 against 82.3, one box) and tie or win at M = 2; from M = 3
 // (two chunks a workgroup, or the persistent kernel) they lose there (151936 at M = 4:
 // 194.2 against 189.5), so those stay at N <= 32768.
-bool rows_takes(const DecodeArgs& a) {
+//
+// Paired (gate and up rows: 2N rows of W): the short workgroups only, at the same M and rows
+// of W; M = 4 past 8192 rows stays on the stream kernel.
+bool rows_takes(const DecodeArgs& a, bool pair) {
   const bool tile = a.ep.form == HKX_EP_FUSED && a.ep.ta.p;
+  if (pair) {
+    const int64_t rows = 2 * (int64_t)a.N;
+    const bool rows_ok = a.M <= 2 ? rows * a.ldb_b < (1LL << 31)
+                                  : a.M == 3 ? rows <= 32768 : a.M == 4 && rows <= 8192;
+    return a.g_total == 32 && rows_ok;
+  }
   const bool n_ok = a.M <= 2 ? (int64_t)a.N * a.ldb_b < (1LL << 31) : a.N <= 32768;
   return a.g_total == 32 && a.M <= 4 && n_ok && stream_fast(a) && !tile;
 }
@@ -631,18 +652,27 @@ bool rows_takes(const DecodeArgs& a) {
 // rotated weights, K = 4096 (persistent -> short, us): N = 12288 M = 1 16.95 -> 16.18, M = 2
 // 17.01 -> 16.65, M = 4 17.15 -> 19.50 (one chunk) / 17.61 (two); N = 28672 M = 1 36.68 ->
 // 34.32; N = 6144 M = 4 10.63 -> 9.93 (two); N = 4096 M = 3 8.07 -> 7.21 (two).
-hipError_t launch_rows(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+hipError_t launch_rows(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s) {
+  if (pair) {
+    const int np = (a.N + 1) / 2;
+    if (a.M <= 2) hipLaunchKernelGGL((rowsq_kernel<1, true>), dim3(np), dim3(512), 0, s, a);
+    else hipLaunchKernelGGL((rowsq_kernel<2, true>), dim3((np + 1) / 2), dim3(512), 0, s, a);
+    return hipGetLastError();
+  }
   const int nck = (a.N + 3) / 4;
   if (a.M <= 2)
-    hipLaunchKernelGGL(rowsq_kernel<1>, dim3(nck), dim3(512), 0, s, a);
+    hipLaunchKernelGGL((rowsq_kernel<1, false>), dim3(nck), dim3(512), 0, s, a);
   else if (a.M == 3 || a.N <= 8192)
-    hipLaunchKernelGGL(rowsq_kernel<2>, dim3((nck + 1) / 2), dim3(512), 0, s, a);
+    hipLaunchKernelGGL((rowsq_kernel<2, false>), dim3((nck + 1) / 2), dim3(512), 0, s, a);
   else
     hipLaunchKernelGGL(rows_kernel, grid, dim3(512), 0, s, a);
   return hipGetLastError();
 }
 
-hipError_t launch_stream(const DecodeArgs& a, dim3 grid, hipStream_t s) {
+hipError_t launch_stream(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s) {
+  if (pair)
+    return a.M > 16 ? launch_stream_ep<kStreamEpFast, 2, true>(a, grid, s)
+                    : launch_stream_ep<kStreamEpFast, 1, true>(a, grid, s);
   if (a.M > 16)
     return stream_fast(a) ? launch_stream_ep<kStreamEpFast, 2>(a, grid, s)
                           : launch_stream_ep<kStreamEpGeneric, 2>(a, grid, s);

@@ -250,9 +250,17 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(const DecodeArgs p) {
 constexpr int kStreamEpFast = 0;
 constexpr int kStreamEpGeneric = 1;
 
-template <int CPB, int EPF, int MF>
+// The paired form (PAIR: C = silu(gate) * up, W's up rows pair_off below its gate rows): a
+// block's 16 rows are the gate and the up rows of 8 columns of C, so both halves of a column
+// meet in wave 0's sums, 32 lanes apart, and the walk, the X loads and the waits are those of
+// a plain GEMM of the same bytes. It replaced the blocked kernel's paired form (each 32-row
+// workgroup loading all of X beside its W, no LDS-DMA stream): 24576 x 4096 at M = 16
+// 41.4 -> 32.4 us (6.2 TB/s), at M = 32 52.5 -> 35.0 (graph replays over rotated weights).
+template <int CPB, int EPF, int MF, bool PAIR = false>
 __global__ void __launch_bounds__(512) stream_kernel(const DecodeArgs p) {
+  static_assert(!PAIR || EPF == 0, "the paired epilogue reads no operand");
   constexpr int NW = 8;
+  constexpr int BC = PAIR ? 8 : 16;  // C columns of a block
   constexpr int CH = 16 * 2048;  // a chunk: 16 rows x 2 KB
   constexpr int NR = 4;          // ring slots
   // then the partial sums: [block parity][wave][fragment][lane], 16 B each -- two parities
@@ -272,7 +280,7 @@ __global__ void __launch_bounds__(512) stream_kernel(const DecodeArgs p) {
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int rf = lane & 15, kq = lane >> 4;
-  const int nb = (p.N + 15) / 16;
+  const int nb = (p.N + BC - 1) / BC;
   const int G = gridDim.x;
   if ((int)blockIdx.x >= nb) return;
   // a workgroup's blocks are consecutive (blocks [bstart, bstart + my_blocks)), and it
@@ -300,11 +308,13 @@ __global__ void __launch_bounds__(512) stream_kernel(const DecodeArgs p) {
   // lane l's 16 bytes land at piece 64 h + l of row r, which holds global piece
   // (64 h + l) ^ (r % 16) of the row's 2 KB. The per-lane part of the address is
   // loop-invariant; the block and the chunk go in the scalar offset.
+  // (paired: waves 0-3 the block's 8 gate rows, waves 4-7 its 8 up rows)
   uint32_t fv[4];
+  const uint32_t pair_b = PAIR && wave >= 4 ? (uint32_t)p.pair_off * p.ldb_b : 0u;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = 2 * wave + (i >> 1), h = i & 1;
-    fv[i] = (uint32_t)r * p.ldb_b + (uint32_t)(((64 * h + lane) ^ r) << 4);
+    fv[i] = (uint32_t)(PAIR ? r & 7 : r) * p.ldb_b + (uint32_t)(((64 * h + lane) ^ r) << 4);
   }
   // With X streamed (CPB = 0) a fill past the last chunk is still issued, out of range (it
   // reads nothing and writes a slot no one reads again: chunk q - 4's, done before the
@@ -321,7 +331,7 @@ __global__ void __launch_bounds__(512) stream_kernel(const DecodeArgs p) {
     const bool live = q < nq;
     const int jb = live ? q / cpb : 0, kc = live ? kchunk(q - jb * cpb) : 0;
     const int bi = block_of(jb);
-    const uint32_t so = live ? __builtin_amdgcn_readfirstlane((uint32_t)bi * 16u * p.ldb_b + (uint32_t)kc * 2048u) : 0u;
+    const uint32_t so = live ? __builtin_amdgcn_readfirstlane((uint32_t)bi * BC * p.ldb_b + pair_b + (uint32_t)kc * 2048u) : 0u;
     const uint32_t oob = live ? 0u : 0x80000000u;
     uint8_t* slot = ring + (q & (NR - 1)) * CH;
 #pragma unroll
@@ -446,7 +456,14 @@ __global__ void __launch_bounds__(512) stream_kernel(const DecodeArgs p) {
     f32x4 sum = __builtin_bit_cast(f32x4, part[0]);
 #pragma unroll
     for (int w2 = 1; w2 < NW; ++w2) sum += __builtin_bit_cast(f32x4, part[w2]);
-    const int m = 16 * f + rf, n = bi * 16 + 4 * kq;
+    const int m = 16 * f + rf, n = bi * BC + 4 * kq;
+    if constexpr (PAIR) {  // lanes 0-31 hold the gate sums of columns n .. n + 3, lane + 32 the up sums
+      f32x4 up;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) up[c] = __shfl_xor(sum[c], 32);
+      if (kq < 2 && m < p.M && n < p.N) store4(p.c, p.c_dt, (int64_t)m * p.ldc + n, silu_mul4(sum, up));
+      continue;
+    }
     if (EPF == kStreamEpFast && fused) {
       const uint8_t* eo = ring + EPV + (j % 3) * 768;
       const f32x4 ra = ra_vec ? unpack_bf16x4(*(const u32x2*)(eo + 512 + 8 * kq))

@@ -61,12 +61,12 @@ hipError_t launch_decode(const DecodeArgs& a, int waves, int fn, int mf, int mod
                          hipStream_t s);
 
 // The streaming decode kernel (stream_kernel): M <= 16, K a multiple of 1024 up to 32768,
-// no split, unpaired.
-bool stream_takes(const DecodeArgs& a, int splits, bool pair);
-hipError_t launch_stream(const DecodeArgs& a, dim3 grid, hipStream_t s);
+// no split, plain or paired (M 17-32 from K = 2048).
+bool stream_takes(const DecodeArgs& a, int splits);
+hipError_t launch_stream(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s);
 // the whole-row decode kernel (K = 4096, M <= 4, N <= 32768), for calls stream_takes accepts
-bool rows_takes(const DecodeArgs& a);
-hipError_t launch_rows(const DecodeArgs& a, dim3 grid, hipStream_t s);
+bool rows_takes(const DecodeArgs& a, bool pair);
+hipError_t launch_rows(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s);
 // the per-wave whole-row decode kernel (K = 1024 with M <= 3, K = 2048 with M <= 2), for calls
 // stream_takes accepts; grid: the workgroups it will be launched with
 bool roww_takes(const DecodeArgs& a, int grid);
