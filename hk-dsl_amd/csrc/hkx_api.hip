@@ -70,6 +70,7 @@ struct Plan {
   // block of rows), and whether this call does (counters given)
   int ncnt;
   bool arrive;
+  bool skinny;  // HKX_KERNEL_AUTO's 8-bit decode kernel (no other field is used)
 };
 
 int cu_count();
@@ -123,6 +124,22 @@ void auto_choose(const HkxGemmArgs* a, int* kernel, int* bm, int* bn, int* split
   int s = 1;
   while (tiles * s * 2 <= 256 && kunits / (s * 2) >= 8) s *= 2;
   *splits = s;
+}
+
+hkx::Fused make_fused(const HkxEpilogue& ep);
+
+// Whether HKX_KERNEL_AUTO runs a call on the 8-bit decode kernel: fp8 e4m3, M <= 32, no
+// epilogue or the dequant form, and a shape where it beats the 64 x 128 tiles (split over K
+// past K = 2048, their shares summed by a second launch). Measured, graph replays over rotated
+// weights, tiles -> decode kernel: 4096 x 4096 at M = 16 10.2 -> 5.9 us, 24576 x 4096 at M = 32
+// 27.0 -> 20.4, 1024 x 8192 at M = 32 10.2 -> 9.5, 8192 x 512 at M = 32 5.6 -> 5.5. Where K is
+// short and the row blocks more than two a CU, the tiles' one launch wins (12288 x 1024: 6.7
+// against 7.2; 32768 x 512: 6.5 against 9.2; 12288 x 2048 at M = 32: 8.6 against 9.3, at M = 16
+// 8.5 against 8.0), so those stay there. hk.ops.gemm_cdna.decode8 is the same rule.
+bool auto_skinny(const HkxGemmArgs* a) {
+  return a->kernel == HKX_KERNEL_AUTO && a->ab_dtype == HKX_FP8E4M3 && a->m <= hkx::kSkinnyM &&
+         (a->n <= 8192 || a->k > 2048 || (a->k >= 1792 && a->m <= 16)) &&
+         (a->ep.form == HKX_EP_NONE || a->ep.form == HKX_EP_FUSED) && hkx::skinny_ep_ok(make_fused(a->ep));
 }
 
 int check_operand(const HkxOperand& o, int i) {
@@ -221,6 +238,15 @@ int make_plan(const HkxGemmArgs* a, Plan* p) {
   int rc = check_epilogue(a->ep);
   if (rc) return rc;
 
+  p->skinny = auto_skinny(a);
+  if (p->skinny) {
+    p->kernel = HKX_KERNEL_AUTO;
+    p->splits = 1;
+    p->via_ws = p->pair = p->arrive = false;
+    p->ws_bytes = 0;
+    p->ncnt = 0;
+    return HKX_OK;
+  }
   int kernel = a->kernel, bm = a->tile_m, bn = a->tile_n, splits = a->splits;
   if (kernel == HKX_KERNEL_AUTO) auto_choose(a, &kernel, &bm, &bn, &splits);
   if (splits < 1) splits = 1;
@@ -566,6 +592,23 @@ int hkx_gemm(const HkxGemmArgs* args, void* stream) {
   const hkx::Fused fused = make_fused(a.ep);
   const bool program = a.ep.form == HKX_EP_PROGRAM;
 
+  if (p.skinny) {
+    hkx::SkinnyArgs d{};
+    d.a = a.a;
+    d.b = a.b;
+    d.c = a.c;
+    d.a_bytes = (uint32_t)((long long)a.m * a.lda);
+    d.b_bytes = (uint32_t)((long long)a.n * a.ldb);
+    d.lda_b = (uint32_t)a.lda;
+    d.ldb_b = (uint32_t)a.ldb;
+    d.ldc = a.ldc;
+    d.M = a.m;
+    d.N = a.n;
+    d.nk = a.k / 128;
+    d.c_dt = a.c_dtype;
+    d.ep = fused;
+    return launched(hkx::launch_skinny(d, false, cu_count(), s), "8-bit decode GEMM");
+  }
   if (p.kernel == HKX_KERNEL_TILE) {
     hkx::TileArgs t{};
     t.ab_fmt = fmt_of(a.ab_dtype);
@@ -795,7 +838,7 @@ int hkx_gemm_noalloc(const HkxGemmArgs* args, void* stream) {
 // the CUs; none where an fp32 share would span 4 GiB. (Shorter splits lost more to the
 // shares' round trip than they gained: K = 1152 and 1280 ran slower split in two.)
 static int mx_splits(int32_t m, int32_t n, int32_t k) {
-  if (m < 1 || n < 1 || k < 128 || k % 128) return 1;
+  if (m < 1 || n < 1 || k < 128 || k % 128 || m <= hkx::kSkinnyM) return 1;
   const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
   const int cu = cu_count();
   if (2 * tiles > cu || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 1;
@@ -859,6 +902,29 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   t.sb_bytes = (uint32_t)((long long)n * sb_ld);
   const int splits = mx_splits(m, n, k);
   const hipStream_t s = (hipStream_t)stream;
+  if (m <= hkx::kSkinnyM) {  // the 8-bit decode kernel takes every such call
+    hkx::SkinnyArgs d{};
+    d.a = a;
+    d.b = b;
+    d.c = c;
+    d.a_bytes = t.a_bytes;
+    d.b_bytes = t.b_bytes;
+    d.lda_b = t.lda_b;
+    d.ldb_b = t.ldb_b;
+    d.ldc = ldc;
+    d.M = m;
+    d.N = n;
+    d.nk = k / 128;
+    d.c_dt = HKX_BF16;
+    d.ep = t.ep;
+    d.sa = sa;
+    d.sb = sb;
+    d.sa_ld = t.sa_ld;
+    d.sb_ld = t.sb_ld;
+    d.sa_bytes = t.sa_bytes;
+    d.sb_bytes = t.sb_bytes;
+    return launched(hkx::launch_skinny(d, true, cu_count(), s), "mx decode GEMM");
+  }
   if (splits == 1) {
     const dim3 g(std::min(t.tiles_m * t.tiles_n, cu_count()));
     // the quadrant kernel (whole-line fills) where it takes the call, else the ring's MX form

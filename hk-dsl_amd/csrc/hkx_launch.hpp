@@ -7,6 +7,7 @@
 
 #include "hkx_decode.hpp"
 #include "hkx_reduce.hpp"
+#include "hkx_skinny.hpp"
 #include "hkx_tile.hpp"
 #include "hkx_tile4.hpp"
 
@@ -56,6 +57,12 @@ hipError_t launch_ring_mx(const TileArgs& a, bool f32_shares, dim3 grid, hipStre
 // MX quantization of bf16 rows (hkx_mx_quant).
 hipError_t launch_mx_quant(const void* x, int64_t ldx, void* q, int64_t ldq, uint8_t* sc,
                            int64_t lds, int m, int k, hipStream_t s);
+
+// The 8-bit decode kernel: M up to kSkinnyM, fp8 e4m3 with the epilogues skinny_ep_ok accepts,
+// or MX.
+constexpr int kSkinnyM = 32;
+bool skinny_ep_ok(const Fused& e);
+hipError_t launch_skinny(SkinnyArgs a, bool mx, int cus, hipStream_t s);
 
 hipError_t launch_decode(const DecodeArgs& a, int waves, int fn, int mf, int mode, dim3 grid,
                          hipStream_t s);

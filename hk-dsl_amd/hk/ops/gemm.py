@@ -116,6 +116,10 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
                          f"({m}, {n})/bfloat16")
     sa, sa_ld = _vec(scale_a, m, "scale_a", a.device)
     sb, sb_ld = _vec(scale_b, n, "scale_b", a.device)
+    # the library's own choice: the 8-bit decode kernel (no tile operand there, so not for
+    # accumulate, and an fp32 out keeps the tiles' sums)
+    decode8 = (code == nat.FP8E4M3 and schedule is None and not fp32_out
+               and gemm_cdna.decode8(m, n, k))
     if code != nat.FP8E4M3:
         name = "t256"   # a pair with e5m2: the ring kernel's generic form
     else:
@@ -138,7 +142,8 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
         keep.append(bb)
         ep.ops[2] = nat.HkxOperand(bb.data_ptr(), nat.ROW, nat.BF16, 1)
         ep.row_add, ep.nops = 2, 3
-    args = nat.gemm_args(a, b, out, kernel=nat.KERNEL_TILE, tile_m=rec["tile_m"],
+    args = nat.gemm_args(a, b, out, kernel=nat.KERNEL_AUTO if decode8 else nat.KERNEL_TILE,
+                         tile_m=rec["tile_m"],
                          tile_n=rec["tile_n"], schedule=nat.SCHEDULES[rec["schedule"]],
                          variant=0 if code != nat.FP8E4M3 else rec.get("variant", 0),
                          splits=rec.get("splits", 1), ep=ep)

@@ -184,6 +184,22 @@ def route(m: int, n: int, k: int, fp8: bool = False) -> str:
     return rule(m, n, k, fp8)
 
 
+#: The most rows the 8-bit decode kernel takes.
+DECODE8_M = 32
+
+
+def decode8(m: int, n: int, k: int) -> bool:
+    """Whether a scaled_mm of e4m3 operands runs on the 8-bit decode kernel
+    (csrc/hkx_skinny.hpp, which the library picks for HKX_KERNEL_AUTO by the same rule) rather
+    than on `route`'s tiles: up to 32 rows, except where K is short and the row blocks are
+    more than two a CU (csrc/hkx_api.hip's auto_skinny has both sides' times), unless a user
+    record names a candidate."""
+    if m > DECODE8_M or not (n <= 8192 or k > 2048 or (k >= 1792 and m <= 16)):
+        return False
+    return not any(key in OVERRIDE and fits(OVERRIDE[key], m, n, k, True)
+                   for key in ((m, n, k), "*"))
+
+
 def resolve(rec: Dict[str, Any], m: int, n: int, k: int, fp8: bool = False) -> Dict[str, Any]:
     """A candidate made concrete for a shape: the decode kernel's split over K (enough
     workgroups for twice the CUs, at least four 128-element groups a split)."""

@@ -196,3 +196,16 @@ def test_fp8_rule_follows_its_sweep(monkeypatch):
     for (m, n, k), name in want.items():
         assert gemm_cdna.route(m, n, k, fp8=True) == name, (m, n, k)
         assert gemm_cdna.fits(name, m, n, k, fp8=True)
+
+
+def test_decode8_rule(monkeypatch):
+    """scaled_mm's 8-bit decode kernel: up to 32 rows but for short K over many row blocks, and
+    a user's record for the call keeps its candidate."""
+    monkeypatch.setattr(gemm_cdna, "OVERRIDE", {})
+    yes = [(1, 6144, 4096), (32, 8192, 512), (16, 24576, 2048), (32, 24576, 2560), (32, 1024, 128)]
+    no = [(33, 6144, 4096), (1, 32768, 512), (32, 24576, 2048), (16, 12288, 1280)]
+    assert all(gemm_cdna.decode8(*c) for c in yes) and not any(gemm_cdna.decode8(*c) for c in no)
+    gemm_cdna.OVERRIDE[(1, 6144, 4096)] = "t128"
+    assert not gemm_cdna.decode8(1, 6144, 4096) and gemm_cdna.decode8(2, 6144, 4096)
+    gemm_cdna.OVERRIDE["*"] = "decode"     # does not take fp8
+    assert gemm_cdna.decode8(2, 6144, 4096)
