@@ -6,14 +6,15 @@
 // * a workgroup owns NB (1-4) blocks of 16 rows of W (one 16 x 16 x 128 MFMA fragment) and its 8
 //   waves cut K between them: in round q of a block wave w takes the 128-byte K-steps
 //   2 (8 q + w) and the next, so a round reads 2 KB of each row, 32 KB in all. Two rounds are
-//   in flight, and two workgroups fit a CU: 128 KB of W in flight a CU. NB is the least that
-//   leaves at most two workgroups a CU, so X is loaded once for all a workgroup's rows;
+//   in flight, and two workgroups fit a CU: 128 KB of W in flight a CU. NB is the most that
+//   keeps two workgroups a CU and the blocks even over the CUs, so X is loaded once for all a
+//   workgroup's rows;
 // * a wave's share of W goes HBM -> LDS by non-temporal 16-byte DMA (4 rows x 256 bytes an
 //   instruction, whole lines) into slots no other wave reads: no barrier until the sums meet;
-// * X and, for MX, both sides' scale dwords go to registers,
-//   issued before the round's fills (after them, each round waited for X: 0.3-1.5 us more). X
-//   is read in whole lines and turned through the slot (see XRegs). Up to K = 4096 (NQ = 1 or 2 rounds a block) X stays in registers for all
-//   the blocks; past that it is streamed with the rounds;
+// * X and, for MX, both sides' scale dwords go to registers, issued before the round's fills
+//   (after them, each round waited for X: 0.3-1.5 us more). X is read in whole lines and
+//   turned through the slot (see XRegs). Up to K = 4096 (NQ = 1 or 2 rounds a block) it stays
+//   in registers for all the blocks; past that it is streamed with the rounds;
 // * K's ragged end and the rows past M and N read zeros through the buffer bounds (a K-step
 //   past the end by an offset past every buffer), whose products are zero;
 // * a block's sums meet in LDS, and wave f finishes the 16 tokens of fragment f under the other

@@ -54,7 +54,8 @@ def capturing() -> bool:
         import torch  # noqa: PLC0415
     except ImportError:
         return False
-    return torch.cuda.is_available() and torch.cuda.is_current_stream_capturing()
+    # (a process that has not initialised CUDA captures nothing; is_available asks the driver)
+    return torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing()
 
 
 def compiling() -> bool:

@@ -231,7 +231,7 @@ def linear(x, weight, bias=None):
     k = x.shape[-1]
     n = weight.shape[0]
     m = x.numel() // k if k else 0
-    key = (m, n, k, x.dtype, weight.dtype, None if bias is None else (bias.dtype, tuple(bias.shape)),
+    key = (m, n, k, x.dtype, weight.dtype, None if bias is None else (bias.dtype, bias.shape),
            _weight_ok(weight), x.get_device())
     plan = ROUTER.plans.get(key)
     if plan is None:
@@ -241,12 +241,12 @@ def linear(x, weight, bias=None):
     if plan.run is None:
         PATCH.count("fallback")
         return _fallback(x, weight, bias)
-    x2 = x.reshape(m, k)
+    x2 = x if x.dim() == 2 else x.reshape(m, k)
     if not x2.is_contiguous() or x2.data_ptr() % 16:
         x2 = x2.clone(memory_format=_contiguous())
     y = plan.run(x2, weight, bias)
     PATCH.count(plan.path)
-    return y.view(*x.shape[:-1], n)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], n)
 
 
 def _contiguous():

@@ -28,16 +28,25 @@ def expand_block_scales(s, block_rows: int = 32):
     return s.repeat_interleave(block_rows, dim=0).contiguous()
 
 
-def _scales(s, rows, k, what):
-    import torch  # noqa: PLC0415
-
+def _scales(torch, s, rows, k, what):
     if s.dtype not in (torch.uint8, torch.int8):
         raise TypeError(f"mxfp8: {what} holds E8M0 bytes (uint8), got {s.dtype}")
-    if s.dim() != 2 or s.shape[0] != rows or s.shape[1] != k // 32:
+    if s.shape != (rows, k // 32):
         raise ValueError(f"mxfp8: {what} is {tuple(s.shape)}, expected ({rows}, {k // 32})")
-    if s.stride(1) != 1 or s.stride(0) % 4 or s.data_ptr() % 4:
+    st = s.stride()
+    if st[1] != 1 or st[0] % 4 or s.data_ptr() % 4:
         s = s.contiguous()
     return s
+
+
+def _rows16(t):
+    """`t` with rows the kernels read in place: unit stride along K, 16-byte aligned."""
+    st = t.stride()
+    return t if st[1] == 1 and st[0] % 16 == 0 and t.data_ptr() % 16 == 0 else t.contiguous()
+
+
+#: (M, N, K) -> the bytes of the workspace its K split needs, asked once a shape.
+_WORKSPACE: dict = {}
 
 
 def gemm(a, b, sa, sb, out=None):
@@ -55,17 +64,20 @@ def gemm(a, b, sa, sb, out=None):
         raise ValueError(f"mxfp8.gemm: K={k} a multiple of 128 and N={n} of 8")
     if not a.is_cuda or b.device != a.device:
         raise ValueError("mxfp8.gemm: a and b are on one GPU")
-    a = a if a.stride(1) == 1 and a.stride(0) % 16 == 0 and a.data_ptr() % 16 == 0 else a.contiguous()
-    b = b if b.stride(1) == 1 and b.stride(0) % 16 == 0 and b.data_ptr() % 16 == 0 else b.contiguous()
-    sa = _scales(sa, m, k, "sa")
-    sb = _scales(sb, n, k, "sb")
+    a, b = _rows16(a), _rows16(b)
+    sa = _scales(torch, sa, m, k, "sa")
+    sb = _scales(torch, sb, n, k, "sb")
     if out is None:
-        out = torch.empty((m, n), device=a.device, dtype=torch.bfloat16)
+        out = a.new_empty((m, n), dtype=torch.bfloat16)
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
         raise ValueError(f"mxfp8.gemm: out is bf16 ({m}, {n}) with unit column stride")
     L = nat.lib()
-    nws = L.hkx_mx_gemm_workspace(m, n, k)
-    ws = nat.workspace(a.device, nws)
+    nws = _WORKSPACE.get((m, n, k))
+    if nws is None:
+        nws = L.hkx_mx_gemm_workspace(m, n, k)
+        if len(_WORKSPACE) < 4096:
+            _WORKSPACE[(m, n, k)] = nws
+    ws = nat.workspace(a.device, nws) if nws else None
     nat.check(L.hkx_mx_gemm(
         a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), sa.data_ptr(), sa.stride(0),
         sb.data_ptr(), sb.stride(0), out.data_ptr(), out.stride(0), m, n, k,
@@ -86,8 +98,8 @@ def quant(x, out=None):
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     q, s = out if out is not None else (
-        torch.empty((m, k), device=x.device, dtype=torch.float8_e4m3fn),
-        torch.empty((m, k // 32), device=x.device, dtype=torch.uint8))
+        x.new_empty((m, k), dtype=torch.float8_e4m3fn),
+        x.new_empty((m, k // 32), dtype=torch.uint8))
     nat.check(nat.lib().hkx_mx_quant(x.data_ptr(), x.stride(0), q.data_ptr(), q.stride(0),
                                      s.data_ptr(), s.stride(0), m, k,
                                      nat.stream_of(x.device)))

@@ -51,6 +51,7 @@ import ctypes
 import hashlib
 import inspect
 import re
+import struct
 import sys
 import types
 import weakref
@@ -542,12 +543,39 @@ def _operand_tensor(name: str, kind: str, v, m: int, n: int):
     return v, v.stride(0)
 
 
+def _in_place(kind: str, v, n: int):
+    """(ld, alignment mask) where `_operand_tensor` passes an operand of this signature on as
+    it is whenever its address is aligned; None where it may convert or copy it."""
+    torch = _torch()
+    if v.dtype not in (torch.bfloat16, torch.float16, torch.float32):
+        return None
+    mask, st = 4 * v.element_size() - 1, v.stride()
+    if kind == COL:
+        return st[0], 0
+    if kind == TILE:
+        return (st[0], mask) if st[1] == 1 and st[0] % 4 == 0 else None
+    if n == 1 or st[-1] not in (0, 1):
+        return None
+    return (0, 0) if st[-1] == 0 else (1, mask)
+
+
+_ARGS = nat.HkxGemmArgs
+_POINTERS = struct.Struct("=QQQqqq")  # a, b, c, lda, ldb, ldc
+_POINTER = struct.Struct("=Q")
+_BUFFER = struct.Struct("=Qq")        # an address and a count
+assert _ARGS.a.offset == 0 and _ARGS.ldc.offset == 40 and nat.HkxOperand.ptr.offset == 0
+
+
 class _Launch:
-    """A call signature made ready: the HkxGemmArgs with everything but the pointers, and
-    how each operand is prepared. `__call__` fills in the pointers and launches."""
+    """A call signature made ready: the bytes of the HkxGemmArgs with everything but the
+    pointers, and how each operand is prepared. `__call__` fills in the pointers of a copy
+    (so calls on several threads do not meet) and launches. What one call costs the host
+    bounds the decode sizes, whose kernels take 5-10 us: filling a ctypes struct field by
+    field, asking the library for the workspace and the torch stream object on every call
+    took 8 of 10 us, and 13 more with one operand."""
 
     def __init__(self, ep: Epilogue, steps: List[Step], m: int, n: int, k: int, out_shape,
-                 out_dtype, fp8: bool):
+                 out_dtype, fp8: bool, operands: Dict[str, Any]):
         self.ep, self.steps, self.m, self.n, self.k = ep, steps, m, n, k
         self.out_shape, self.out_dtype = out_shape, out_dtype
         st = steps[0]
@@ -569,44 +597,61 @@ class _Launch:
             args.variant = s.get("variant", 0)
         args.splits = s.get("splits", 1)
         args.ep = ep.struct()
-        self.args = args
-        self.size = ctypes.sizeof(nat.HkxGemmArgs)
+        #: per operand: (name, kind, offset of its HkxOperand, alignment mask or None)
+        self.operands = []
+        for i, name in enumerate(ep.tensors):
+            kind, v = ep.kinds[name], operands[name]
+            as_is = _in_place(kind, v, out_shape[1])
+            if as_is is not None:
+                args.ep.ops[i].ld = as_is[0]
+                args.ep.ops[i].dtype = nat.dtype_code(v.dtype)
+            at = _ARGS.ep.offset + nat.HkxEpilogue.ops.offset + i * ctypes.sizeof(nat.HkxOperand)
+            self.operands.append((name, kind, at, None if as_is is None else as_is[1]))
+        self.decode = args.kernel == nat.KERNEL_DECODE
+        self.raw = bytes(args)
         self.lib = nat.lib()
-        self.ncnt = None  # arrival counters the plan takes (asked once, at the first call)
+        #: (workspace bytes, arrival counters) of the plan, which the signature decides:
+        #: asked at the first call that launches
+        self.need = None
 
     def __call__(self, a, b, out, operands: Dict[str, Any]):
-        if a.stride(1) != 1 or (a.stride(0) * a.element_size()) % 16 or a.data_ptr() % 16:
+        pa, sa, pb, sb = a.data_ptr(), a.stride(), b.data_ptr(), b.stride()
+        keep = None  # copies that must outlive the launch call
+        if sa[1] != 1 or sa[0] % 8 or pa % 16:
             a = a.contiguous()
-        if b.stride(1) != 1 or (b.stride(0) * b.element_size()) % 16 or b.data_ptr() % 16:
+            pa, sa = a.data_ptr(), a.stride()
+        if sb[1] != 1 or sb[0] % 8 or pb % 16:
             b = b.contiguous()
-        args = nat.HkxGemmArgs()
-        ctypes.memmove(ctypes.addressof(args), ctypes.addressof(self.args), self.size)
-        args.a, args.b, args.c = a.data_ptr(), b.data_ptr(), out.data_ptr()
-        args.lda, args.ldb, args.ldc = a.stride(0), b.stride(0), out.stride(0)
-        keep = []
-        for i, name in enumerate(self.ep.tensors):
-            t, ld = _operand_tensor(name, self.ep.kinds[name], operands[name], self.m,
-                                    self.out_shape[1])
-            keep.append(t)
-            o = args.ep.ops[i]
-            o.ptr, o.dtype, o.ld = t.data_ptr(), nat.dtype_code(t.dtype), ld
-        dev = a.device
-        L = self.lib
-        need = L.hkx_gemm_workspace(ctypes.byref(args))
-        if need:
-            ws = nat.workspace(dev, need)
-            args.ws, args.ws_bytes = ws.data_ptr(), ws.numel() * 4
-        if self.ncnt is None:
+            pb, sb = b.data_ptr(), b.stride()
+        raw = bytearray(self.raw)
+        _POINTERS.pack_into(raw, 0, pa, pb, out.data_ptr(), sa[0], sb[0], out.stride(0))
+        for name, kind, at, mask in self.operands:
+            t = operands[name]
+            p = t.data_ptr()
+            if mask is None or p & mask:
+                t, ld = _operand_tensor(name, kind, t, self.m, self.out_shape[1])
+                keep = (keep, t)
+                o = nat.HkxOperand.from_buffer(raw, at)
+                o.ptr, o.dtype, o.ld = t.data_ptr(), nat.dtype_code(t.dtype), ld
+            else:
+                _POINTER.pack_into(raw, at, p)
+        args = _ARGS.from_buffer(raw)
+        dev, L, need = a.device, self.lib, self.need
+        if need is None:
             # a decode split finishes in the kernel (one launch; measured level with the
             # two-launch form); a tile split keeps its reduction launch (the in-kernel finish
             # of the 4-wave kernel measured 4-10 us slower at M = 16-128)
-            self.ncnt = (L.hkx_gemm_counters(ctypes.byref(args))
-                         if args.kernel == nat.KERNEL_DECODE else 0)
-        if self.ncnt:
-            cnt = nat.counters(dev, self.ncnt)
+            need = (L.hkx_gemm_workspace(args), L.hkx_gemm_counters(args) if self.decode else 0)
+        if need[0]:
+            ws = nat.workspace(dev, need[0])
+            keep = (keep, ws)
+            _BUFFER.pack_into(raw, _ARGS.ws.offset, ws.data_ptr(), ws.numel() * 4)
+        if need[1]:
+            cnt = nat.counters(dev, need[1])
             if cnt is not None:
-                args.counters, args.counters_len = cnt.data_ptr(), cnt.numel()
-        nat.check(L.hkx_gemm(ctypes.byref(args), ctypes.c_void_p(nat.stream_of(dev))))
+                _BUFFER.pack_into(raw, _ARGS.counters.offset, cnt.data_ptr(), cnt.numel())
+        nat.check(L.hkx_gemm(args, nat.stream_of(dev)))
+        self.need = need
         return out
 
 
@@ -618,7 +663,7 @@ _LAUNCH: Dict[Tuple, Any] = {}
 def _sig(item):
     name, v = item
     try:
-        return (name, tuple(v.shape), v.dtype, v.stride())
+        return (name, v.shape, v.dtype, v.stride())
     except AttributeError:
         return (name, type(v), v)
 
@@ -639,10 +684,11 @@ def _identity(acc):
 
 
 def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operands):
-    key = (epilogue, tuple(a.shape), tuple(b.shape), a.dtype, b.dtype,
-           out_dtype if out is None else (tuple(out.shape), out.dtype, out.stride()),
-           a.device, tuple(map(_sig, operands.items())),
-           None if schedule is None else repr(sorted(_sched_record(schedule).items())))
+    key = (epilogue, a.shape, b.shape, a.dtype, b.dtype,
+           out_dtype if out is None else (out.shape, out.dtype, out.stride()),
+           a.device, tuple(map(_sig, operands.items())) if operands else (),
+           schedule if schedule is None or type(schedule) is str
+           else repr(sorted(_sched_record(schedule).items())))
     try:
         got = _LAUNCH[key]
     except KeyError:
@@ -651,7 +697,7 @@ def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operan
         got = _slow(a, b, epilogue, out, out_dtype, operands, schedule)
     go, shape, dtype = got
     if out is None:
-        out = _torch().empty(shape, device=a.device, dtype=dtype)
+        out = a.new_empty(shape, dtype=dtype)
     return go(a, b, out, operands)
 
 
@@ -691,7 +737,7 @@ def _slow(a, b, epilogue, out, out_dtype, operands, schedule=None):
     if paired:
         for st in steps:
             st.cols = (0, cn)
-    go = _Launch(ep, steps, m, cn, k, (m, cn), tdt, fp8=False)
+    go = _Launch(ep, steps, m, cn, k, (m, cn), tdt, fp8=False, operands=operands)
     return go, (m, cn), tdt
 
 

@@ -1,0 +1,68 @@
+"""A second call of a signature only fills in pointers: it must still see what its own tensors
+are -- strides, addresses that need a copy, values -- and refuse what the first would."""
+
+import pytest
+import torch
+
+import hk
+from hk import _native as nat
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+T = hk.templates.gemm
+E4 = torch.float8_e4m3fn
+
+
+def _misaligned(t):
+    """The same values one element past an aligned address."""
+    buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    out = buf[1:].view(t.shape)
+    out.copy_(t)
+    return out
+
+
+@pytest.mark.parametrize("m", [2, 300])
+def test_template_operands(m):
+    g = torch.Generator(device=DEV).manual_seed(m)
+    n, k = 512, 1024
+    x, w = torch.randn(m, k, generator=g, device=DEV).bfloat16(), torch.randn(n, k, generator=g, device=DEV).bfloat16()
+    b, r = torch.randn(n, generator=g, device=DEV).bfloat16(), torch.randn(m, n, generator=g, device=DEV).bfloat16()
+    want = T(x, w, epilogue=T.bias_residual, bias=b, residual=r)
+    wide = torch.zeros(m, k + 64, device=DEV).bfloat16()
+    wide[:, :k] = x
+    for xs, ws, bs, rs in [(x, w, b, r), (x, w, _misaligned(b), r), (wide[:, :k], w, b, r),
+                           (x, w, b.float(), r.float()), (x, w, b, torch.cat([r, r], 1)[:, :n])]:
+        assert torch.equal(T(xs, ws, epilogue=T.bias_residual, bias=bs, residual=rs), want)
+    for xs, ws, rs in [(_misaligned(x), w, r), (x, _misaligned(w), r), (x, w, _misaligned(r))]:
+        with pytest.raises(nat.HkxError, match="aligned"):
+            T(xs, ws, epilogue=T.bias_residual, bias=b, residual=rs)
+    assert not torch.equal(T(x, w, epilogue=T.bias_residual, bias=b + 1, residual=r), want)
+
+
+@pytest.mark.parametrize("m", [2, 64, 300])  # the decode kernel, a split with a workspace, tiles
+def test_scaled_mm_signatures(m):
+    g = torch.Generator(device=DEV).manual_seed(m)
+    n, k = 1024, 8192
+    a, w = (torch.randn(r, k, generator=g, device=DEV).to(E4) for r in (m, n))
+    sa, sb = torch.rand(m, 1, generator=g, device=DEV), torch.rand(n, generator=g, device=DEV)
+    bias = torch.randn(n, generator=g, device=DEV).bfloat16()
+    want = hk.ops.scaled_mm(a, w, sa, sb, bias=bias)
+    wide = torch.zeros(m, k + 64, device=DEV).to(E4)
+    wide[:, :k] = a
+    for s1, s2, x, bs in [(sa, sb, a, bias), (sa, sb, wide[:, :k], bias),
+                          (sa.double(), sb.float(), a, bias.float()),
+                          (sa.expand(m, 2)[:, 0], sb, a, bias)]:
+        assert torch.equal(hk.ops.scaled_mm(x, w, s1, s2, bias=bs), want)
+    out = torch.empty(m, n, device=DEV, dtype=torch.bfloat16)
+    assert hk.ops.scaled_mm(a, w, sa, sb, bias=bias, out=out) is out and torch.equal(out, want)
+    assert torch.equal(hk.ops.scaled_mm(a, w, sa, sb), hk.ops.scaled_mm(a, w, sa, sb))
+    with pytest.raises(ValueError, match="unit stride"):
+        hk.ops.scaled_mm(a.t().contiguous().t(), w, sa, sb, bias=bias)
+    with pytest.raises(nat.HkxError, match="aligned"):
+        hk.ops.scaled_mm(a, w, sa, _misaligned(sb), bias=bias)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        y = hk.ops.scaled_mm(a, w, sa, sb, bias=bias)
+    side.synchronize()
+    assert torch.equal(y, want)
