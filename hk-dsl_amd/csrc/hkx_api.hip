@@ -460,9 +460,10 @@ hipError_t tile_dispatch(const Plan& p, const hkx::TileArgs& t, bool fp8, int mo
   // The ring kernel: one workgroup a CU (a split's share of them) walking its tiles. A call
   // it does not take (an unaligned C, N % 8 != 0, a strided 16-bit column scale) runs on
   // the ping-pong kernel, which takes every 256 x 256 call.
-  if (t.ab_fmt > 1) {  // e5m2 pairs: the ring kernel only (make_plan and hkx_gemm checked)
+  if (t.ab_fmt > 1) {  // e5m2 pairs: 256 x 256 ring tiles (make_plan and hkx_gemm checked)
     dim3 g = grid;
     g.x = std::min<unsigned>(g.x, (unsigned)std::max(1, cu_count() / (int)grid.y));
+    if (grid.y == 1 && hkx::quad_takes(t, fp8, mode)) return hkx::launch_quad(t, fp8, mode, g, s);
     return hkx::launch_ring(t, fp8, mode, g, s);
   }
   if (p.schedule == HKX_TILE_RING && bm == 128) {  // the 128-row quadrant form, or the 4-wave kernel

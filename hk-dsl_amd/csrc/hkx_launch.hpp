@@ -49,6 +49,9 @@ bool quad_takes(const TileArgs& a, bool fp8, int mode);
 bool quad128_takes(const TileArgs& a, bool fp8, int mode);
 hipError_t launch_quad128(const TileArgs& a, int mode, dim3 grid, hipStream_t s);
 hipError_t launch_quad(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s);
+// Its fp8 forms with e5m2 operands (a.ab_fmt 2-4, the dequant forms) and with an fp32 C
+// (kEpDeqAcc), by compiled form.
+hipError_t launch_quad_fmt(const TileArgs& a, int epf, dim3 grid, hipStream_t s);
 // Its MX form (fp8 operands, E8M0 block scales in a.sa / a.sb, bf16 C, one pass).
 hipError_t launch_quad_mx(const TileArgs& a, dim3 grid, hipStream_t s);
 // The MX form (fp8 operands, E8M0 block scales in a.sa / a.sb), no epilogue: bf16 C, or

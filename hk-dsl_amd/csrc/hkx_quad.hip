@@ -15,8 +15,23 @@ bool one32(const Opnd& o) { return o.p && o.dt == HKX_FP32 && o.ld == 0 && ((uin
 // The compiled epilogue form the quadrant kernel runs a call with, or -1 if it does not
 // take the call. Vector operands reach LDS by 16-byte DMA: unit stride, 16-byte aligned.
 int quad_form(const TileArgs& a, bool fp8, int mode) {
-  if (mode == kStoreF32)  // fp32 shares of a K split (or one fp32 sum a later pass finishes)
-    return a.c_dt == HKX_FP32 && a.ep.form == HKX_EP_NONE && ring_takes(a, fp8, mode) ? kEpNone : -1;
+  if (mode == kStoreF32) {
+    if (a.c_dt != HKX_FP32 || !ring_takes(a, fp8, mode)) return -1;
+    // fp32 shares of a K split (or one fp32 sum a later pass finishes)
+    if (a.ep.form == HKX_EP_NONE) return kEpNone;
+    // an fp32 C of fp8 operands: the dequant scales, and a tile added (a weight gradient's sum),
+    // fp32 with 16-byte aligned rows whose offsets fit 32 bits; C's rows 16-byte aligned, N % 4
+    // == 0 (every call's)
+    const Fused& e = a.ep;
+    if (!fp8 || a.kt_split < a.kt_total || e.form != HKX_EP_FUSED || e.act != HKX_ACT_NONE || e.cmul != 1.0f ||
+        e.cadd != 0.0f || e.ra.p || !a.c_aligned)
+      return -1;
+    if (!(vec32_16(e.cs) || one32(e.cs)) || !(vec32_16(e.rs) || one32(e.rs))) return -1;
+    if (e.ta.p && (e.ta.dt != HKX_FP32 || ((uintptr_t)e.ta.p & 15) || e.ta.ld % 4 ||
+                   (int64_t)((a.M + 255) / 256) * 256 * e.ta.ld * 4 >= (1LL << 32)))
+      return -1;
+    return kEpDeqAcc;
+  }
   if ((mode != kStore16 && mode != kPair16) || a.c_dt != HKX_BF16 || a.kt_split < a.kt_total)
     return -1;
   if (!ring_takes(a, fp8, mode)) return -1;
@@ -45,7 +60,10 @@ int quad_form(const TileArgs& a, bool fp8, int mode) {
 }  // namespace
 
 bool quad_takes(const TileArgs& a, bool fp8, int mode) {
-  return a.ab_fmt <= 1 && quad_form(a, fp8, mode) >= 0;
+  const int epf = quad_form(a, fp8, mode);
+  // e5m2 pairs: the dequant forms (other epilogues stay on the ring kernel's generic form)
+  if (a.ab_fmt > 1) return epf == kEpDeq || epf == kEpDeqBias || epf == kEpDeqAcc;
+  return epf >= 0;
 }
 
 bool quad128_takes(const TileArgs& a, bool fp8, int mode) {
@@ -64,6 +82,7 @@ bool quad128_takes(const TileArgs& a, bool fp8, int mode) {
 hipError_t launch_quad(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s) {
   const int epf = quad_form(a, fp8, mode);
   if (epf < 0) return hipErrorInvalidValue;
+  if (a.ab_fmt > 1 || epf == kEpDeqAcc) return launch_quad_fmt(a, epf, grid, s);
   if (mode == kStoreF32) {
     if (fp8)
       hipLaunchKernelGGL((quad_kernel<HKX_ACT_NONE, kEpNone, false, true, false, 256, true>), grid, dim3(512), 0, s, a);

@@ -52,7 +52,7 @@
 namespace hkx {
 
 template <int ACT, int EPF, bool PAIR = false, bool FP8 = false, bool MX = false, int BM = 256,
-          bool SHARE = false>
+          bool SHARE = false, int FMT = 1>
 __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
   constexpr int BN = PAIR ? 128 : 256;  // BN: C columns of a tile
   static_assert(BM == 256 || (BM == 128 && !FP8 && !MX), "128-row tiles: bf16 only");
@@ -70,10 +70,15 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
   constexpr int SCO = EPV;
   constexpr int SMEM = EPV + (MX ? 3 * 8192 : 3 * 3 * 1024);
   static_assert(!MX || (FP8 && EPF == kEpNone), "MX scales go with fp8 operands, no epilogue");
-  static_assert(FP8 ? (EPF == kEpNone || EPF == kEpDeq || EPF == kEpDeqBias) && ACT == HKX_ACT_NONE
+  static_assert(FP8 ? (EPF == kEpNone || EPF == kEpDeq || EPF == kEpDeqBias || EPF == kEpDeqAcc) &&
+                          ACT == HKX_ACT_NONE
                     : (EPF == kEpNone || EPF == kEpBias || EPF == kEpTile), "forms");
   static_assert(!PAIR || (!FP8 && EPF == kEpNone && ACT == HKX_ACT_NONE), "the paired form is silu * up");
   static_assert(SMEM <= 160 * 1024, "LDS");
+  // fp8 operand formats (TileArgs::ab_fmt): 1 e4m3 x e4m3, 2 e5m2 x e5m2, 3 A e4m3 x B e5m2,
+  // 4 A e5m2 x B e4m3; the MFMA's format fields of its first operand, B, and second, A
+  constexpr int kFmtB = FMT == 2 || FMT == 3, kFmtA = FMT == 2 || FMT == 4;
+  static_assert(FMT == 1 || (FP8 && !MX && !SHARE), "e5m2 operands: the plain fp8 forms");
 
   // Fragments are 16 x 16: bf16 on v_mfma_f32_16x16x32_bf16, fp8 (plain and MX) on
   // v_mfma_scale_f32_16x16x128_f8f6f4, the K-tile's 128 bytes in one MFMA. The fp8 16 x 16 x 128
@@ -191,7 +196,7 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
   // tile lt - 1's.
   // kEpTile: the bias is optional (absent, its DMA reads zeros from an empty buffer)
   constexpr bool bias = EPF == kEpBias || EPF == kEpDeqBias || EPF == kEpTile;
-  constexpr bool deq = EPF == kEpDeq || EPF == kEpDeqBias;
+  constexpr bool deq = EPF == kEpDeq || EPF == kEpDeqBias || EPF == kEpDeqAcc;
   const Fused& e = p.ep;
   const __amdgpu_buffer_rsrc_t rvec = make_rsrc(
       wave == 0 ? (deq ? e.cs.p : nullptr) : wave == 1 ? (deq ? e.rs.p : nullptr) : (bias ? e.ra.p : nullptr),
@@ -293,8 +298,8 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
             acc[i][j][f][g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
                 bf[g][h], af[f][h], c, 0, 0, 0, (int)scb[j][g], 0, (int)sca[i][f]);
           else if constexpr (FP8)
-            acc[i][j][f][g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[g][h], af[f][h], c, 0, 0, 0,
-                                                                               0, 0, 0);
+            acc[i][j][f][g] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(bf[g][h], af[f][h], c, kFmtB,
+                                                                               kFmtA, 0, 0, 0, 0);
           else
             acc[i][j][f][g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[g][h], af[f][h], c, 0, 0, 0);
         }
@@ -305,7 +310,7 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
   // q = l / 16) holds columns 4 q + [0, 4) of each 16-column fragment; the two fragments
   // of a 32-column block trade quarters (v_permlane16_swap) so each lane stores 16
   // contiguous bytes.
-  const uint32_t row_b = (uint32_t)p.ldc * (SHARE ? 4u : 2u);
+  const uint32_t row_b = (uint32_t)p.ldc * (SHARE || EPF == kEpDeqAcc ? 4u : 2u);
   const __amdgpu_buffer_rsrc_t rc = make_rsrc(
       SHARE ? (const void*)((const float*)p.c + (int64_t)blockIdx.y * p.split_stride) : p.c,
       (uint32_t)p.M * row_b);
@@ -352,6 +357,51 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
           const int col = 128 * j + 32 * wc + 16 * g + 4 * q;
           csc[j][g] = rs_bc ? f32x4{rs0, rs0, rs0, rs0} : *(const f32x4*)(ev + 1024 + col * 4);
         }
+    }
+    if constexpr (EPF == kEpDeqAcc) {
+      // fp32 C: the lane's row 128 i + 64 grp + 16 f + rf, columns 128 j + 32 wc + 16 g + 4 q +
+      // [0, 4), 16 bytes a store. The tile operand is usually C itself (a gradient added to):
+      // read and written by the same lane. Four fragments' reads are issued together and two
+      // such groups ahead of their adds and stores (48 registers; a whole block ahead spilled).
+      const uint32_t tb = (uint32_t)e.ta.ld * 4u;
+      const __amdgpu_buffer_rsrc_t rt = make_rsrc(e.ta.p, e.ta.p ? (uint32_t)p.M * tb : 0u);
+      const bool add = e.ta.p != nullptr;
+      constexpr int NG = 4 * NI;  // groups of four fragments: half a 64 x 32 block
+      f32x4 tv[3][2][NB];
+      auto load = [&](int b, f32x4 (&t)[2][NB]) {
+        const int i = b >> 2, j = (b >> 1) & 1, f0 = 2 * (b & 1);
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+          for (int g = 0; g < NB; ++g) {
+            const int row = m0 + 128 * i + 64 * grp + 16 * (f0 + f) + rf;
+            const int col = n0 + 128 * j + 32 * wc + 16 * g + 4 * q;
+            t[f][g] = __builtin_bit_cast(
+                f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                           rt, col < p.N ? (uint32_t)row * tb + (uint32_t)col * 4u : 0xfffffff0u, 0, 0));
+          }
+      };
+      if (add) {
+        load(0, tv[0]);
+        load(1, tv[1]);
+      }
+#pragma unroll
+      for (int b = 0; b < NG; ++b) {
+        const int i = b >> 2, j = (b >> 1) & 1, f0 = 2 * (b & 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (add && b + 2 < NG) load(b + 2, tv[(b + 2) % 3]);
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+          for (int g = 0; g < NB; ++g) {
+            f32x4 v = acc[i][j][f0 + f][g] * (csc[j][g] * rsc[i][f0 + f]);
+            if (add) v += tv[b % 3][f][g];
+            const int ml = 128 * i + 64 * grp + 16 * (f0 + f) + rf;
+            const int n = n0 + 128 * j + 32 * wc + 16 * g + 4 * q;
+            store_c(__builtin_bit_cast(i32x4, v), n < p.N, (uint32_t)(m0 + ml) * row_b + (uint32_t)n * 4u);
+          }
+      }
+      return;
     }
     [[maybe_unused]] f32x4 bv[2][2];
     if constexpr (bias) {

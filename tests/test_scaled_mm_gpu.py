@@ -114,3 +114,33 @@ def test_e4m3_one_value_scales_on_the_256_tiles(form, with_bias):
     ref = O.scaled_mm(a8, b8, sa_r, sb_r, bias if with_bias else None)
     O.assert_close(got, ref, rtol=3e-2, atol=1e-2)
     assert O.rel_to_max(got.cpu(), ref) < 8e-3
+
+
+@pytest.mark.parametrize("da,db", [(E4, E4), (E5, E5), (E4, E5), (E5, E4)])
+@pytest.mark.parametrize("m,n,k,scales", [(256, 256, 128, "one"), (300, 516, 384, "vec"), (777, 1032, 2176, "mixed"),
+                                          (4096, 1024, 256, "one")])
+def test_fp32_out_and_accumulate_on_the_quadrant_kernel(da, db, m, n, k, scales):
+    """The 256 x 256 fp32 output, plain and added to, in every operand format: ragged tiles of
+    M and N, one K-tile and odd counts, several tiles a workgroup, scales of one value and of
+    one a row. Bound: the fp8 MFMA keeps a K-step's products to about 2^-16 of their largest
+    (up to 1.3e-5 of sum |a b| at K = 128), fp32 adds 2^-23 of the sum added to."""
+    g = torch.Generator().manual_seed(m + n + k)
+    a = (torch.randn(m, k, generator=g) * 20).to(da)
+    b = (torch.randn(n, k, generator=g) * 20).to(db)
+    sa = torch.rand(m, 1, generator=g) + 0.5 if scales != "one" else torch.tensor([0.75])
+    sb = torch.rand(n, generator=g) + 0.5 if scales == "vec" else torch.tensor([1.25])
+    c0 = torch.randn(m, n, generator=g) * 100
+    how = dict(schedule="t256") if (da, db) == (E4, E4) else {}
+    print(f"case quad fp32 {da} {db} {m} {n} {k} {scales}", flush=True)
+    out, acc = torch.full((m, n), 9.0, device=DEV), c0.to(DEV)
+    args = (a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV))
+    hk.ops.scaled_mm(*args, out=out, **how)
+    hk.ops.scaled_mm(*args, out=acc, accumulate=True, **how)
+    hk.ops.scaled_mm(*args, out=acc, accumulate=True, **how)
+    torch.cuda.synchronize()
+    af = a.float().double() * sa.double()
+    bf = b.float().double() * sb.double().reshape(-1, 1)
+    ref, big = af @ bf.t(), af.abs() @ bf.abs().t()
+    assert ((out.cpu().double() - ref).abs() <= 2.0 ** -15 * big).all()
+    lim = 2 * 2.0 ** -15 * big + 2.0 ** -22 * (c0.abs() + 2 * big)
+    assert ((acc.cpu().double() - c0.double() - 2 * ref).abs() <= lim).all()
