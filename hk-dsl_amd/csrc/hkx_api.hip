@@ -834,25 +834,83 @@ int hkx_gemm_noalloc(const HkxGemmArgs* args, void* stream) {
   return hkx_gemm(&a, stream);
 }
 
-// The MX GEMM's K split: where its 256 x 256 tiles fill less than half the CUs, up to 8
-// splits of at least 8 k-tiles (1024 K) each, so the tiles times the splits stay within
-// the CUs; none where an fp32 share would span 4 GiB. (Shorter splits lost more to the
-// shares' round trip than they gained: K = 1152 and 1280 ran slower split in two.)
-static int mx_splits(int32_t m, int32_t n, int32_t k) {
-  if (m < 1 || n < 1 || k < 128 || k % 128 || m <= hkx::kSkinnyM) return 1;
-  const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
-  const int cu = cu_count();
-  if (2 * tiles > cu || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 1;
-  const int s = std::min(std::min(cu / tiles, (k / 128) / 8), 8);
-  if (s < 2) return 1;
-  const int kper = (k / 128 + s - 1) / s;  // no empty last split
-  return (k / 128 + kper - 1) / kper;
+// How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles of the
+// 4-wave kernel, K split over workgroups into fp32 shares a second launch sums; or, for the
+// first `cut` columns, on whole waves of 256 x 256 quadrant tiles, the rest of N on the tiles
+// (cut = n: all of it).
+struct MxPlan {
+  int bm, bn, splits, cut;
+  size_t ws_bytes;  // the workspace a caller passes (mx_share_bytes)
+};
+
+// A plan's estimated time in us: waves of one-a-CU workgroups, each a fixed part and a time a
+// 128-K unit by tile shape, or W's bytes at the rate these tiles stream them; a split adds its
+// sum's launch and the shares' round trip. Fitted to a sweep of every tile and split at 165
+// shapes (M 33-6000, N 768-16384, K 512-14336, one box): its pick is 0.3% slower than the best
+// on average, 1.13x at worst (M = 1000, 1024 x 8192). Before, every call ran on 256 x 256
+// tiles: 5120 x 4096 at M = 256 30.7 -> 14.9 us, 4096 x 1280 at M = 512 22.4 -> 8.7, 12800 x
+// 6144 at M = 256 51.1 -> 40.4, 1024 x 8192 at M = 64 21.3 -> 10.0.
+static double mx_cost(int m, int n, int k, int bm, int bn, int splits) {
+  const double fixed = bm == 256 ? 6.3 : bm == 64 ? 4.3 : bn == 128 ? 5.9 : 7.5;
+  const double unit = bm == 256 ? 1.53 : bm == 64 ? 0.47 : bn == 128 ? 0.56 : 0.90;
+  const long tiles = (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * splits;
+  const int cus = cu_count(), kper = (k / 128 + splits - 1) / splits;
+  const long waves = (tiles + cus - 1) / cus;
+  double t = fixed * (1.0 + 0.4 * (waves - 1)) + unit * kper * waves;
+  t = std::max(t, 5.0 + (double)n * k / 7.5e6);
+  if (splits > 1) t += 2.2 + (double)splits * m * n * 8.0 / 5.4e6;
+  return t;
 }
 
-size_t hkx_mx_gemm_workspace(int32_t m, int32_t n, int32_t k) {
-  const int s = mx_splits(m, n, k);
-  return s > 1 ? (size_t)s * (size_t)m * (size_t)n * 4u : 0;
+// The fp32 shares a call may use, and asks its caller for: up to 8 splits of 8 K units or more
+// of all of C where 256 x 256 tiles fill less than half the CUs, none otherwise (or where a
+// share would span 4 GiB). The plan below stays within it.
+static size_t mx_share_bytes(int32_t m, int32_t n, int32_t k) {
+  if (m <= hkx::kSkinnyM) return 0;
+  const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
+  const int cu = cu_count();
+  if (2 * tiles > cu || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 0;
+  const int s = std::min(std::min(cu / tiles, (k / 128) / 8), 8);
+  if (s < 2) return 0;
+  const int kper = (k / 128 + s - 1) / s;  // no empty last split
+  return (size_t)((k / 128 + kper - 1) / kper) * m * n * 4u;
 }
+
+static MxPlan mx_plan(int32_t m, int32_t n, int32_t k) {
+  if (m < 1 || n < 1 || k < 128 || k % 128) return {256, 256, 1, n, 0};
+  if (m <= hkx::kSkinnyM) return {0, 0, 1, 0, 0};
+  // the best tile and split of some columns: splits of 4 K units or more, no empty one, their
+  // shares within the workspace
+  const size_t room = mx_share_bytes(m, n, k);
+  struct Pick {
+    int bm, bn, splits;
+    double t;
+  };
+  auto best = [&](int cols, bool small_only) {
+    static const int kTiles[4][3] = {{64, 128, 8}, {128, 128, 4}, {128, 256, 2}, {256, 256, 1}};
+    Pick b{256, 256, 1, 1e30};
+    for (int i = 0; i < (small_only ? 3 : 4); ++i)
+      for (int s = 1; s <= kTiles[i][2]; s *= 2) {
+        const int units = k / 128, kper = (units + s - 1) / s;
+        if (s > 1 && (units / s < 4 || (units + kper - 1) / kper != s || (size_t)s * m * cols * 4u > room))
+          continue;
+        const double t = mx_cost(m, cols, k, kTiles[i][0], kTiles[i][1], s);
+        if (t < b.t) b = {kTiles[i][0], kTiles[i][1], s, t};
+      }
+    return b;
+  };
+  const Pick all = best(n, false);
+  const int cut = wave_cut(m, n, 256);
+  if (cut > 0 && cut < n) {  // whole waves on 256 x 256 tiles and the rest on smaller ones
+    const Pick rest = best(n - cut, true);
+    if (mx_cost(m, cut, k, 256, 256, 1) + rest.t < all.t)
+      return {rest.bm, rest.bn, rest.splits, cut, room};
+  }
+  if (all.bm == 256) return {256, 256, 1, n, room};
+  return {all.bm, all.bn, all.splits, 0, room};
+}
+
+size_t hkx_mx_gemm_workspace(int32_t m, int32_t n, int32_t k) { return mx_plan(m, n, k).ws_bytes; }
 
 int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const uint8_t* sa,
                 int64_t sa_ld, const uint8_t* sb, int64_t sb_ld, void* c, int64_t ldc, int32_t m,
@@ -887,8 +945,7 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   t.M = m;
   t.N = n;
   t.kt_total = t.kt_split = k / 128;
-  t.tiles_m = (m + 255) / 256;
-  t.tiles_n = (n + 255) / 256;
+  const MxPlan q = mx_plan(m, n, k);
   t.wgm = kWgmRows;
   t.pair_off = n;
   t.c_dt = HKX_BF16;
@@ -901,9 +958,8 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   t.sb_ld = (uint32_t)sb_ld;
   t.sa_bytes = (uint32_t)((long long)m * sa_ld);
   t.sb_bytes = (uint32_t)((long long)n * sb_ld);
-  const int splits = mx_splits(m, n, k);
   const hipStream_t s = (hipStream_t)stream;
-  if (m <= hkx::kSkinnyM) {  // the 8-bit decode kernel takes every such call
+  if (!q.bm) {  // the 8-bit decode kernel takes every call of M <= 32
     hkx::SkinnyArgs d{};
     d.a = a;
     d.b = b;
@@ -926,41 +982,52 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
     d.sb_bytes = t.sb_bytes;
     return launched(hkx::launch_skinny(d, true, cu_count(), s), "mx decode GEMM");
   }
-  if (splits == 1) {
-    const dim3 g(std::min(t.tiles_m * t.tiles_n, cu_count()));
-    // the quadrant kernel (whole-line fills) where it takes the call, else the ring's MX form
-    if (hkx::quad_takes(t, true, hkx::kStore16)) return launched(hkx::launch_quad_mx(t, g, s), "mx GEMM");
-    return launched(hkx::launch_ring_mx(t, false, g, s), "mx GEMM");
-  }
-  const size_t need = hkx_mx_gemm_workspace(m, n, k);
-  if (!ws || ws_bytes < need || !aligned(ws, 16))
+  if (q.ws_bytes && (!ws || ws_bytes < q.ws_bytes || !aligned(ws, 16)))
     return fail(HKX_ERR_WORKSPACE, "mx_gemm: needs %zu bytes of 16-byte aligned workspace, got %zu",
-                need, ws ? ws_bytes : (size_t)0);
+                q.ws_bytes, ws ? ws_bytes : (size_t)0);
+  if (q.cut) {  // whole waves of 256 x 256 tiles, one pass
+    t.N = q.cut;
+    t.tiles_m = (m + 255) / 256;
+    t.tiles_n = (q.cut + 255) / 256;
+    const dim3 g(std::min(t.tiles_m * t.tiles_n, cu_count()));
+    int rc = launched(hkx::launch_quad_mx(t, g, s), "mx GEMM");
+    if (rc || q.cut >= n) return rc;
+    // the rest of N as a call of its own: W's rows and their scales, C's columns
+    t.b = (const uint8_t*)b + (int64_t)q.cut * ldb;
+    t.b_bytes -= (uint32_t)((int64_t)q.cut * ldb);
+    t.sb = sb + (int64_t)q.cut * sb_ld;
+    t.sb_bytes -= (uint32_t)((int64_t)q.cut * sb_ld);
+    t.c = (uint8_t*)c + (int64_t)q.cut * 2;
+    t.N = n - q.cut;
+  }
+  t.tiles_m = (m + q.bm - 1) / q.bm;
+  t.tiles_n = (t.N + q.bn - 1) / q.bn;
+  const dim3 g(t.tiles_m * t.tiles_n, q.splits);
+  if (q.splits == 1) return launched(hkx::launch_tile4_mx(t, q.bm, q.bn, false, g, s), "mx GEMM (tiles)");
   // split s of K into fp32 share s (M x N, row stride N), one tile a workgroup
   hkx::TileArgs tw = t;
   tw.c = ws;
-  tw.ldc = n;
-  tw.split_stride = (int64_t)m * n;
+  tw.ldc = t.N;
+  tw.split_stride = (int64_t)m * t.N;
   tw.c_dt = HKX_FP32;
-  tw.kt_split = (k / 128 + splits - 1) / splits;
-  int rc = launched(hkx::launch_ring_mx(tw, true, dim3(t.tiles_m * t.tiles_n, splits), s),
-                    "mx GEMM (split over K)");
+  tw.kt_split = (k / 128 + q.splits - 1) / q.splits;
+  int rc = launched(hkx::launch_tile4_mx(tw, q.bm, q.bn, true, g, s), "mx GEMM (split over K)");
   if (rc) return rc;
   hkx::ReduceArgs r{};
   r.ws = (const float*)ws;
-  r.split_stride = (int64_t)m * n;
-  r.ws_ld = n;
-  r.c = c;
+  r.split_stride = tw.split_stride;
+  r.ws_ld = t.N;
+  r.c = t.c;
   r.ldc = ldc;
-  r.splits = splits;
+  r.splits = q.splits;
   r.M = m;
-  r.N = n;
+  r.N = t.N;
   r.c_dt = HKX_BF16;
   r.pair = 0;
   r.f = t.ep;
   HkxEpilogue none{};
   none.form = HKX_EP_NONE;
-  const dim3 rg(((n + 3) / 4 + 255) / 256, m < 65535 ? m : 65535);
+  const dim3 rg(((t.N + 3) / 4 + 255) / 256, m < 65535 ? m : 65535);
   return launched(hkx::launch_reduce(r, none, false, rg, s), "mx GEMM (sum of the splits)");
 }
 

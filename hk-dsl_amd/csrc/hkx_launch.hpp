@@ -54,9 +54,9 @@ hipError_t launch_quad(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStre
 hipError_t launch_quad_fmt(const TileArgs& a, int epf, dim3 grid, hipStream_t s);
 // Its MX form (fp8 operands, E8M0 block scales in a.sa / a.sb, bf16 C, one pass).
 hipError_t launch_quad_mx(const TileArgs& a, dim3 grid, hipStream_t s);
-// The MX form (fp8 operands, E8M0 block scales in a.sa / a.sb), no epilogue: bf16 C, or
-// fp32 shares of a K split (f32_shares, a.c the workspace, grid.y the splits).
-hipError_t launch_ring_mx(const TileArgs& a, bool f32_shares, dim3 grid, hipStream_t s);
+// The 4-wave tile kernel's MX form: 64 x 128, 128 x 128 or 128 x 256 tiles, bf16 C or fp32
+// shares of a K split (f32_shares, a.c the workspace, grid.y the splits).
+hipError_t launch_tile4_mx(const TileArgs& a, int bm, int bn, bool f32_shares, dim3 grid, hipStream_t s);
 // MX quantization of bf16 rows (hkx_mx_quant).
 hipError_t launch_mx_quant(const void* x, int64_t ldx, void* q, int64_t ldq, uint8_t* sc,
                            int64_t lds, int m, int k, hipStream_t s);

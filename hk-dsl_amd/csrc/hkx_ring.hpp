@@ -15,8 +15,7 @@
 // * MFMA: bf16 as v_mfma_f32_16x16x32_bf16 (4 x 8 fragments of 16 x 16 a wave; one k-step is
 //   a half-stage), fp8 e4m3 as v_mfma_scale_f32_32x32x64_f8f6f4 (2 x 4 fragments of 32 x 32).
 //   B's fragment is the first operand, so a lane ends with runs of four consecutive columns
-//   of one row of C. The MX form passes each lane's E8M0 byte for its fragment row and 32-K
-//   block as the MFMA's scales.
+//   of one row of C.
 // * Tile boundaries cost nothing in the pipeline: the fills of the next tile's first
 //   half-stages are in flight while this tile's last k-steps run and its epilogue is
 //   applied; the epilogue goes from the accumulators straight to global memory (no LDS
@@ -76,7 +75,7 @@ constexpr int kEpTile = 5;     // act(acc + ra[n] + ta[m][n]), ra (optional) and
 // FP8: 0 bf16 operands; 1 fp8 e4m3 x e4m3; 2 e5m2 x e5m2; 3 A e4m3 x B e5m2; 4 A e5m2 x B
 // e4m3 (TileArgs::ab_fmt). The scaled MFMA takes its first operand's format (here B's, as
 // B's fragment goes first) in cbsz and its second's (A's) in blgp: 0 e4m3, 1 e5m2.
-template <int FP8, int MODE, int ACT, int EPF, bool MX = false>
+template <int FP8, int MODE, int ACT, int EPF>
 __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
   constexpr int FMT_B = (FP8 == 2 || FP8 == 3) ? 1 : 0;
   constexpr int FMT_A = (FP8 == 2 || FP8 == 4) ? 1 : 0;
@@ -86,11 +85,7 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
   constexpr int HS = 512 * 64;                 // one half-stage buffer
   constexpr int NBUF = 4;
   constexpr int EPO = NBUF * HS;  // epilogue operands: [tile parity][cs, rs, ra][256 slots]
-  // MX scales: [chunk % 3][512 rows] of 16 bytes, a chunk the E8M0 bytes of 8 half-stages
-  // (16 blocks of 32 K) of every A and B row of the tile
-  constexpr int SCO = EPO + 2 * 3 * 1024;
-  constexpr int SMEM = SCO + (MX ? 3 * 512 * 16 : 0);
-  static_assert(!MX || FP8, "MX scales go with fp8 operands");
+  constexpr int SMEM = EPO + 2 * 3 * 1024;
   constexpr bool PAIR = (MODE == kPair16 || MODE == kPairWs);
   constexpr int OUTW = PAIR ? BN / 2 : BN;
   static_assert(!(PAIR && FP8) && !(MODE == kStore8 && PAIR), "modes");
@@ -149,23 +144,10 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
   uint32_t fa = 0, fb = 0;
   const uint32_t sa_step = 128u * p.lda_b, sb_step = (PAIR ? 64u : 128u) * p.ldb_b;
   int f_lt = 0, f_kv = 0, f_u = 0;  // the next fill: local tile, half-stage in it, global
-  const __amdgpu_buffer_rsrc_t rsa = make_rsrc(MX ? p.sa : nullptr, MX ? p.sa_bytes : 0u);
-  const __amdgpu_buffer_rsrc_t rsb = make_rsrc(MX ? p.sb : nullptr, MX ? p.sb_bytes : 0u);
-  uint32_t fsa = 0, fsb = 0;  // this lane's scale row (MX)
-  // MX scale chunks a tile; chunks rotate through three LDS buffers across tiles too. A
-  // chunk's buffer is refilled three chunks later, three half-stages before that chunk's
-  // first read, so at least 2 + 2 - 3 half-stages after the old chunk's last one (every
-  // chunk is 2 half-stages or more): with two buffers a 2-half-stage chunk (the end of
-  // K = 1152) let the refill land under the other group's last reads.
-  const int cpt = (hpt + 7) >> 3;
   auto fill_tile = [&](int lt) {
     int m0, n0;
     tile_at(lt, m0, n0);
     const int ln = opaque_lane();
-    if constexpr (MX) {
-      fsa = (uint32_t)(m0 + 64 * (wave & 3) + ln) * p.sa_ld;
-      fsb = (uint32_t)(n0 + 64 * (wave & 3) + ln) * p.sb_ld;
-    }
     const int r = 16 * wave + (ln >> 2);  // row of instruction 0 (A), 2 (B, less 256)
     const uint32_t ch = (uint32_t)(((ln & 3) ^ swz4(r)) << 4);
     fa = (uint32_t)(m0 + r) * p.lda_b + ch;
@@ -188,20 +170,6 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
     for (int i = 0; i < 4; ++i)
       buf_load16_lds(i < 2 ? ra : rb, base + i * 8192, i < 2 ? fa : fb,
                      so + (uint32_t)(i & 1) * (i < 2 ? sa_step : sb_step));
-    if constexpr (MX) {
-      // every 8th half-stage of a tile, after its operands: the scales of the 8 from it on
-      // (16 bytes of E8M0 a row, blocks 2 uk .. 2 uk + 15), lane l of wave w for row
-      // 64 w + l (A rows, then B). Issued after the half-stage's own fills, it is done
-      // whenever they are, before that half-stage is read; one more load only makes the
-      // waits count stricter.
-      if ((f_kv & 7) == 0) {
-        const uint32_t uk = (uint32_t)(2 * kt0 + f_kv);
-        const int chunk = f_lt * cpt + (f_kv >> 3);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wave < 4 ? rsa : rsb,
-            (__attribute__((address_space(3))) void*)(smem + SCO + (chunk % 3) * 8192 + wave * 1024),
-            16, wave < 4 ? fsa : fsb, __builtin_amdgcn_readfirstlane(2u * uk), 0, 0);
-      }
-    }
     ++f_u;
     if (f_u < nu) {
       if (++f_kv == hpt) {
@@ -266,27 +234,8 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
   }
   constexpr int FB = FR * 64;  // bytes of a fragment's rows in a buffer
   const int a_off = row0 * 64, b_off = (BM + col0) * 64;
-  // MX: lanes l / 32 = h give the scale of 32-K block h of the MFMA's 64 for their fragment
-  // row. Half-stage k of a tile (k % 8 = r in its chunk) has blocks 2 r and 2 r + 1 of the
-  // chunk: byte 2 (r & 1) + h of dword r / 2 of the row's 16 bytes, shifted down to byte 0,
-  // the MFMA's scale select.
-  uint32_t sfa[FM], sfb[FN];
-  const int sc_sh = 8 * (lane >> 5);
-  auto read_scales = [&](int lt, int k) {
-    if constexpr (MX) {
-      const int r = k & 7;
-      const uint32_t* sc =
-          (const uint32_t*)(smem + SCO + ((lt * cpt + (k >> 3)) % 3) * 8192) + (r >> 1);
-      const int rf = lane & 31, sh = sc_sh + 16 * (r & 1);
-#pragma unroll
-      for (int j = 0; j < FN; ++j) sfb[j] = sc[4 * (BM + col0 + 32 * j + rf)] >> sh;
-#pragma unroll
-      for (int i = 0; i < FM; ++i) sfa[i] = sc[4 * (row0 + 32 * i + rf)] >> sh;
-    }
-  };
-  auto read_frags = [&](int u, int lt, int k, Frag (&af)[FM], Frag (&bf)[FN]) {
+  auto read_frags = [&](int u, Frag (&af)[FM], Frag (&bf)[FN]) {
     const uint8_t* s = smem + (u & (NBUF - 1)) * HS;
-    read_scales(lt, k);
     if constexpr (FP8) {
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
@@ -315,10 +264,7 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         const Acc c = decltype(zero)::value ? Acc{} : acc[i][j];
-        if constexpr (MX)
-          acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], c, 0, 0, 0,
-                                                                     (int)sfb[j], 0, (int)sfa[i]);
-        else if constexpr (FP8)
+        if constexpr (FP8)
           acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], c, FMT_B,
                                                                      FMT_A, 0, 0, 0, 0);
         else
@@ -500,7 +446,7 @@ __global__ void __launch_bounds__(512, 1) ring_kernel(const TileArgs p) {
   for (int lt = 0; lt < my_tiles; ++lt) {
     for (int k = 0; k < hpt; ++k, ++u) {
       // memory phase
-      read_frags(u, lt, k, af, bf);
+      read_frags(u, af, bf);
       if (k == 0 && lt + 1 < my_tiles) ep_load(lt + 1);
       fill_next();
       __builtin_amdgcn_s_waitcnt(wait_vm_lgkm0(8));

@@ -48,7 +48,7 @@ struct TileArgs {
   int32_t c_dt;
   int32_t c_aligned;   // C's rows are 16-byte aligned: whole-chunk stores
   Fused ep;
-  // MX block scales (the ring kernel's MX form): E8M0 bytes, one a row and 32 K, row
+  // MX block scales (the MX forms): E8M0 bytes, one a row and 32 K, row
   // strides in bytes; bounds in bytes for the buffer resources
   const uint8_t* sa;
   const uint8_t* sb;

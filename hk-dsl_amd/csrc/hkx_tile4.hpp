@@ -33,7 +33,14 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // s_waitcnt vmcnt(n) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14)
 constexpr int tile4_vmcnt_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
-template <int BM, int BN, bool FP8, int MODE, int ACT = -1>
+// The MX form (MX: fp8 e4m3 operands with E8M0 block scales, a 16-bit C with no epilogue or
+// fp32 shares): the scale of 32-K block h of a k-step comes from lane half h, byte 2 ks + h of
+// its row's dword for the stage. The dwords of 4 stages reach LDS as 16 bytes a row by DMA with
+// the first fills of every 4th stage (a chunk; older than those fills, so the wait for the
+// stage covers it) into one of two buffers (the chunk before last was read before an earlier
+// barrier), and each wave reads a dword a fragment and stage, shifted down h bytes, byte 0 or 2
+// picked by op_sel.
+template <int BM, int BN, bool FP8, int MODE, int ACT = -1, bool MX = false>
 __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
   constexpr int TM = BM / 2, TN = BN / 2;
   constexpr int FM = TM / 32, FN = TN / 32;
@@ -49,11 +56,14 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
   constexpr int RS = OUTW * OB + 16;  // staging row stride, bytes
   constexpr int STAGING = STAGED ? BM * RS : 0;
   // LDS stages: as many as fit beside the row operands, up to four
-  constexpr int NST = 4 * STAGE + 2 * BN * 4 <= 160 * 1024   ? 4
-                      : 3 * STAGE + 2 * BN * 4 <= 160 * 1024 ? 3
-                                                             : 2;
+  constexpr int BESIDE = 2 * BN * 4 + (MX ? 2 * ROWS * 16 : 0) + 16;
+  constexpr int NST = 4 * STAGE + BESIDE <= 160 * 1024   ? 4
+                      : 3 * STAGE + BESIDE <= 160 * 1024 ? 3
+                                                         : 2;
   constexpr int ROWOP = (NST * STAGE > STAGING) ? NST * STAGE : STAGING;  // + the row operands
-  constexpr int SMEM = ROWOP + 2 * BN * 4;
+  constexpr int SCO = ROWOP + 2 * BN * 4;  // MX: then the scale chunks, [chunk % 2][row][16 bytes]
+  constexpr int SMEM = SCO + (MX ? 2 * ROWS * 16 : 0);
+  static_assert(!MX || (FP8 && (MODE == kStore16 || MODE == kStoreF32)), "MX: fp8, no epilogue");
   static_assert(FM >= 1 && FN >= 1 && BM % 64 == 0 && (BN == 256 || BN == 128), "tiling");
   static_assert(!PAIR || FN % 2 == 0, "the paired form needs gate/up fragment pairs");
   static_assert(SMEM <= 160 * 1024, "LDS");
@@ -118,6 +128,24 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
       if (i >= lo && i < hi) buf_load16_lds(i < NA ? ra : rb, base + i * 4096, voff[i], so);
   };
 
+  // MX: the scales of stages 4 c .. 4 c + 3 of every row of the tile (A's rows, then B's), 64
+  // rows a wave
+  [[maybe_unused]] auto scale_fill = [&](int c) {
+    if constexpr (MX) {
+      const int r = wave * 64 + lane;
+#pragma unroll
+      for (int w0 = 0; w0 < ROWS; w0 += 256) {
+        if (wave * 64 + w0 >= ROWS) break;
+        const bool isa = wave * 64 + w0 < BM;  // (BM is a multiple of 64)
+        const uint32_t row = (uint32_t)(isa ? m0 + r + w0 : n0 + r + w0 - BM);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            make_rsrc(isa ? p.sa : p.sb, isa ? p.sa_bytes : p.sb_bytes),
+            (__attribute__((address_space(3))) void*)(smem + SCO + (c & 1) * ROWS * 16 + (wave * 64 + w0) * 16), 16,
+            row * (isa ? p.sa_ld : p.sb_ld) + (uint32_t)(kt0 + 4 * c) * 4u, 0, 0, 0);
+      }
+    }
+  };
+
   // ---- fragment reads: lane l reads row l & 31 of a fragment, k-half l >> 5
   const int rf = lane & 31, h = lane >> 5;
   const int sw = swz(rf & 15);
@@ -126,7 +154,9 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
   for (int q = 0; q < 4; ++q) {
     // bf16: k-step q reads logical chunk 2q + h. fp8: k-step q / 2 reads chunks
     // 4 (q / 2) + 2h and + 1, as halves q & 1.
-    const int lc = FP8 ? (4 * (q >> 1) + 2 * h + (q & 1)) : (2 * q + h);
+    // MX: the MFMA takes a lane's bytes 0-15 as 32-K block 0 of the k-step and 16-31 as block 1,
+    // 16 K of each from either lane half: chunks 4 (q / 2) + h and + 2.
+    const int lc = MX ? (4 * (q >> 1) + 2 * (q & 1) + h) : FP8 ? (4 * (q >> 1) + 2 * h + (q & 1)) : (2 * q + h);
     rdo[q] = rf * 128 + ((lc ^ sw) << 4);
   }
   const int a_base = wm * TM * 128;
@@ -162,12 +192,30 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
 #pragma unroll
     for (int j = 0; j < FN; ++j) acc[i][j] = f32x16{};
 
-  auto mma = [&](const Frag (&af)[FM], const Frag (&bf)[FN]) {
+  // MX: the scales of a stage's fragments (this stage's, and the next's while its last k-step runs)
+  [[maybe_unused]] uint32_t sca[FM], scb[FN], scan[FM], scbn[FN];
+  auto read_scales = [&](int kt, uint32_t (&sa)[FM], uint32_t (&sb)[FN]) {
+    if constexpr (MX) {
+      const uint8_t* sc = smem + SCO + ((kt >> 2) & 1) * ROWS * 16 + (kt & 3) * 4 + rf * 16;
+#pragma unroll
+      for (int i = 0; i < FM; ++i) sa[i] = *(const uint32_t*)(sc + (wm * TM + 32 * i) * 16) >> (8 * h);
+#pragma unroll
+      for (int j = 0; j < FN; ++j) sb[j] = *(const uint32_t*)(sc + (BM + wn * TN + 32 * j) * 16) >> (8 * h);
+    }
+  };
+  auto mma = [&](const Frag (&af)[FM], const Frag (&bf)[FN], int ks = 0) {
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
-        if constexpr (FP8)
+        if constexpr (MX) {
+          if (ks == 0)
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], acc[i][j], 0, 0, 0,
+                                                                       (int)scb[j], 0, (int)sca[i]);
+          else
+            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], acc[i][j], 0, 0, 2,
+                                                                       (int)scb[j], 2, (int)sca[i]);
+        } else if constexpr (FP8)
           acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[j], af[i], acc[i][j], 0,
                                                                      0, 0, 0, 0, 0);
         else
@@ -214,11 +262,13 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
   };
+  scale_fill(0);
 #pragma unroll
   for (int st = 0; st < NST - 1; ++st) fill_part(min(st, nkt - 1), st, 0, NCH);
   fill_part(min(NST - 1, nkt - 1), NST - 1, 0, F0);
   sync_fills(true);
   read_frags(0, 0, a0, b0);
+  read_scales(0, sca, scb);
 
   // One iteration is one 128-byte K stage: KS k-steps of FM x FN MFMAs, fragment reads one
   // k-step ahead. The body is one basic block (fills and reads past the last stage are
@@ -238,10 +288,10 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
     for (int ks = 0; ks < KS - 1; ++ks) {
       if (ks & 1) {
         read_frags(s, ks + 1, a0, b0);
-        mma(a1, b1);
+        mma(a1, b1, ks);
       } else {
         read_frags(s, ks + 1, a1, b1);
-        mma(a0, b0);
+        mma(a0, b0, ks);
       }
       {
         // the rest of tile kt + 1's fills, begun under iteration kt - 1's last k-step
@@ -267,10 +317,12 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
     // waited for), and the next stage -- tile kt + 1 -- has landed: each wave waits for its
     // own fills of it: all but its newest (NST - 2) NCH
     sync_fills(false);
+    if (MX && ((kt + NST) & 3) == 0 && kt + NST < nkt) scale_fill((kt + NST) >> 2);
     fill_part(min(kt + NST, nkt - 1), s, 0, F0);
     // KS is even: step KS-1 multiplies set 1 while the next stage's step 0 reads set 0
     read_frags((kt + 1) % NST, 0, a0, b0);
-    mma(a1, b1);
+    read_scales(kt + 1, scan, scbn);  // (past the last stage: never used)
+    mma(a1, b1, KS - 1);
 #pragma unroll
     for (int q = 0; q < NRD; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -280,6 +332,12 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
     __builtin_amdgcn_sched_group_barrier(0x008, FM * FN - NRD, 0);
     __builtin_amdgcn_sched_group_barrier(0x020, NCH, 0);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MX) {
+#pragma unroll
+      for (int i = 0; i < FM; ++i) sca[i] = scan[i];
+#pragma unroll
+      for (int j = 0; j < FN; ++j) scb[j] = scbn[j];
+    }
   }
   __builtin_amdgcn_s_waitcnt(0x3f70);  // the last (unused) fills land before LDS is reused
 

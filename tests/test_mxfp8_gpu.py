@@ -141,3 +141,19 @@ def test_mx_quant_every_code_and_the_special_values():
     # inf / 2^121 clamps to 448; a NaN is left out of the largest value and clamps to -448
     assert q[0, :2].tolist() == [0x7e, 0x80] and q[1, :2].tolist() == [0xfe, 0x00]
     assert q[2, :3].tolist() == [0xfe, 0x7e, 0xc0]
+
+
+@pytest.mark.parametrize("m,n,k", [(33, 128, 128), (64, 1032, 512), (65, 264, 1152), (100, 1792, 5120), (129, 520, 640),
+                                   (512, 4096, 1280), (40, 1024, 8192), (700, 1032, 4224), (1000, 5128, 1152),
+                                   (1500, 2304, 2176), (2300, 7688, 640), (4100, 5128, 384)])
+def test_mx_tiles_splits_and_wave_cuts(m, n, k):
+    """The 4-wave tiles' MX form at the plans the shapes pick: one tile and one K unit, ragged
+    rows and columns, unit counts of every remainder by 4 (a scale chunk), K splits, and whole
+    waves of 256 x 256 tiles with the rest of N on smaller ones (the last two)."""
+    a, b, sa, sb = _operands(m, n, k, seed=m + n + k, block_weight_scales=False)
+    out = torch.full((m + 1, n + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    print(f"case mx tiles {m}x{n}x{k}", flush=True)
+    mxfp8.gemm(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV), out=out[:m, :n])
+    ref = O.mx_gemm(a, b, sa, sb)
+    assert O.rel_to_max(out[:m, :n].cpu(), ref) < 5e-3
+    assert (out[m] == 7.0).all() and (out[:, n:] == 7.0).all()
