@@ -613,6 +613,7 @@ int hkx_gemm(const HkxGemmArgs* args, void* stream) {
   if (p.kernel == HKX_KERNEL_TILE) {
     hkx::TileArgs t{};
     t.ab_fmt = fmt_of(a.ab_dtype);
+    t.cus = cu_count();
     t.a = a.a;
     t.b = a.b;
     t.a_bytes = (uint32_t)((long long)a.m * a.lda * eb);
@@ -934,6 +935,7 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
       (long long)((m + 255) / 256) * 256 * ldc * 2 >= (1LL << 32))
     return fail(HKX_ERR_SHAPE, "mx_gemm: A, B or C spans 4 GiB or more; split the call");
   hkx::TileArgs t{};
+  t.cus = cu_count();
   t.a = a;
   t.b = b;
   t.c = c;

@@ -20,14 +20,21 @@ template <int BM, int BN>
 hipError_t launch_tile4(const TileArgs& a, bool fp8, int mode, dim3 grid,
                         hipStream_t s);
 
+// Whether a grid of the 4-wave kernel's 128-column tiles runs its two-a-CU form: past one
+// workgroup a CU, where the second hides what a lone wave a SIMD waits for and fills the last
+// wave's idle CUs (700 x 4096 x 4096 on 64 x 128 tiles 44.5 -> 39.4 us, 2048 x 4096 x 4096 on
+// 128 x 128 ones 79.4 -> 72.1, 333 x 4096 x 14336 split 4 ways 79.2 -> 74.6). Up to one a CU
+// the one-a-CU form's deeper stages stay.
+inline bool tile4_two(const TileArgs& a, dim3 grid) { return grid.x * grid.y > (unsigned)a.cus; }
+
 // A 16- or 8-bit C with the fused form's activation fixed at compile time (the epilogue is
 // then straight-line code); any other store takes it at run time.
-#define HKX_TILE4_STAGED(BM, BN, FP8, MODE)                                                 \
+#define HKX_TILE4_STAGED(BM, BN, FP8, MODE, RES)                                            \
   switch (a.ep.form == HKX_EP_FUSED ? a.ep.act : HKX_ACT_NONE) {                            \
-    case HKX_ACT_GELU_TANH: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_GELU_TANH>), grid, block, 0, s, a); break; \
-    case HKX_ACT_SILU: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_SILU>), grid, block, 0, s, a); break;           \
-    case HKX_ACT_RELU: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_RELU>), grid, block, 0, s, a); break;           \
-    default: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_NONE>), grid, block, 0, s, a); break;                    \
+    case HKX_ACT_GELU_TANH: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_GELU_TANH, false, RES>), grid, block, 0, s, a); break; \
+    case HKX_ACT_SILU: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_SILU, false, RES>), grid, block, 0, s, a); break;           \
+    case HKX_ACT_RELU: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_RELU, false, RES>), grid, block, 0, s, a); break;           \
+    default: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, MODE, HKX_ACT_NONE, false, RES>), grid, block, 0, s, a); break;                    \
   }
 
 hipError_t launch_pp(const TileArgs& a, bool fp8, int mode, bool mf16, dim3 grid, hipStream_t s);
@@ -110,29 +117,27 @@ hipError_t launch_reduce(const ReduceArgs& a, const HkxEpilogue& ep, bool progra
     return hipGetLastError();                                                                \
   }
 
+// (two workgroups a CU where the tile's stages allow it and the grid has more than one a CU)
 #define HKX_TILE4_LAUNCHER(BM, BN)                                                           \
-  template <>                                                                                \
-  hipError_t launch_tile4<BM, BN>(const TileArgs& a, bool fp8, int mode, dim3 grid,        \
-                                  hipStream_t s) {                                           \
+  template <bool FP8, int RES>                                                               \
+  static hipError_t launch_res(const TileArgs& a, int mode, dim3 grid, hipStream_t s) {      \
     const dim3 block(256);                                                                   \
-    if (fp8) {                                                                               \
-      switch (mode) {                                                                        \
-        case kStore16: HKX_TILE4_STAGED(BM, BN, true, kStore16) break;                                \
-        case kStore8: HKX_TILE4_STAGED(BM, BN, true, kStore8) break;                         \
-        case kStoreF32: hipLaunchKernelGGL((tile4_kernel<BM, BN, true, kStoreF32>), grid, block, 0, s, a); break; \
-        default: return hipErrorInvalidValue;                                                \
-      }                                                                                      \
-    } else {                                                                                 \
-      switch (mode) {                                                                        \
-        case kStore16: HKX_TILE4_STAGED(BM, BN, false, kStore16) break;                               \
-        case kStore8: HKX_TILE4_STAGED(BM, BN, false, kStore8) break;                        \
-        case kStoreF32: hipLaunchKernelGGL((tile4_kernel<BM, BN, false, kStoreF32>), grid, block, 0, s, a); break; \
-        case kPair16: hipLaunchKernelGGL((tile4_kernel<BM, BN, false, kPair16>), grid, block, 0, s, a); break;     \
-        case kPairWs: hipLaunchKernelGGL((tile4_kernel<BM, BN, false, kPairWs>), grid, block, 0, s, a); break;     \
-        default: return hipErrorInvalidValue;                                                \
-      }                                                                                      \
+    switch (mode) {                                                                          \
+      case kStore16: HKX_TILE4_STAGED(BM, BN, FP8, kStore16, RES) break;                     \
+      case kStore8: HKX_TILE4_STAGED(BM, BN, FP8, kStore8, RES) break;                       \
+      case kStoreF32: hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, kStoreF32, -1, false, RES>), grid, block, 0, s, a); break; \
+      case kPair16: if constexpr (!FP8) { hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, kPair16, -1, false, RES>), grid, block, 0, s, a); break; } return hipErrorInvalidValue; \
+      case kPairWs: if constexpr (!FP8) { hipLaunchKernelGGL((tile4_kernel<BM, BN, FP8, kPairWs, -1, false, RES>), grid, block, 0, s, a); break; } return hipErrorInvalidValue; \
+      default: return hipErrorInvalidValue;                                                  \
     }                                                                                        \
     return hipGetLastError();                                                                \
+  }                                                                                          \
+  template <>                                                                                \
+  hipError_t launch_tile4<BM, BN>(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s) { \
+    if constexpr (BN == 128) {                                                               \
+      if (tile4_two(a, grid)) return fp8 ? launch_res<true, 2>(a, mode, grid, s) : launch_res<false, 2>(a, mode, grid, s); \
+    }                                                                                        \
+    return fp8 ? launch_res<true, 1>(a, mode, grid, s) : launch_res<false, 1>(a, mode, grid, s); \
   }
 
 }  // namespace hkx

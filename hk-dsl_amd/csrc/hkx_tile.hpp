@@ -46,6 +46,7 @@ struct TileArgs {
   int32_t tiles_m, tiles_n, wgm;
   int32_t pair_off;    // B rows from a gate row to its up row (paired form)
   int32_t c_dt;
+  int32_t cus;         // the GPU's CUs (the launchers' rules)
   int32_t c_aligned;   // C's rows are 16-byte aligned: whole-chunk stores
   Fused ep;
   // MX block scales (the MX forms): E8M0 bytes, one a row and 32 K, row

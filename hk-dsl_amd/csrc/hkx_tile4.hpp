@@ -15,6 +15,8 @@
 //   The fills of tile kt + NST go into the stage iteration kt read, begun right after its
 //   one barrier and spread under the next iteration's k-steps; with three stages they have
 //   one iteration more to land (a wave a SIMD has nothing else to hide their latency with).
+//   RES = 2 is the form of which two workgroups fit a CU (128-column tiles in half the LDS: two
+//   stages at 128 x 128, three at 64 x 128), for grids of more than one a CU.
 // * Fragment reads are software-pipelined one k-step ahead (two register sets), and the
 //   reads of the next stage's first k-step are issued under the last k-step's MFMAs.
 // * MFMA: v_mfma_f32_32x32x16_bf16 / v_mfma_f32_32x32x64_f8f6f4 (fp8 e4m3), B's fragment
@@ -40,8 +42,8 @@ constexpr int tile4_vmcnt_lgkm0(int n) { return (n & 15) | ((n >> 4) << 14) | (7
 // stage covers it) into one of two buffers (the chunk before last was read before an earlier
 // barrier), and each wave reads a dword a fragment and stage, shifted down h bytes, byte 0 or 2
 // picked by op_sel.
-template <int BM, int BN, bool FP8, int MODE, int ACT = -1, bool MX = false>
-__global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
+template <int BM, int BN, bool FP8, int MODE, int ACT = -1, bool MX = false, int RES = 1>
+__global__ void __launch_bounds__(256, RES) tile4_kernel(const TileArgs p) {
   constexpr int TM = BM / 2, TN = BN / 2;
   constexpr int FM = TM / 32, FN = TN / 32;
   constexpr int ROWS = BM + BN;
@@ -57,16 +59,15 @@ __global__ void __launch_bounds__(256, 1) tile4_kernel(const TileArgs p) {
   constexpr int STAGING = STAGED ? BM * RS : 0;
   // LDS stages: as many as fit beside the row operands, up to four
   constexpr int BESIDE = 2 * BN * 4 + (MX ? 2 * ROWS * 16 : 0) + 16;
-  constexpr int NST = 4 * STAGE + BESIDE <= 160 * 1024   ? 4
-                      : 3 * STAGE + BESIDE <= 160 * 1024 ? 3
-                                                         : 2;
+  constexpr int LDS = 160 * 1024 / RES;
+  constexpr int NST = 4 * STAGE + BESIDE <= LDS ? 4 : 3 * STAGE + BESIDE <= LDS ? 3 : 2;
   constexpr int ROWOP = (NST * STAGE > STAGING) ? NST * STAGE : STAGING;  // + the row operands
   constexpr int SCO = ROWOP + 2 * BN * 4;  // MX: then the scale chunks, [chunk % 2][row][16 bytes]
   constexpr int SMEM = SCO + (MX ? 2 * ROWS * 16 : 0);
   static_assert(!MX || (FP8 && (MODE == kStore16 || MODE == kStoreF32)), "MX: fp8, no epilogue");
   static_assert(FM >= 1 && FN >= 1 && BM % 64 == 0 && (BN == 256 || BN == 128), "tiling");
   static_assert(!PAIR || FN % 2 == 0, "the paired form needs gate/up fragment pairs");
-  static_assert(SMEM <= 160 * 1024, "LDS");
+  static_assert(SMEM + 16 <= LDS, "LDS");
   using Frag = typename std::conditional<FP8, i32x8, bf16x8>::type;
 
   // (+16 bytes: the split finish's flag. A second __shared__ object would make the compiler

@@ -128,25 +128,60 @@ def fits(name: str, m: int, n: int, k: int, fp8: bool = False) -> bool:
     return True
 
 
-def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
-    """The route when no record or table entry names one: the decode kernel at M <= 32
-    (bf16); else the largest tile whose count fills three quarters of the CUs -- 256 x 256,
-    128 x 256 (the quadrant kernel's 128-row form for bf16 up to K = 4096, the 4-wave
-    kernel otherwise), 128 x 128; else 64 x 128 tiles (up to M = 128) or 128 x 128 ones,
-    split over K in powers of two while the workgroups stay within the CUs and each split
-    keeps 16 or more 128-byte K units. On the shipped table's 132 measured points its pick
-    is 2% slower than the best candidate on average (the rule before the 128-column tiles:
-    26%).
+#: The rule's tiles: candidate -> (cost class, the fewest rows it is considered from).
+_RULE = {"t64x128": ("64x128", 1), "t64x128k2": ("64x128", 1), "t64x128k4": ("64x128", 1),
+         "t64x128k8": ("64x128", 1), "t128x128": ("128x128", 65), "t128x128k2": ("128x128", 65),
+         "t128x128k4": ("128x128", 65), "t128": ("128x256", 65), "t128k2": ("128x256", 65),
+         "t128k4": ("128x256", 65), "q128": ("q128", 65), "t256": ("256x256", 129),
+         "t256k2": ("256x256", 129), "t256k4": ("256x256", 129), "t256k8": ("256x256", 129)}
+#: A cost class: us fixed, us a K unit (64 bf16), and the part of the fixed time a further wave
+#: of workgroups pays.
+_COST = {"64x128": (3.2, 0.313, 0.39), "128x128": (5.8, 0.407, 0.51), "128x256": (6.6, 0.758, 0.37),
+         "q128": (6.7, 0.662, 0.52), "256x256": (9.7, 0.96, 0.56)}
+#: Up to here a call between two measured Ms takes the rule.
+BETWEEN_M = 2048
 
-    fp8 has no measured table, so its last step follows one measured sweep (scaled_mm with
-    dequant and bias, N x K in {4096 x 4096, 12288 x 4096, 4096 x 12288}, M 256-4096, every
+
+def _cost(name: str, m: int, n: int, k: int) -> float:
+    """A tile candidate's estimated us: waves of one-a-CU workgroups, or W at the rate the
+    tiles stream it; a split adds the sum's launch and its fp32 shares' round trip."""
+    c = CANDIDATES[name]
+    fixed, unit, more = _COST[_RULE[name][0]]
+    splits = c.get("splits", 1)
+    tiles = -(-m // c["tile_m"]) * -(-n // c["tile_n"]) * splits
+    waves = -(-tiles // CUS)
+    t = fixed * (1 + more * (waves - 1)) + unit * -(-(k // 64) // splits) * waves
+    t = max(t, 5 + 2 * n * k / 8e6)
+    return t if splits == 1 else t + 2.2 + splits * m * n * 8 / 6.1e6
+
+
+def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
+    """The route when no record or table entry names one: the decode kernel at M <= 32 (bf16),
+    else, for bf16, the tile and split of the least `_cost`. Its numbers are fitted to a sweep
+    of the tiles and splits at 202 shapes (M 33-3300, N 512-24576, K 640-14336, one box): its
+    pick is 0.8% slower than the best on average, 1.27x at worst; the steps it replaced (the
+    largest tile whose count fills three quarters of the CUs, else splits) and the table's
+    nearest M together 12%, 1.66x (300 x 6144 x 4096 on 128 x 256 tiles split 4 ways 52.9 us,
+    on 64 x 128 ones 31.8; 333 x 4096 x 14336 79 -> 63; 256 x 1024 x 1024 12.1 -> 8.7).
+
+    fp8 has no such sweep: the largest tile whose count fills three quarters of the CUs -- 256 x
+    256, 128 x 256, 128 x 128; else 64 x 128 tiles or 128 x 128 ones, split over K in powers of
+    two while the workgroups stay within the CUs and each split keeps 16 or more 128-byte K
+    units. Its last step follows one measured sweep (scaled_mm with dequant and bias, N x K in
+    {4096 x 4096, 12288 x 4096, 4096 x 12288}, M 256-4096, every
     tile candidate, M 16-4096): from M = 129 to 512, 64 x 128 tiles, split only where each
     split keeps 32 K units (4096 x 4096 at M = 256: 12.1-12.2 us on 64 x 128 tiles against
     19.6 on 128 x 128 ones split in two; at M = 512 13.9 against 21.9; 4096 x 12288 at M =
-    256 split in two, 23.9 against 29.9 unsplit); up to M = 128 the bf16 steps."""
-    if not fp8 and m <= 32 and k % 128 == 0:
-        return "decode"
-    kunits = k * (1 if fp8 else 2) // 128
+    256 split in two, 23.9 against 29.9 unsplit)."""
+    if not fp8:
+        if m <= 32 and k % 128 == 0:
+            return "decode"
+        units = k // 64
+        return min((c for c, (_, least) in _RULE.items()
+                    if m >= least and (CANDIDATES[c].get("splits", 1) == 1
+                                       or units // CANDIDATES[c]["splits"] >= 4)),
+                   key=lambda c: _cost(c, m, n, k))
+    kunits = k // 128
 
     def tiles(bm, bn):
         return math.ceil(m / bm) * math.ceil(n / bn)
@@ -154,13 +189,13 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
     if m > 128 and tiles(256, 256) >= 0.75 * CUS:
         return "t256"
     if m > 64 and tiles(128, 256) >= 0.75 * CUS:
-        return "q128" if not fp8 and kunits <= 64 else "t128"
+        return "t128"
     if m > 64 and tiles(128, 128) >= 0.75 * CUS:
         return "t128x128"
-    bm = 64 if m <= (512 if fp8 else 128) else 128
+    bm = 64 if m <= 512 else 128
     t = tiles(bm, 128)
     most = 8 if bm == 64 else 4  # the split candidates there are
-    per_split = 32 if fp8 and m > 128 else 16  # K units a split keeps at least
+    per_split = 32 if m > 128 else 16  # K units a split keeps at least
     splits = 1
     while t * splits * 2 <= CUS and kunits // (splits * 2) >= per_split and splits < most:
         splits *= 2
@@ -169,7 +204,9 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
 
 def route(m: int, n: int, k: int, fp8: bool = False) -> str:
     """The candidate an M x N x K call runs: a user record, else the measured table's
-    nearest M (log scale) for this N x K, else `rule` (gemm_cdna.py:969-999)."""
+    nearest M (log scale) for this N x K, else `rule` (gemm_cdna.py:969-999). Between two
+    measured Ms, 5% or more from the nearer, the rule answers too, up to BETWEEN_M: there the
+    tiles are few waves and the nearest M's pick may leave a wave nearly empty."""
     for key in ((m, n, k), "*"):
         if key in OVERRIDE and fits(OVERRIDE[key], m, n, k, fp8):
             return OVERRIDE[key]
@@ -178,6 +215,8 @@ def route(m: int, n: int, k: int, fp8: bool = False) -> str:
         if ent:
             ms = sorted(int(x) for x in ent)
             best = min(ms, key=lambda x: abs(math.log(x) - math.log(m)))
+            if 32 < m <= BETWEEN_M and abs(math.log(best / m)) >= 0.05:
+                return rule(m, n, k)
             name = ent[str(best)]
             if fits(name, m, n, k, fp8):
                 return name
