@@ -134,25 +134,29 @@ _RULE = {"t64x128": ("64x128", 1), "t64x128k2": ("64x128", 1), "t64x128k4": ("64
          "t128x128k4": ("128x128", 65), "t128": ("128x256", 65), "t128k2": ("128x256", 65),
          "t128k4": ("128x256", 65), "q128": ("q128", 65), "t256": ("256x256", 129),
          "t256k2": ("256x256", 129), "t256k4": ("256x256", 129), "t256k8": ("256x256", 129)}
-#: A cost class: us fixed, us a K unit (64 bf16), and the part of the fixed time a further wave
-#: of workgroups pays.
+#: A cost class: us fixed, us a 128-byte K unit, and the part of the fixed time a further wave of
+#: workgroups pays; "split" the us of the sum's launch and the bytes a us of its shares and of W.
 _COST = {"64x128": (3.2, 0.313, 0.39), "128x128": (5.8, 0.407, 0.51), "128x256": (6.6, 0.758, 0.37),
-         "q128": (6.7, 0.662, 0.52), "256x256": (9.7, 0.96, 0.56)}
+         "q128": (6.7, 0.662, 0.52), "256x256": (9.7, 0.96, 0.56), "split": (2.2, 6.1e6, 8e6)}
+_COST8 = {"64x128": (4.5, 0.254, 0.32), "128x128": (5.0, 0.412, 0.26), "128x256": (8.3, 0.71, 0.475),
+          "256x256": (8.3, 0.89, 0.37), "split": (2.4, 5.3e6, 6.7e6)}
 #: Up to here a call between two measured Ms takes the rule.
 BETWEEN_M = 2048
 
 
-def _cost(name: str, m: int, n: int, k: int) -> float:
+def _cost(name: str, m: int, n: int, k: int, fp8: bool = False) -> float:
     """A tile candidate's estimated us: waves of one-a-CU workgroups, or W at the rate the
     tiles stream it; a split adds the sum's launch and its fp32 shares' round trip."""
     c = CANDIDATES[name]
-    fixed, unit, more = _COST[_RULE[name][0]]
+    kbytes, table = (k, _COST8) if fp8 else (2 * k, _COST)
+    fixed, unit, more = table[_RULE[name][0]]
+    launch, share_rate, w_rate = table["split"]
     splits = c.get("splits", 1)
     tiles = -(-m // c["tile_m"]) * -(-n // c["tile_n"]) * splits
     waves = -(-tiles // CUS)
-    t = fixed * (1 + more * (waves - 1)) + unit * -(-(k // 64) // splits) * waves
-    t = max(t, 5 + 2 * n * k / 8e6)
-    return t if splits == 1 else t + 2.2 + splits * m * n * 8 / 6.1e6
+    t = fixed * (1 + more * (waves - 1)) + unit * -(-(kbytes // 128) // splits) * waves
+    t = max(t, 5 + n * kbytes / w_rate)
+    return t if splits == 1 else t + launch + splits * m * n * 8 / share_rate
 
 
 def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
@@ -161,18 +165,14 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
     of the tiles and splits at 202 shapes (M 33-3300, N 512-24576, K 640-14336, one box): its
     pick is 0.8% slower than the best on average, 1.27x at worst; the steps it replaced (the
     largest tile whose count fills three quarters of the CUs, else splits) and the table's
-    nearest M together 12%, 1.66x (300 x 6144 x 4096 on 128 x 256 tiles split 4 ways 52.9 us,
-    on 64 x 128 ones 31.8; 333 x 4096 x 14336 79 -> 63; 256 x 1024 x 1024 12.1 -> 8.7).
+    nearest M together 12%, 1.66x (300 x 6144 x 4096 on 128 x 256 tiles split 4 ways 46.0 us,
+    on 64 x 128 ones 27.7; 333 x 4096 x 14336 79 -> 63; 256 x 1024 x 1024 12.1 -> 8.7).
 
-    fp8 has no such sweep: the largest tile whose count fills three quarters of the CUs -- 256 x
-    256, 128 x 256, 128 x 128; else 64 x 128 tiles or 128 x 128 ones, split over K in powers of
-    two while the workgroups stay within the CUs and each split keeps 16 or more 128-byte K
-    units. Its last step follows one measured sweep (scaled_mm with dequant and bias, N x K in
-    {4096 x 4096, 12288 x 4096, 4096 x 12288}, M 256-4096, every
-    tile candidate, M 16-4096): from M = 129 to 512, 64 x 128 tiles, split only where each
-    split keeps 32 K units (4096 x 4096 at M = 256: 12.1-12.2 us on 64 x 128 tiles against
-    19.6 on 128 x 128 ones split in two; at M = 512 13.9 against 21.9; 4096 x 12288 at M =
-    256 split in two, 23.9 against 29.9 unsplit)."""
+    fp8 has two: `_rule8_steps`, and past 64 rows and from K = 1024 the tile and split of the
+    least fp8 cost where that is 7% or more under the steps' (fitted to 279 shapes of scaled_mm
+    with bias, M 33-4096: the steps were 6.6% slower than the best on average and 1.66x at
+    worst, both together 1%: 1300 x 6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x
+    1024 on 64 x 128 ones 8.9 -> 6.5)."""
     if not fp8:
         if m <= 32 and k % 128 == 0:
             return "decode"
@@ -181,6 +181,23 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
                     if m >= least and (CANDIDATES[c].get("splits", 1) == 1
                                        or units // CANDIDATES[c]["splits"] >= 4)),
                    key=lambda c: _cost(c, m, n, k))
+    steps = _rule8_steps(m, n, k)
+    if m <= 64 or k < 1024:
+        return steps
+    best = min((c for c, (cls, least) in _RULE.items()
+                if cls != "q128" and m >= least and (CANDIDATES[c].get("splits", 1) == 1
+                                                     or k // 128 // CANDIDATES[c]["splits"] >= 8)),
+               key=lambda c: _cost(c, m, n, k, True))
+    return best if _cost(best, m, n, k, True) <= 0.93 * _cost(steps, m, n, k, True) else steps
+
+
+def _rule8_steps(m: int, n: int, k: int) -> str:
+    """fp8: the largest tile whose count fills three quarters of the CUs -- 256 x 256, 128 x 256,
+    128 x 128; else 64 x 128 tiles or 128 x 128 ones, split over K in powers of two while the
+    workgroups stay within the CUs and each split keeps 16 or more 128-byte K units. From M =
+    129 to 512, 64 x 128 tiles, split only where each split keeps 32 K units (4096 x 4096 at M =
+    256: 12.1-12.2 us on 64 x 128 tiles against 19.6 on 128 x 128 ones split in two; at M = 512
+    13.9 against 21.9; 4096 x 12288 at M = 256 split in two, 23.9 against 29.9 unsplit)."""
     kunits = k // 128
 
     def tiles(bm, bn):

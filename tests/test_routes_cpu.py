@@ -209,3 +209,26 @@ def test_decode8_rule(monkeypatch):
     assert not gemm_cdna.decode8(1, 6144, 4096) and gemm_cdna.decode8(2, 6144, 4096)
     gemm_cdna.OVERRIDE["*"] = "decode"     # does not take fp8
     assert gemm_cdna.decode8(2, 6144, 4096)
+
+
+def test_rules_by_cost(monkeypatch):
+    """The rules' picks at sweep points where the former steps lost most, each the measured best
+    or within 2% of it; and every pick is a candidate that takes its shape."""
+    monkeypatch.setattr(gemm_cdna, "OVERRIDE", {})
+    bf16 = {(256, 1024, 1024): "t64x128", (150, 1024, 1024): "t64x128", (200, 512, 4096): "t64x128k8",
+            (300, 6144, 4096): "t64x128"}
+    fp8 = {(1300, 6144, 4096): "t256", (900, 1024, 1024): "t64x128", (2600, 4096, 4096): "t256",
+           (2048, 512, 4096): "t64x128", (700, 11008, 640): "t128"}
+    assert {s: gemm_cdna.rule(*s) for s in bf16} == bf16
+    assert {s: gemm_cdna.rule(*s, fp8=True) for s in fp8} == fp8
+    for m in (1, 33, 64, 65, 129, 333, 1000, 5000):
+        for n in (4, 516, 4096, 30000):
+            for k in (128, 640, 4096, 16384):
+                for f8 in (False, True):
+                    assert gemm_cdna.fits(gemm_cdna.rule(m, n, k, fp8=f8), m, n, k, f8)
+    # between the table's Ms the rule answers; at one of them and past 2048 rows the table does
+    table = gemm_cdna.table()["4096x14336"]
+    assert gemm_cdna.route(333, 4096, 14336) == gemm_cdna.rule(333, 4096, 14336)
+    assert gemm_cdna.route(256, 4096, 14336) == table["256"]
+    assert gemm_cdna.route(1000, 4096, 14336) == table["1024"]
+    assert gemm_cdna.route(3000, 4096, 14336) in table.values()
