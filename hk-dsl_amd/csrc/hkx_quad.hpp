@@ -363,6 +363,8 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
       // [0, 4), 16 bytes a store. The tile operand is usually C itself (a gradient added to):
       // read and written by the same lane. Four fragments' reads are issued together and two
       // such groups ahead of their adds and stores (48 registers; a whole block ahead spilled).
+      // 4096 x 4096 over K = 8192, e5m2 x e4m3: 143.6 us on the ring kernel's generic form, 114.9
+      // here; what is left past the 96 us of a bf16 C is this one tile a CU's read and write.
       const uint32_t tb = (uint32_t)e.ta.ld * 4u;
       const __amdgpu_buffer_rsrc_t rt = make_rsrc(e.ta.p, e.ta.p ? (uint32_t)p.M * tb : 0u);
       const bool add = e.ta.p != nullptr;

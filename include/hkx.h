@@ -69,7 +69,8 @@ extern "C" {
 #define HKX_FP8E4M3 3 /* OCP e4m3 (float8_e4m3fn): max 448, no inf */
 #define HKX_INT8 4
 /* fp8 operand pairs with e5m2 (OCP float8_e5m2: max 57344, inf and nan), as ab_dtype only;
- * they run on the 256 x 256 ring tile kernel: */
+ * they run on 256 x 256 ring tiles (the quadrant kernel's dequant forms, else the half-stage
+ * ring kernel): */
 #define HKX_FP8E5M2 5        /* A and B e5m2 */
 #define HKX_FP8_E4M3_E5M2 6  /* A e4m3, B e5m2 (e.g. activations against a gradient) */
 #define HKX_FP8_E5M2_E4M3 7  /* A e5m2, B e4m3 */
@@ -194,7 +195,7 @@ typedef struct HkxEpilogue {
 
 /* HKX_KERNEL_DECODE variant bits. */
 #define HKX_DEC_STREAM 1  /* one workgroup a CU streaming W (M <= 16, or M <= 32 from K =
-                             2048; K a multiple of 1024 up to 32768, no split, unpaired): in
+                             2048; K a multiple of 1024 up to 32768, no split): in
                              blocks of 16 rows, or, with no residual and no vector scale, in
                              chunks of whole rows -- 4 rows at K = 4096, M <= 4, N <= 32768
                              or at M <= 2 any N with W under 2 GiB (one or two chunks a short
@@ -294,14 +295,16 @@ int hkx_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
  * (N, K/32) E8M0 bytes (scale 2^(s - 127) for its row and 32 K), row strides lda, ldb,
  * ldc in elements and sa_ld, sb_ld in bytes. K a multiple of 128, N of 8; sa and sb
  * 4-byte aligned with sa_ld, sb_ld multiples of 4 and >= K/32; C's rows 16-byte aligned.
- * M any. Where the 256 x 256 tiles fill less than half the CUs and K is 2048 or more, K is
- * split over workgroups (1024 K or more each, at most 8) into fp32 shares in ws (hkx_mx_gemm_workspace() bytes; HKX_ERR_WORKSPACE if
- * smaller), summed in split order by a second pass. */
+ * M any. Up to M = 32 the 8-bit decode kernel runs it in one pass; above that the plan of
+ * tiles, K splits and columns of least estimated time. A split's fp32 shares go through ws
+ * (hkx_mx_gemm_workspace() bytes where 256 x 256 tiles fill less than half the CUs and K is 2048
+ * or more; HKX_ERR_WORKSPACE if smaller), summed in split order by a second pass. */
 int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const uint8_t* sa,
                 int64_t sa_ld, const uint8_t* sb, int64_t sb_ld, void* c, int64_t ldc,
                 int32_t m, int32_t n, int32_t k, void* ws, size_t ws_bytes, void* stream);
 
-/* Bytes of fp32 workspace hkx_mx_gemm needs at M x N x K (0 if it runs in one pass). */
+/* Bytes of fp32 workspace hkx_mx_gemm takes at M x N x K (0: none; its plan uses all of it or
+ * less). */
 size_t hkx_mx_gemm_workspace(int32_t m, int32_t n, int32_t k);
 
 /* x bf16 (M, K) -> q fp8-e4m3 (M, K) and s (M, K/32) E8M0 bytes: per 32-column block,
