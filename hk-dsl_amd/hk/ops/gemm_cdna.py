@@ -140,7 +140,7 @@ _COST = {"64x128": (3.2, 0.313, 0.39), "128x128": (5.8, 0.407, 0.51), "128x256":
          "q128": (6.7, 0.662, 0.52), "256x256": (9.7, 0.96, 0.56), "split": (2.2, 6.1e6, 8e6)}
 _COST8 = {"64x128": (4.5, 0.254, 0.32), "128x128": (5.0, 0.412, 0.26), "128x256": (8.3, 0.71, 0.475),
           "256x256": (8.3, 0.89, 0.37), "split": (2.4, 5.3e6, 6.7e6)}
-#: Up to here a call between two measured Ms takes the rule.
+#: Up to here a call between two measured Ms may take the rule.
 BETWEEN_M = 2048
 
 
@@ -160,45 +160,54 @@ def _cost(name: str, m: int, n: int, k: int, fp8: bool = False) -> float:
 
 
 def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
-    """The route when no record or table entry names one: the decode kernel at M <= 32 (bf16),
-    else, for bf16, the tile and split of the least `_cost`. Its numbers are fitted to a sweep
-    of the tiles and splits at 202 shapes (M 33-3300, N 512-24576, K 640-14336, one box): its
-    pick is 0.8% slower than the best on average, 1.27x at worst; the steps it replaced (the
-    largest tile whose count fills three quarters of the CUs, else splits) and the table's
-    nearest M together 12%, 1.66x (300 x 6144 x 4096 on 128 x 256 tiles split 4 ways 46.0 us,
-    on 64 x 128 ones 27.7; 333 x 4096 x 14336 79 -> 63; 256 x 1024 x 1024 12.1 -> 8.7).
+    """The route when no record or table entry names one: the decode kernel at M <= 32 (bf16);
+    else `_steps`, and past 64 rows the tile and split of the least `_cost` where that is 7% or
+    more under the steps'.
 
-    fp8 has two: `_rule8_steps`, and past 64 rows and from K = 1024 the tile and split of the
-    least fp8 cost where that is 7% or more under the steps' (fitted to 279 shapes of scaled_mm
-    with bias, M 33-4096: the steps were 6.6% slower than the best on average and 1.66x at
-    worst, both together 1%: 1300 x 6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x
-    1024 on 64 x 128 ones 8.9 -> 6.5)."""
-    if not fp8:
-        if m <= 32 and k % 128 == 0:
-            return "decode"
-        units = k // 64
-        return min((c for c, (_, least) in _RULE.items()
-                    if m >= least and (CANDIDATES[c].get("splits", 1) == 1
-                                       or units // CANDIDATES[c]["splits"] >= 4)),
-                   key=lambda c: _cost(c, m, n, k))
-    steps = _rule8_steps(m, n, k)
-    if m <= 64 or k < 1024:
+    The bf16 numbers are fitted to a sweep of the tiles and splits at 202 shapes (M 33-3300, N
+    512-24576, K 640-14336, one box; 300 x 6144 x 4096 on 128 x 256 tiles split 4 ways 46.0 us,
+    on 64 x 128 ones 27.7; 333 x 4096 x 14336 79 -> 63; 256 x 1024 x 1024 12.1 -> 8.7). Its 2 to
+    4 weights a shape left part of W cached. With W read from memory (700 MB of weights in turn)
+    few workgroups can't draw its rate, which the cost does not know: at M <= 64, 64 x 16384 x
+    5120 unsplit 49.8 us against 37.9 split in two, 64 x 4096 x 8192 split 4 ways 24.5 against
+    20.1 split 8 ways; so the steps, which fill the CUs, stay there. 256-row tiles split 4 or 8
+    ways lose the same way at few rows or a short K (160 x 16384 x 8192 85.5 us against 76.6, 700
+    x 4096 x 8192 62.0 against 57.8) and gain at more of both (M 300-900, 4096 x 14336: 1.06 to
+    1.34 times the steps' rate), so bf16 takes them past 256 rows from K = 12288. Past 64 rows the cost still gains there (100 x 20480 x 5120 79.8 -> 59.0, 160 x 8192 x 8192
+    63.4 -> 43.9).
+
+    fp8 takes the cost from K = 1024 (fitted to 279 shapes of scaled_mm with bias, M 33-4096: the
+    steps were 6.6% slower than the best on average and 1.66x at worst, both together 1%: 1300 x
+    6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x 1024 on 64 x 128 ones 8.9 ->
+    6.5)."""
+    if not fp8 and m <= 32 and k % 128 == 0:
+        return "decode"
+    steps = _steps(m, n, k, fp8)
+    if m <= 64 or (fp8 and k < 1024):
         return steps
-    best = min((c for c, (cls, least) in _RULE.items()
-                if cls != "q128" and m >= least and (CANDIDATES[c].get("splits", 1) == 1
-                                                     or k // 128 // CANDIDATES[c]["splits"] >= 8)),
-               key=lambda c: _cost(c, m, n, k, True))
-    return best if _cost(best, m, n, k, True) <= 0.93 * _cost(steps, m, n, k, True) else steps
+    kunits, least_units = (k // 128, 8) if fp8 else (k // 64, 4)
+    out = ("q128",) if fp8 else () if m > 256 and k >= 12288 else ("t256k4", "t256k8")
+    best = min((c for c, (_, least) in _RULE.items()
+                if c not in out and m >= least and (CANDIDATES[c].get("splits", 1) == 1
+                                                    or kunits // CANDIDATES[c]["splits"] >= least_units)),
+               key=lambda c: _cost(c, m, n, k, fp8))
+    return best if _less(best, steps, m, n, k, fp8) else steps
 
 
-def _rule8_steps(m: int, n: int, k: int) -> str:
-    """fp8: the largest tile whose count fills three quarters of the CUs -- 256 x 256, 128 x 256,
-    128 x 128; else 64 x 128 tiles or 128 x 128 ones, split over K in powers of two while the
-    workgroups stay within the CUs and each split keeps 16 or more 128-byte K units. From M =
-    129 to 512, 64 x 128 tiles, split only where each split keeps 32 K units (4096 x 4096 at M =
-    256: 12.1-12.2 us on 64 x 128 tiles against 19.6 on 128 x 128 ones split in two; at M = 512
-    13.9 against 21.9; 4096 x 12288 at M = 256 split in two, 23.9 against 29.9 unsplit)."""
-    kunits = k // 128
+def _less(name: str, than: str, m: int, n: int, k: int, fp8: bool = False) -> bool:
+    return _cost(name, m, n, k, fp8) <= 0.93 * _cost(than, m, n, k, fp8)
+
+
+def _steps(m: int, n: int, k: int, fp8: bool = False) -> str:
+    """The largest tile whose count fills three quarters of the CUs -- 256 x 256, 128 x 256 (the
+    quadrant kernel's 128-row form for bf16 up to K = 4096, the 4-wave kernel otherwise), 128 x
+    128; else 64 x 128 tiles (up to M = 128) or 128 x 128 ones, split over K in powers of two
+    while the workgroups stay within the CUs and each split keeps 16 or more 128-byte K units.
+    fp8 from M = 129 to 512: 64 x 128 tiles, split only where each split keeps 32 K units (4096
+    x 4096 at M = 256: 12.1-12.2 us on 64 x 128 tiles against 19.6 on 128 x 128 ones split in
+    two; at M = 512 13.9 against 21.9; 4096 x 12288 at M = 256 split in two, 23.9 against 29.9
+    unsplit)."""
+    kunits = k * (1 if fp8 else 2) // 128
 
     def tiles(bm, bn):
         return math.ceil(m / bm) * math.ceil(n / bn)
@@ -206,13 +215,13 @@ def _rule8_steps(m: int, n: int, k: int) -> str:
     if m > 128 and tiles(256, 256) >= 0.75 * CUS:
         return "t256"
     if m > 64 and tiles(128, 256) >= 0.75 * CUS:
-        return "t128"
+        return "q128" if not fp8 and kunits <= 64 else "t128"
     if m > 64 and tiles(128, 128) >= 0.75 * CUS:
         return "t128x128"
-    bm = 64 if m <= 512 else 128
+    bm = 64 if m <= (512 if fp8 else 128) else 128
     t = tiles(bm, 128)
     most = 8 if bm == 64 else 4  # the split candidates there are
-    per_split = 32 if m > 128 else 16  # K units a split keeps at least
+    per_split = 32 if fp8 and m > 128 else 16  # K units a split keeps at least
     splits = 1
     while t * splits * 2 <= CUS and kunits // (splits * 2) >= per_split and splits < most:
         splits *= 2
@@ -222,8 +231,10 @@ def _rule8_steps(m: int, n: int, k: int) -> str:
 def route(m: int, n: int, k: int, fp8: bool = False) -> str:
     """The candidate an M x N x K call runs: a user record, else the measured table's
     nearest M (log scale) for this N x K, else `rule` (gemm_cdna.py:969-999). Between two
-    measured Ms, 5% or more from the nearer, the rule answers too, up to BETWEEN_M: there the
-    tiles are few waves and the nearest M's pick may leave a wave nearly empty."""
+    measured Ms, 5% or more from the nearer, the rule answers too, past 64 rows up to BETWEEN_M,
+    where its cost is 7% or more under the nearest M's pick: there the tiles are few waves and
+    that pick may leave a wave nearly empty (300 x 24576 x 4096 109.6 -> 83.2 us). A pick that
+    has no cost class stays (1300 x 24576 x 4096: its 225.5 us, the rule's 234.7)."""
     for key in ((m, n, k), "*"):
         if key in OVERRIDE and fits(OVERRIDE[key], m, n, k, fp8):
             return OVERRIDE[key]
@@ -232,9 +243,11 @@ def route(m: int, n: int, k: int, fp8: bool = False) -> str:
         if ent:
             ms = sorted(int(x) for x in ent)
             best = min(ms, key=lambda x: abs(math.log(x) - math.log(m)))
-            if 32 < m <= BETWEEN_M and abs(math.log(best / m)) >= 0.05:
-                return rule(m, n, k)
             name = ent[str(best)]
+            if 64 < m <= BETWEEN_M and abs(math.log(best / m)) >= 0.05 and name in _RULE:
+                other = rule(m, n, k)
+                if _less(other, name, m, n, k):
+                    return other
             if fits(name, m, n, k, fp8):
                 return name
     return rule(m, n, k, fp8)

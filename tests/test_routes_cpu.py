@@ -232,3 +232,13 @@ def test_rules_by_cost(monkeypatch):
     assert gemm_cdna.route(256, 4096, 14336) == table["256"]
     assert gemm_cdna.route(1000, 4096, 14336) == table["1024"]
     assert gemm_cdna.route(3000, 4096, 14336) in table.values()
+
+
+def test_rule_keeps_the_cus_full_on_uncached_weights():
+    """Points measured with W read from memory, where fewer workgroups or 256-row tiles split 4
+    or more ways were 5-26% slower than these (64 x 16384 x 5120 unsplit 49.8 us against 37.9)."""
+    best = {(64, 16384, 5120): "t64x128k2", (40, 4096, 8192): "t64x128k8",
+            (64, 16384, 8192): "t64x128k2", (160, 16384, 8192): "t128x128",
+            (160, 8192, 8192): "t128x128k2", (100, 20480, 5120): "t128x128",
+            (700, 4096, 8192): "t128x128", (333, 4096, 14336): "t256k8"}
+    assert {s: gemm_cdna.rule(*s) for s in best} == best
