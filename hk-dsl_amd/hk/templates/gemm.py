@@ -655,15 +655,17 @@ class _Launch:
         return out
 
 
-#: (epilogue, shapes, dtypes, device, operand signatures) -> a prepared launch: a call
-#: that hits it only fills pointers and launches (templates/gemm.py:728-760).
+#: (epilogue, shapes, dtypes, devices, operand signatures) -> a prepared launch: a call
+#: that hits it only fills pointers and launches (templates/gemm.py:728-760). Every tensor's
+#: device is part of it: a hit makes no check, and a host tensor's address is not one the
+#: kernels may read.
 _LAUNCH: Dict[Tuple, Any] = {}
 
 
 def _sig(item):
     name, v = item
     try:
-        return (name, v.shape, v.dtype, v.stride())
+        return (name, v.shape, v.dtype, v.stride(), v.device)
     except AttributeError:
         return (name, type(v), v)
 
@@ -685,8 +687,8 @@ def _identity(acc):
 
 def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operands):
     key = (epilogue, a.shape, b.shape, a.dtype, b.dtype,
-           out_dtype if out is None else (out.shape, out.dtype, out.stride()),
-           a.device, tuple(map(_sig, operands.items())) if operands else (),
+           out_dtype if out is None else (out.shape, out.dtype, out.stride(), out.device),
+           a.device, b.device, tuple(map(_sig, operands.items())) if operands else (),
            schedule if schedule is None or type(schedule) is str
            else repr(sorted(_sched_record(schedule).items())))
     try:
@@ -727,6 +729,8 @@ def _slow(a, b, epilogue, out, out_dtype, operands, schedule=None):
     if out is not None and (tuple(out.shape) != (m, cn) or out.stride(1) != 1):
         raise ValueError(f"hk.templates.gemm: out is {tuple(out.shape)}, expected ({m}, {cn}) "
                          f"with unit column stride")
+    if out is not None and out.device != a.device:
+        raise ValueError(f"hk.templates.gemm: out is on {out.device}, A on {a.device}")
     ep = bind(epilogue or _identity, operands, m, cn, tdt)
     for name in ep.tensors:
         if operands[name].device != a.device:

@@ -66,3 +66,21 @@ def test_scaled_mm_signatures(m):
         y = hk.ops.scaled_mm(a, w, sa, sb, bias=bias)
     side.synchronize()
     assert torch.equal(y, want)
+
+
+def test_template_refuses_host_tensors_after_a_good_call():
+    """The prepared call is one of the same devices: with B, an operand or out on the host the
+    checks run again and refuse it, before any launch."""
+    m, n, k = 3, 256, 512
+    x, w = torch.randn(m, k, device=DEV).bfloat16(), torch.randn(n, k, device=DEV).bfloat16()
+    b, r = torch.randn(n, device=DEV).bfloat16(), torch.randn(m, n, device=DEV).bfloat16()
+    out = torch.empty(m, n, device=DEV, dtype=torch.bfloat16)
+    kw = dict(epilogue=T.bias_residual, bias=b, residual=r, out=out)
+    T(x, w, **kw)
+    for name, v in (("bias", b), ("residual", r), ("out", out)):
+        with pytest.raises(ValueError, match=f"{name} is on cpu"):
+            T(x, w, **dict(kw, **{name: v.cpu()}))
+    with pytest.raises(ValueError, match="on one GPU"):
+        T(x, w.cpu(), **kw)
+    with pytest.raises(ValueError, match="on one GPU"):
+        T(x.cpu(), w, **kw)
