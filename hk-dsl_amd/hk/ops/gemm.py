@@ -91,8 +91,11 @@ _OP = ctypes.sizeof(nat.HkxOperand)
 def _signature(torch, a, b, scale_a, scale_b, bias):
     """What decides a call's checks and plan, where its operands are passed on as they are:
     tensors, the scales fp32 and contiguous, the bias bf16 and contiguous, all on A's device.
-    None otherwise (numbers, other dtypes, strides): those are converted call by call."""
+    None otherwise (numbers, other dtypes, strides, another device): those are checked and
+    converted call by call."""
     tensor, dev = torch.Tensor, a.device
+    if b.device != dev:
+        return None
     for t in (scale_a, scale_b):
         if (type(t) is not tensor or t.dtype is not torch.float32 or t.device != dev
                 or not t.is_contiguous()):
@@ -147,7 +150,7 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
       a training backward's gradient against a weight); e4m3 x e4m3 runs on every tile
       kernel, a pair with e5m2 on the 256 x 256 ring kernel;
     * scale_a one value or one a row of A ((M,) or (M, 1)), scale_b one value or one a row
-      of B ((N,) or (1, N)); bias (N,);
+      of B ((N,) or (1, N)), taken to A's GPU if they are elsewhere; bias (N,);
     * an fp32 `out` (M, N) takes the product unrounded, and with `accumulate=True` it is
       added to: out += (A @ B^T) * scale_a * scale_b (a weight gradient into its fp32
       main_grad); no bias either way.
@@ -184,6 +187,11 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
     elif tuple(out.shape) != (m, n) or out.dtype != torch.bfloat16 or out.stride(1) != 1:
         raise ValueError(f"scaled_mm: out is {tuple(out.shape)}/{out.dtype}, expected "
                          f"({m}, {n})/bfloat16")
+    for t, what in ((b, "B"), (bias, "bias"), (out, "out")):
+        if t is not None and t.device != a.device:
+            raise ValueError(f"scaled_mm: {what} is on {t.device}, A on {a.device}")
+    if not a.is_cuda:
+        raise ValueError(f"scaled_mm: A and B are on one GPU, got {a.device}")
     sa, sa_ld = _vec(scale_a, m, "scale_a", a.device)
     sb, sb_ld = _vec(scale_b, n, "scale_b", a.device)
     # the library's own choice: the 8-bit decode kernel (no tile operand there, so not for

@@ -31,3 +31,32 @@ def test_a_template_call_with_a_tensor_elsewhere_is_not_the_ready_one(moved, mon
     assert len(checked) == 1   # the second is the first's
     call(moved)
     assert len(checked) == 2
+
+
+def _scaled(**elsewhere):
+    dev = dict(dict.fromkeys(("a", "b", "bias", "out"), "cpu"), **elsewhere)
+    a = torch.zeros(4, 128, device=dev["a"]).to(torch.float8_e4m3fn)
+    b = torch.zeros(8, 128, device=dev["b"]).to(torch.float8_e4m3fn)
+    return a, b, dict(bias=torch.zeros(8, device=dev["bias"]).bfloat16(),
+                      out=torch.zeros(4, 8, device=dev["out"]).bfloat16())
+
+
+def test_scaled_mm_refuses_tensors_on_other_devices():
+    for name in ("b", "bias", "out"):
+        a, b, kw = _scaled(**{name: "meta"})
+        with pytest.raises(ValueError, match="scaled_mm: .* is on meta, A on cpu"):
+            hk.ops.scaled_mm(a, b, 1.0, 1.0, **kw)
+    a, b, kw = _scaled()
+    with pytest.raises(ValueError, match="on one GPU"):
+        hk.ops.scaled_mm(a, b, 1.0, 1.0, **kw)
+
+
+def test_scaled_mm_makes_no_call_ready_with_a_tensor_elsewhere():
+    from hk.ops import gemm as G
+
+    one = torch.ones(1)
+    for name in ("b", "bias"):
+        a, b, kw = _scaled()
+        assert G._signature(torch, a, b, one, one, kw["bias"]) is not None
+        a, b, kw = _scaled(**{name: "meta"})
+        assert G._signature(torch, a, b, one, one, kw["bias"]) is None

@@ -84,3 +84,21 @@ def test_template_refuses_host_tensors_after_a_good_call():
         T(x, w.cpu(), **kw)
     with pytest.raises(ValueError, match="on one GPU"):
         T(x.cpu(), w, **kw)
+
+
+@pytest.mark.parametrize("m", [2, 300])
+def test_scaled_mm_refuses_host_tensors_after_a_good_call(m):
+    n, k = 256, 512
+    a, w = (torch.randn(r, k, device=DEV).to(E4) for r in (m, n))
+    sa, sb = torch.rand(m, 1, device=DEV), torch.rand(n, device=DEV)
+    bias = torch.randn(n, device=DEV).bfloat16()
+    want = hk.ops.scaled_mm(a, w, sa, sb, bias=bias)
+    for args, kw in [((a, w.cpu(), sa, sb), dict(bias=bias)), ((a, w, sa, sb), dict(bias=bias.cpu())),
+                     ((a, w, sa, sb), dict(bias=bias, out=torch.empty(m, n, dtype=torch.bfloat16))),
+                     ((a.cpu(), w, sa, sb), dict(bias=bias))]:
+        with pytest.raises(ValueError, match="is on"):
+            hk.ops.scaled_mm(*args, **kw)
+    with pytest.raises(ValueError, match="on one GPU"):
+        hk.ops.scaled_mm(a.cpu(), w.cpu(), sa, sb)
+    # scales elsewhere are taken to A's GPU, as ever
+    assert torch.equal(hk.ops.scaled_mm(a, w, sa.cpu(), sb.cpu(), bias=bias), want)
