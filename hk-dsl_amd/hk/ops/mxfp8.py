@@ -46,6 +46,13 @@ def _rows16(t):
     return t if st[1] == 1 and st[0] % 16 == 0 and t.data_ptr() % 16 == 0 else t.contiguous()
 
 
+def _on(device, call, **tensors):
+    """The kernels read and write addresses of `device`: a tensor elsewhere is refused."""
+    for name, t in tensors.items():
+        if t is not None and t.device != device:
+            raise ValueError(f"{call}: {name} is on {t.device}, not on {device}")
+
+
 #: (M, N, K) -> the bytes of the workspace its K split needs, asked once a shape.
 _WORKSPACE: dict = {}
 
@@ -65,6 +72,7 @@ def gemm(a, b, sa, sb, out=None):
         raise ValueError(f"mxfp8.gemm: K={k} a multiple of 128 and N={n} of 8")
     if not a.is_cuda or b.device != a.device:
         raise ValueError("mxfp8.gemm: a and b are on one GPU")
+    _on(a.device, "mxfp8.gemm", sa=sa, sb=sb, out=out)
     a, b = _rows16(a), _rows16(b)
     sa = _scales(torch, sa, m, k, "sa")
     sb = _scales(torch, sb, n, k, "sb")
@@ -96,6 +104,10 @@ def quant(x, out=None):
     m, k = x.shape
     if k % 32:
         raise ValueError(f"mxfp8.quant: K={k}, a multiple of 32")
+    if not x.is_cuda:
+        raise ValueError(f"mxfp8.quant: x is on a GPU, got {x.device}")
+    if out is not None:
+        _on(x.device, "mxfp8.quant", q=out[0], s=out[1])
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     q, s = out if out is not None else (

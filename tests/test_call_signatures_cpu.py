@@ -60,3 +60,32 @@ def test_scaled_mm_makes_no_call_ready_with_a_tensor_elsewhere():
         assert G._signature(torch, a, b, one, one, kw["bias"]) is not None
         a, b, kw = _scaled(**{name: "meta"})
         assert G._signature(torch, a, b, one, one, kw["bias"]) is None
+
+
+def test_mxfp8_refuses_tensors_on_other_devices():
+    """On fake GPU tensors (no GPU, no memory): whatever a check lets through would be asked for
+    its address, which they don't have."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    from hk.ops import mxfp8
+
+    m, n, k = 40, 64, 256
+    with FakeTensorMode():
+        def make(**elsewhere):
+            dev = dict(dict.fromkeys(("a", "b", "sa", "sb", "out"), "cuda:0"), **elsewhere)
+            a, b = (torch.empty(r, k, device=dev[t], dtype=torch.float8_e4m3fn)
+                    for r, t in ((m, "a"), (n, "b")))
+            sa, sb = (torch.empty(r, k // 32, device=dev[t], dtype=torch.uint8)
+                      for r, t in ((m, "sa"), (n, "sb")))
+            return a, b, sa, sb, torch.empty(m, n, device=dev["out"], dtype=torch.bfloat16)
+
+        for name in ("a", "b", "sa", "sb", "out"):
+            with pytest.raises(ValueError, match="one GPU" if name in "ab" else f"{name} is on cpu"):
+                mxfp8.gemm(*make(**{name: "cpu"}))
+        x = torch.empty(m, k, device="cuda:0", dtype=torch.bfloat16)
+        a, _, sa, _, _ = make()
+        for q, s in ((a, make(sa="cpu")[2]), (make(a="cpu")[0], sa)):
+            with pytest.raises(ValueError, match="is on cpu"):
+                mxfp8.quant(x, out=(q, s))
+        with pytest.raises(ValueError, match="on a GPU"):
+            mxfp8.quant(torch.empty(m, k, dtype=torch.bfloat16))
