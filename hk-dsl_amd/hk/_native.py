@@ -182,6 +182,20 @@ def stream_of(device) -> int:
     return _RAW_STREAM[0](index)
 
 
+_PLAIN: list = []
+
+
+def empty(like, shape, dtype):
+    """An uninitialised tensor on `like`'s device. new_empty costs the host 0.3 us less than
+    torch.empty, but makes a tensor of `like`'s own class: results are plain tensors."""
+    if _PLAIN and type(like) is _PLAIN[0]:
+        return like.new_empty(shape, dtype=dtype)
+    import torch  # noqa: PLC0415
+
+    _PLAIN[:] = [torch.Tensor]
+    return torch.empty(shape, dtype=dtype, device=like.device)
+
+
 _WS: dict = {}
 
 

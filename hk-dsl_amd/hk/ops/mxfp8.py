@@ -77,7 +77,7 @@ def gemm(a, b, sa, sb, out=None):
     sa = _scales(torch, sa, m, k, "sa")
     sb = _scales(torch, sb, n, k, "sb")
     if out is None:
-        out = a.new_empty((m, n), dtype=torch.bfloat16)
+        out = nat.empty(a, (m, n), torch.bfloat16)
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
         raise ValueError(f"mxfp8.gemm: out is bf16 ({m}, {n}) with unit column stride")
     L = nat.lib()
@@ -111,8 +111,7 @@ def quant(x, out=None):
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
     q, s = out if out is not None else (
-        x.new_empty((m, k), dtype=torch.float8_e4m3fn),
-        x.new_empty((m, k // 32), dtype=torch.uint8))
+        nat.empty(x, (m, k), torch.float8_e4m3fn), nat.empty(x, (m, k // 32), torch.uint8))
     nat.check(nat.lib().hkx_mx_quant(x.data_ptr(), x.stride(0), q.data_ptr(), q.stride(0),
                                      s.data_ptr(), s.stride(0), m, k,
                                      nat.stream_of(x.device)))

@@ -699,7 +699,7 @@ def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operan
         got = _slow(a, b, epilogue, out, out_dtype, operands, schedule)
     go, shape, dtype = got
     if out is None:
-        out = a.new_empty(shape, dtype=dtype)
+        out = nat.empty(a, shape, dtype)
     return go(a, b, out, operands)
 
 

@@ -89,3 +89,23 @@ def test_mxfp8_refuses_tensors_on_other_devices():
                 mxfp8.quant(x, out=(q, s))
         with pytest.raises(ValueError, match="on a GPU"):
             mxfp8.quant(torch.empty(m, k, dtype=torch.bfloat16))
+
+
+def test_results_are_plain_tensors():
+    """Also of a subclass of Tensor: C is not one of A's class."""
+    from hk import _native as nat
+
+    class Tagged(torch.Tensor):
+        pass
+
+    def go(a, b, out, operands):
+        return out
+
+    a, b = torch.zeros(4, 64).bfloat16(), torch.zeros(8, 64).bfloat16()
+    for x in (a, a.as_subclass(Tagged), torch.nn.Parameter(a, requires_grad=False)):
+        y = nat.empty(x, (4, 8), torch.float32)
+        assert type(y) is torch.Tensor and y.shape == (4, 8) and y.dtype is torch.float32
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(T, "_LAUNCH", {})
+            mp.setattr(T, "_slow", lambda *args: (go, (4, 8), torch.bfloat16))
+            assert type(T(x, b)) is torch.Tensor

@@ -102,3 +102,21 @@ def test_scaled_mm_refuses_host_tensors_after_a_good_call(m):
         hk.ops.scaled_mm(a.cpu(), w.cpu(), sa, sb)
     # scales elsewhere are taken to A's GPU, as ever
     assert torch.equal(hk.ops.scaled_mm(a, w, sa.cpu(), sb.cpu(), bias=bias), want)
+
+
+def test_results_are_plain_tensors():
+    class Tagged(torch.Tensor):
+        pass
+
+    from hk.ops import mxfp8
+
+    x = torch.randn(40, 512, device=DEV).bfloat16().as_subclass(Tagged)
+    w = torch.randn(256, 512, device=DEV)
+    assert type(T(x, w.bfloat16())) is torch.Tensor
+    q, s = mxfp8.quant(x)
+    assert type(q) is torch.Tensor and type(s) is torch.Tensor
+    wq, ws = mxfp8.quant(w.bfloat16())
+    assert type(mxfp8.gemm(q.as_subclass(Tagged), wq, s, ws)) is torch.Tensor
+    one = torch.ones(1, device=DEV)
+    for _ in range(2):
+        assert type(hk.ops.scaled_mm(q.as_subclass(Tagged), wq, one, one)) is torch.Tensor
