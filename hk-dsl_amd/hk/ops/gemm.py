@@ -198,11 +198,15 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
     # accumulate, and an fp32 out keeps the tiles' sums)
     decode8 = (code == nat.FP8E4M3 and schedule is None and not fp32_out
                and gemm_cdna.decode8(m, n, k))
-    if code != nat.FP8E4M3:
-        name = "t256"   # a pair with e5m2: the ring kernel's generic form
+    if decode8:
+        tile = dict(kernel=nat.KERNEL_AUTO)
     else:
-        name = schedule or gemm_cdna.route(m, n, k, fp8=True)
-    rec = gemm_cdna.resolve(gemm_cdna.CANDIDATES[name], m, n, k, fp8=True)
+        # a pair with e5m2: 256 x 256 ring tiles
+        name = "t256" if code != nat.FP8E4M3 else schedule or gemm_cdna.route(m, n, k, fp8=True)
+        rec = gemm_cdna.resolve(gemm_cdna.CANDIDATES[name], m, n, k, fp8=True)
+        tile = dict(kernel=nat.KERNEL_TILE, tile_m=rec["tile_m"], tile_n=rec["tile_n"],
+                    schedule=nat.SCHEDULES[rec["schedule"]], splits=rec.get("splits", 1),
+                    variant=0 if code != nat.FP8E4M3 else rec.get("variant", 0))
     ep = nat.HkxEpilogue()
     ep.form = nat.EP_FUSED
     ep.cmul = 1.0
@@ -220,11 +224,7 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
         keep.append(bb)
         ep.ops[2] = nat.HkxOperand(bb.data_ptr(), nat.ROW, nat.BF16, 1)
         ep.row_add, ep.nops = 2, 3
-    args = nat.gemm_args(a, b, out, kernel=nat.KERNEL_AUTO if decode8 else nat.KERNEL_TILE,
-                         tile_m=rec["tile_m"],
-                         tile_n=rec["tile_n"], schedule=nat.SCHEDULES[rec["schedule"]],
-                         variant=0 if code != nat.FP8E4M3 else rec.get("variant", 0),
-                         splits=rec.get("splits", 1), ep=ep)
+    args = nat.gemm_args(a, b, out, ep=ep, **tile)
     args.ab_dtype = code
     nat.run(args, a.device)
     if key is not None and len(_READY) < _READY_CAP:

@@ -17,6 +17,7 @@ contract over this build's kernels:
 
 from __future__ import annotations
 
+import functools
 import json
 import math
 import os
@@ -159,6 +160,7 @@ def _cost(name: str, m: int, n: int, k: int, fp8: bool = False) -> float:
     return t if splits == 1 else t + launch + splits * m * n * 8 / share_rate
 
 
+@functools.lru_cache(maxsize=8192)
 def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
     """The route when no record or table entry names one: the decode kernel at M <= 32 (bf16);
     else `_steps`, and past 64 rows the tile and split of the least `_cost` where that is 7% or
@@ -173,13 +175,17 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
     20.1 split 8 ways; so the steps, which fill the CUs, stay there. 256-row tiles split 4 or 8
     ways lose the same way at few rows or a short K (160 x 16384 x 8192 85.5 us against 76.6, 700
     x 4096 x 8192 62.0 against 57.8) and gain at more of both (M 300-900, 4096 x 14336: 1.06 to
-    1.34 times the steps' rate), so bf16 takes them past 256 rows from K = 12288. Past 64 rows the cost still gains there (100 x 20480 x 5120 79.8 -> 59.0, 160 x 8192 x 8192
-    63.4 -> 43.9).
+    1.34 times the steps' rate), so bf16 takes them past 256 rows from K = 12288. Past 64 rows
+    the cost still gains there (100 x 20480 x 5120 79.8 -> 59.0, 160 x 8192 x 8192 63.4 -> 43.9).
 
     fp8 takes the cost from K = 1024 (fitted to 279 shapes of scaled_mm with bias, M 33-4096: the
     steps were 6.6% slower than the best on average and 1.66x at worst, both together 1%: 1300 x
     6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x 1024 on 64 x 128 ones 8.9 ->
-    6.5)."""
+    6.5).
+
+    The answer depends on the arguments alone and is kept: the costs of a shape take the host
+    15-30 us, and a scaled_mm call that is not a prepared one (out, an fp32 sum, a number for a
+    scale) asks every time."""
     if not fp8 and m <= 32 and k % 128 == 0:
         return "decode"
     steps = _steps(m, n, k, fp8)

@@ -242,3 +242,19 @@ def test_rule_keeps_the_cus_full_on_uncached_weights():
             (160, 8192, 8192): "t128x128k2", (100, 20480, 5120): "t128x128",
             (700, 4096, 8192): "t128x128", (333, 4096, 14336): "t256k8"}
     assert {s: gemm_cdna.rule(*s) for s in best} == best
+
+
+def test_a_shapes_route_is_worked_out_once(monkeypatch):
+    """Calls that are not prepared ask the route every time: only the first evaluates the costs,
+    and a user's record still answers at once."""
+    monkeypatch.setattr(gemm_cdna, "OVERRIDE", {})
+    asked = []
+    cost = gemm_cdna._cost
+    monkeypatch.setattr(gemm_cdna, "_cost", lambda *a: asked.append(a) or cost(*a))
+    shape = (517, 4096, 4224)
+    first = gemm_cdna.route(*shape, fp8=True)
+    assert asked
+    asked.clear()
+    assert gemm_cdna.route(*shape, fp8=True) == first and not asked
+    gemm_cdna.OVERRIDE[shape] = "t64"
+    assert gemm_cdna.route(*shape, fp8=True) == "t64"
