@@ -196,6 +196,17 @@ def empty(like, shape, dtype):
     return torch.empty(shape, dtype=dtype, device=like.device)
 
 
+def remember(store: dict, key, value, cap: int) -> None:
+    """Keep `value` under `key` in a store of at most `cap`: when full the oldest gives way, so
+    what a program calls now is always kept (a shape still in use comes back at its next call)."""
+    while len(store) >= cap:
+        try:
+            store.pop(next(iter(store)), None)
+        except (StopIteration, RuntimeError):  # another thread's turn came between
+            pass
+    store[key] = value
+
+
 _WS: dict = {}
 
 

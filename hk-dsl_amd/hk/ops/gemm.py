@@ -77,7 +77,7 @@ def _pair_code(a, b) -> int:
 
 #: Call signature -> a call made ready (`_ready`), so that a call of the same shapes, dtypes
 #: and forms only fills in its pointers: the checks and the args struct took 15 us a call, twice
-#: the decode kernel. Entries hold no tensor and no address.
+#: the decode kernel. Entries hold no tensor and no address; past _READY_CAP the oldest goes.
 _READY: dict = {}
 _READY_CAP = 4096
 _ARGS = nat.HkxGemmArgs
@@ -227,8 +227,8 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
     args = nat.gemm_args(a, b, out, ep=ep, **tile)
     args.ab_dtype = code
     nat.run(args, a.device)
-    if key is not None and len(_READY) < _READY_CAP:
-        _READY[key] = _ready(args, (m, n))
+    if key is not None:
+        nat.remember(_READY, key, _ready(args, (m, n)), _READY_CAP)
     del keep
     return out
 

@@ -84,8 +84,7 @@ def gemm(a, b, sa, sb, out=None):
     nws = _WORKSPACE.get((m, n, k))
     if nws is None:
         nws = L.hkx_mx_gemm_workspace(m, n, k)
-        if len(_WORKSPACE) < 4096:
-            _WORKSPACE[(m, n, k)] = nws
+        nat.remember(_WORKSPACE, (m, n, k), nws, 4096)
     ws = nat.workspace(a.device, nws) if nws else None
     nat.check(L.hkx_mx_gemm(
         a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), sa.data_ptr(), sa.stride(0),

@@ -109,3 +109,13 @@ def test_results_are_plain_tensors():
             mp.setattr(T, "_LAUNCH", {})
             mp.setattr(T, "_slow", lambda *args: (go, (4, 8), torch.bfloat16))
             assert type(T(x, b)) is torch.Tensor
+
+
+def test_a_full_store_takes_the_newest_call():
+    from hk import _native as nat
+
+    store = {}
+    for key in range(10):
+        nat.remember(store, key, key * key, 4)
+        assert store[key] == key * key and len(store) <= 4
+    assert sorted(store) == [6, 7, 8, 9]

@@ -120,3 +120,16 @@ def test_results_are_plain_tensors():
     one = torch.ones(1, device=DEV)
     for _ in range(2):
         assert type(hk.ops.scaled_mm(q.as_subclass(Tagged), wq, one, one)) is torch.Tensor
+
+
+def test_a_new_shape_is_made_ready_when_the_store_is_full(monkeypatch):
+    from hk.ops import gemm as G
+
+    monkeypatch.setattr(G, "_READY", {})
+    monkeypatch.setattr(G, "_READY_CAP", 3)
+    w, one = torch.randn(64, 256, device=DEV).to(E4), torch.ones(1, device=DEV)
+    for m in (1, 2, 3, 4, 50, 70):
+        a = torch.randn(m, 256, device=DEV).to(E4)
+        want = hk.ops.scaled_mm(a, w, one, one)
+        assert len(G._READY) <= 3 and G._signature(torch, a, w, one, one, None) in G._READY
+        assert torch.equal(hk.ops.scaled_mm(a, w, one, one), want)
