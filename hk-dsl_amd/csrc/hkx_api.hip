@@ -74,7 +74,6 @@ struct Plan {
 };
 
 int cu_count();
-int wave_cut(int m, int n, int outw);
 
 bool tile_shape_ok(int bm, int bn) {
   return (bm == 256 && bn == 256) || (bm == 128 && bn == 256) || (bm == 64 && bn == 256) ||
@@ -128,17 +127,11 @@ void auto_choose(const HkxGemmArgs* a, int* kernel, int* bm, int* bn, int* split
 
 hkx::Fused make_fused(const HkxEpilogue& ep);
 
-// Whether HKX_KERNEL_AUTO runs a call on the 8-bit decode kernel: fp8 e4m3, M <= 32, no
-// epilogue or the dequant form, and a shape where it beats the 64 x 128 tiles (split over K
-// past K = 2048, their shares summed by a second launch). Measured, graph replays over rotated
-// weights, tiles -> decode kernel: 4096 x 4096 at M = 16 10.2 -> 5.9 us, 24576 x 4096 at M = 32
-// 27.0 -> 20.4, 1024 x 8192 at M = 32 10.2 -> 9.5, 8192 x 512 at M = 32 5.6 -> 5.5. Where K is
-// short and the row blocks more than two a CU, the tiles' one launch wins (12288 x 1024: 6.7
-// against 7.2; 32768 x 512: 6.5 against 9.2; 12288 x 2048 at M = 32: 8.6 against 9.3, at M = 16
-// 8.5 against 8.0), so those stay there. hk.ops.gemm_cdna.decode8 is the same rule.
+// Whether HKX_KERNEL_AUTO runs a call on the 8-bit decode kernel: fp8 e4m3, no epilogue or the
+// dequant form, and a shape skinny_wins names.
 bool auto_skinny(const HkxGemmArgs* a) {
-  return a->kernel == HKX_KERNEL_AUTO && a->ab_dtype == HKX_FP8E4M3 && a->m <= hkx::kSkinnyM &&
-         (a->n <= 8192 || a->k > 2048 || (a->k >= 1792 && a->m <= 16)) &&
+  return a->kernel == HKX_KERNEL_AUTO && a->ab_dtype == HKX_FP8E4M3 &&
+         hkx::skinny_wins(a->m, a->n, a->k) &&
          (a->ep.form == HKX_EP_NONE || a->ep.form == HKX_EP_FUSED) && hkx::skinny_ep_ok(make_fused(a->ep));
 }
 
@@ -334,7 +327,7 @@ int make_plan(const HkxGemmArgs* a, Plan* p) {
     // the rest of N past the whole waves, split over K so that its tiles fill the CUs
     // (at least 4 K units a split, at most 8 splits)
     const int outw = pair ? p->tile_n / 2 : p->tile_n;
-    const int cut = wave_cut(a->m, a->n, outw);
+    const int cut = hkx::wave_cut(a->m, a->n, outw, cu_count());
     if (cut < a->n) {
       const int rest = a->n - cut;
       const int tiles = ((a->m + 255) / 256) * ((rest + outw - 1) / outw);
@@ -429,29 +422,6 @@ int cu_count() {
     cached[dev] = n;
   }
   return cached[dev];
-}
-
-// The columns of N whose 256 x 256 tiles fill whole waves of one-a-CU workgroups at M's
-// tile rows (0 where one wave takes more than N has): the reference's wave_cut
-// (python/hk/ops/gemm_cdna.py:923-930).
-int wave_cut(int m, int n, int outw) {
-  const int mb = (m + 255) / 256, cus = cu_count();
-  if (mb > cus) return 0;
-  const int per = cus / mb;
-  return (n / outw / per) * per * outw;
-}
-
-// Whether a paired decode call the stream kernel can take also runs on it. Up to K = 4096
-// (X held in registers) it always does: 1.06-2.4x the blocked kernel at 1536 to 28672 rows of
-// W, M = 1 to 32. Past that X is streamed with every 16-row block, and where those blocks are
-// more than the CUs but at most two a CU, the blocked kernel's 32-row workgroups are one wave
-// and read X half as often: it stays there above M = 16 (8192 x 6144 at M = 24: 24.6 against
-// 27.6 us) or where the last blocks leave CUs idle (6144 x 5120 at M = 8: 16.5 against 17.4);
-// on either side the stream kernel wins (4096 x 8192 at M = 16: 24.3 -> 16.1 us, 12288 x 5120
-// at M = 16: 34.5 -> 26.6, 28672 x 8192 at M = 1: 95.3 -> 78.5).
-bool pair_streams(int m, int n, int k) {
-  const int blocks = (n + 7) / 8, cus = cu_count();
-  return k <= 4096 || blocks <= cus || blocks > 2 * cus || (m <= 16 && blocks > cus * 7 / 4);
 }
 
 hipError_t tile_dispatch(const Plan& p, const hkx::TileArgs& t, bool fp8, int mode, dim3 grid,
@@ -676,7 +646,7 @@ int hkx_gemm(const HkxGemmArgs* args, void* stream) {
           o->p = (const uint8_t*)o->p + (int64_t)c0 * elem_bytes(o->dt);
       return r;
     };
-    const int cut = (p.variant & HKX_RING_WAVESPLIT) && !p.via_ws ? wave_cut(a.m, a.n, outw)
+    const int cut = (p.variant & HKX_RING_WAVESPLIT) && !p.via_ws ? hkx::wave_cut(a.m, a.n, outw, cu_count())
                     : p.sk_cut;
     if (cut < a.n && ((p.variant & HKX_RING_WAVESPLIT) ? cut > 0 : p.sk_splits > 0)) {
       if (cut > 0) {  // whole waves of 256 x 256 tiles on the ring kernel
@@ -777,7 +747,7 @@ int hkx_gemm(const HkxGemmArgs* args, void* stream) {
     }
     const int gw = std::min((a.n + 7) / 8, cu_count());
     const bool stream = (p.variant & HKX_DEC_STREAM) && hkx::stream_takes(d, p.splits) &&
-                        (!p.pair || pair_streams(a.m, a.n, a.k));
+                        (!p.pair || hkx::pair_streams(a.m, a.n, a.k, cu_count()));
     if (stream && !p.pair && hkx::roww_takes(d, gw)) {
       rc = launched(hkx::launch_roww(d, dim3(gw), s), "decode GEMM");
     } else if (stream && hkx::rows_takes(d, p.pair)) {
@@ -835,83 +805,9 @@ int hkx_gemm_noalloc(const HkxGemmArgs* args, void* stream) {
   return hkx_gemm(&a, stream);
 }
 
-// How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles of the
-// 4-wave kernel, K split over workgroups into fp32 shares a second launch sums; or, for the
-// first `cut` columns, on whole waves of 256 x 256 quadrant tiles, the rest of N on the tiles
-// (cut = n: all of it).
-struct MxPlan {
-  int bm, bn, splits, cut;
-  size_t ws_bytes;  // the workspace a caller passes (mx_share_bytes)
-};
-
-// A plan's estimated time in us: waves of one-a-CU workgroups, each a fixed part and a time a
-// 128-K unit by tile shape, or W's bytes at the rate these tiles stream them; a split adds its
-// sum's launch and the shares' round trip. Fitted to a sweep of every tile and split at 165
-// shapes (M 33-6000, N 768-16384, K 512-14336, one box): its pick is 0.3% slower than the best
-// on average, 1.13x at worst (M = 1000, 1024 x 8192). Before, every call ran on 256 x 256
-// tiles: 5120 x 4096 at M = 256 30.7 -> 14.9 us, 4096 x 1280 at M = 512 22.4 -> 8.7, 12800 x
-// 6144 at M = 256 51.1 -> 40.4, 1024 x 8192 at M = 64 21.3 -> 10.0.
-static double mx_cost(int m, int n, int k, int bm, int bn, int splits) {
-  const double fixed = bm == 256 ? 6.3 : bm == 64 ? 4.3 : bn == 128 ? 5.9 : 7.5;
-  const double unit = bm == 256 ? 1.53 : bm == 64 ? 0.47 : bn == 128 ? 0.56 : 0.90;
-  const long tiles = (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * splits;
-  const int cus = cu_count(), kper = (k / 128 + splits - 1) / splits;
-  const long waves = (tiles + cus - 1) / cus;
-  double t = fixed * (1.0 + 0.4 * (waves - 1)) + unit * kper * waves;
-  t = std::max(t, 5.0 + (double)n * k / 7.5e6);
-  if (splits > 1) t += 2.2 + (double)splits * m * n * 8.0 / 5.4e6;
-  return t;
+size_t hkx_mx_gemm_workspace(int32_t m, int32_t n, int32_t k) {
+  return hkx::mx_plan(m, n, k, cu_count()).ws_bytes;
 }
-
-// The fp32 shares a call may use, and asks its caller for: up to 8 splits of 8 K units or more
-// of all of C where 256 x 256 tiles fill less than half the CUs, none otherwise (or where a
-// share would span 4 GiB). The plan below stays within it.
-static size_t mx_share_bytes(int32_t m, int32_t n, int32_t k) {
-  if (m <= hkx::kSkinnyM) return 0;
-  const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
-  const int cu = cu_count();
-  if (2 * tiles > cu || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 0;
-  const int s = std::min(std::min(cu / tiles, (k / 128) / 8), 8);
-  if (s < 2) return 0;
-  const int kper = (k / 128 + s - 1) / s;  // no empty last split
-  return (size_t)((k / 128 + kper - 1) / kper) * m * n * 4u;
-}
-
-static MxPlan mx_plan(int32_t m, int32_t n, int32_t k) {
-  if (m < 1 || n < 1 || k < 128 || k % 128) return {256, 256, 1, n, 0};
-  if (m <= hkx::kSkinnyM) return {0, 0, 1, 0, 0};
-  // the best tile and split of some columns: splits of 4 K units or more, no empty one, their
-  // shares within the workspace
-  const size_t room = mx_share_bytes(m, n, k);
-  struct Pick {
-    int bm, bn, splits;
-    double t;
-  };
-  auto best = [&](int cols, bool small_only) {
-    static const int kTiles[4][3] = {{64, 128, 8}, {128, 128, 4}, {128, 256, 2}, {256, 256, 1}};
-    Pick b{256, 256, 1, 1e30};
-    for (int i = 0; i < (small_only ? 3 : 4); ++i)
-      for (int s = 1; s <= kTiles[i][2]; s *= 2) {
-        const int units = k / 128, kper = (units + s - 1) / s;
-        if (s > 1 && (units / s < 4 || (units + kper - 1) / kper != s || (size_t)s * m * cols * 4u > room))
-          continue;
-        const double t = mx_cost(m, cols, k, kTiles[i][0], kTiles[i][1], s);
-        if (t < b.t) b = {kTiles[i][0], kTiles[i][1], s, t};
-      }
-    return b;
-  };
-  const Pick all = best(n, false);
-  const int cut = wave_cut(m, n, 256);
-  if (cut > 0 && cut < n) {  // whole waves on 256 x 256 tiles and the rest on smaller ones
-    const Pick rest = best(n - cut, true);
-    if (mx_cost(m, cut, k, 256, 256, 1) + rest.t < all.t)
-      return {rest.bm, rest.bn, rest.splits, cut, room};
-  }
-  if (all.bm == 256) return {256, 256, 1, n, room};
-  return {all.bm, all.bn, all.splits, 0, room};
-}
-
-size_t hkx_mx_gemm_workspace(int32_t m, int32_t n, int32_t k) { return mx_plan(m, n, k).ws_bytes; }
 
 int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const uint8_t* sa,
                 int64_t sa_ld, const uint8_t* sb, int64_t sb_ld, void* c, int64_t ldc, int32_t m,
@@ -947,7 +843,7 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   t.M = m;
   t.N = n;
   t.kt_total = t.kt_split = k / 128;
-  const MxPlan q = mx_plan(m, n, k);
+  const hkx::MxPlan q = hkx::mx_plan(m, n, k, cu_count());
   t.wgm = kWgmRows;
   t.pair_off = n;
   t.c_dt = HKX_BF16;

@@ -7,6 +7,7 @@
 
 #include "hkx_decode.hpp"
 #include "hkx_reduce.hpp"
+#include "hkx_rules.hpp"
 #include "hkx_skinny.hpp"
 #include "hkx_tile.hpp"
 #include "hkx_tile4.hpp"
@@ -19,13 +20,6 @@ hipError_t launch_tile(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStre
 template <int BM, int BN>
 hipError_t launch_tile4(const TileArgs& a, bool fp8, int mode, dim3 grid,
                         hipStream_t s);
-
-// Whether a grid of the 4-wave kernel's 128-column tiles runs its two-a-CU form: past one
-// workgroup a CU, where the second hides what a lone wave a SIMD waits for and fills the last
-// wave's idle CUs (700 x 4096 x 4096 on 64 x 128 tiles 44.5 -> 39.4 us, 2048 x 4096 x 4096 on
-// 128 x 128 ones 79.4 -> 72.1, 333 x 4096 x 14336 split 4 ways 79.2 -> 74.6). Up to one a CU
-// the one-a-CU form's deeper stages stay.
-inline bool tile4_two(const TileArgs& a, dim3 grid) { return grid.x * grid.y > (unsigned)a.cus; }
 
 // A 16- or 8-bit C with the fused form's activation fixed at compile time (the epilogue is
 // then straight-line code); any other store takes it at run time.
@@ -68,9 +62,7 @@ hipError_t launch_tile4_mx(const TileArgs& a, int bm, int bn, bool f32_shares, d
 hipError_t launch_mx_quant(const void* x, int64_t ldx, void* q, int64_t ldq, uint8_t* sc,
                            int64_t lds, int m, int k, hipStream_t s);
 
-// The 8-bit decode kernel: M up to kSkinnyM, fp8 e4m3 with the epilogues skinny_ep_ok accepts,
-// or MX.
-constexpr int kSkinnyM = 32;
+// The 8-bit decode kernel (hkx_rules.hpp has its rule).
 bool skinny_ep_ok(const Fused& e);
 hipError_t launch_skinny(SkinnyArgs a, bool mx, int cus, hipStream_t s);
 
@@ -135,7 +127,7 @@ hipError_t launch_reduce(const ReduceArgs& a, const HkxEpilogue& ep, bool progra
   template <>                                                                                \
   hipError_t launch_tile4<BM, BN>(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s) { \
     if constexpr (BN == 128) {                                                               \
-      if (tile4_two(a, grid)) return fp8 ? launch_res<true, 2>(a, mode, grid, s) : launch_res<false, 2>(a, mode, grid, s); \
+      if (tile4_two(grid.x * grid.y, a.cus)) return fp8 ? launch_res<true, 2>(a, mode, grid, s) : launch_res<false, 2>(a, mode, grid, s); \
     }                                                                                        \
     return fp8 ? launch_res<true, 1>(a, mode, grid, s) : launch_res<false, 1>(a, mode, grid, s); \
   }

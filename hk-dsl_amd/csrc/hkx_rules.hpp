@@ -1,0 +1,131 @@
+// The library's choices between kernels, by shape and CUs alone: plain C++, no HIP, so that a
+// host program can ask them.
+#pragma once
+
+#include <algorithm>
+#include <cstddef>
+#include <cstdint>
+
+namespace hkx {
+
+// The 8-bit decode kernel: M up to kSkinnyM, fp8 e4m3 with the epilogues skinny_ep_ok accepts,
+// or MX.
+constexpr int kSkinnyM = 32;
+
+// Whether an e4m3 call of M <= 32 is faster there than on the 64 x 128 tiles (split over K past
+// K = 2048, their shares summed by a second launch). Measured, graph replays over rotated
+// weights, tiles -> decode kernel: 4096 x 4096 at M = 16 10.2 -> 5.9 us, 24576 x 4096 at M = 32
+// 27.0 -> 20.4, 1024 x 8192 at M = 32 10.2 -> 9.5, 8192 x 512 at M = 32 5.6 -> 5.5. Where K is
+// short and the row blocks more than two a CU, the tiles' one launch wins (12288 x 1024: 6.7
+// against 7.2; 32768 x 512: 6.5 against 9.2; 12288 x 2048 at M = 32: 8.6 against 9.3, at M = 16
+// 8.5 against 8.0), so those stay there. hk.ops.gemm_cdna.decode8 is the same rule.
+inline bool skinny_wins(int m, int n, int k) {
+  return m <= kSkinnyM && (n <= 8192 || k > 2048 || (k >= 1792 && m <= 16));
+}
+
+// The columns of N whose 256 x 256 tiles fill whole waves of one-a-CU workgroups at M's
+// tile rows (0 where one wave takes more than N has): the reference's wave_cut
+// (python/hk/ops/gemm_cdna.py:923-930).
+inline int wave_cut(int m, int n, int outw, int cus) {
+  const int mb = (m + 255) / 256;
+  if (mb > cus) return 0;
+  const int per = cus / mb;
+  return (n / outw / per) * per * outw;
+}
+
+// Whether a paired decode call the stream kernel can take also runs on it. Up to K = 4096
+// (X held in registers) it always does: 1.06-2.4x the blocked kernel at 1536 to 28672 rows of
+// W, M = 1 to 32. Past that X is streamed with every 16-row block, and where those blocks are
+// more than the CUs but at most two a CU, the blocked kernel's 32-row workgroups are one wave
+// and read X half as often: it stays there above M = 16 (8192 x 6144 at M = 24: 24.6 against
+// 27.6 us) or where the last blocks leave CUs idle (6144 x 5120 at M = 8: 16.5 against 17.4);
+// on either side the stream kernel wins (4096 x 8192 at M = 16: 24.3 -> 16.1 us, 12288 x 5120
+// at M = 16: 34.5 -> 26.6, 28672 x 8192 at M = 1: 95.3 -> 78.5).
+inline bool pair_streams(int m, int n, int k, int cus) {
+  const int blocks = (n + 7) / 8;
+  return k <= 4096 || blocks <= cus || blocks > 2 * cus || (m <= 16 && blocks > cus * 7 / 4);
+}
+
+// Whether a grid of the 4-wave kernel's 128-column tiles runs its two-a-CU form: past one
+// workgroup a CU, where the second hides what a lone wave a SIMD waits for and fills the last
+// wave's idle CUs (700 x 4096 x 4096 on 64 x 128 tiles 44.5 -> 39.4 us, 2048 x 4096 x 4096 on
+// 128 x 128 ones 79.4 -> 72.1, 333 x 4096 x 14336 split 4 ways 79.2 -> 74.6). Up to one a CU
+// the one-a-CU form's deeper stages stay.
+inline bool tile4_two(unsigned wgs, int cus) { return wgs > (unsigned)cus; }
+
+// How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles of the
+// 4-wave kernel, K split over workgroups into fp32 shares a second launch sums; or, for the
+// first `cut` columns, on whole waves of 256 x 256 quadrant tiles, the rest of N on the tiles
+// (cut = n: all of it).
+struct MxPlan {
+  int bm, bn, splits, cut;
+  size_t ws_bytes;  // the workspace a caller passes (mx_share_bytes)
+};
+
+// A plan's estimated time in us: waves of one-a-CU workgroups, each a fixed part and a time a
+// 128-K unit by tile shape, or W's bytes at the rate these tiles stream them; a split adds its
+// sum's launch and the shares' round trip. Fitted to a sweep of every tile and split at 165
+// shapes (M 33-6000, N 768-16384, K 512-14336, one box): its pick is 0.3% slower than the best
+// on average, 1.13x at worst (M = 1000, 1024 x 8192). Before, every call ran on 256 x 256
+// tiles: 5120 x 4096 at M = 256 30.7 -> 14.9 us, 4096 x 1280 at M = 512 22.4 -> 8.7, 12800 x
+// 6144 at M = 256 51.1 -> 40.4, 1024 x 8192 at M = 64 21.3 -> 10.0.
+inline double mx_cost(int m, int n, int k, int bm, int bn, int splits, int cus) {
+  const double fixed = bm == 256 ? 6.3 : bm == 64 ? 4.3 : bn == 128 ? 5.9 : 7.5;
+  const double unit = bm == 256 ? 1.53 : bm == 64 ? 0.47 : bn == 128 ? 0.56 : 0.90;
+  const long tiles = (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn) * splits;
+  const int kper = (k / 128 + splits - 1) / splits;
+  const long waves = (tiles + cus - 1) / cus;
+  double t = fixed * (1.0 + 0.4 * (waves - 1)) + unit * kper * waves;
+  t = std::max(t, 5.0 + (double)n * k / 7.5e6);
+  if (splits > 1) t += 2.2 + (double)splits * m * n * 8.0 / 5.4e6;
+  return t;
+}
+
+// The fp32 shares a call may use, and asks its caller for: up to 8 splits of 8 K units or more
+// of all of C where 256 x 256 tiles fill less than half the CUs, none otherwise (or where a
+// share would span 4 GiB). The plan below stays within it.
+inline size_t mx_share_bytes(int32_t m, int32_t n, int32_t k, int cus) {
+  if (m <= kSkinnyM) return 0;
+  const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
+  if (2 * tiles > cus || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 0;
+  const int s = std::min(std::min(cus / tiles, (k / 128) / 8), 8);
+  if (s < 2) return 0;
+  const int kper = (k / 128 + s - 1) / s;  // no empty last split
+  return (size_t)((k / 128 + kper - 1) / kper) * m * n * 4u;
+}
+
+inline MxPlan mx_plan(int32_t m, int32_t n, int32_t k, int cus) {
+  if (m < 1 || n < 1 || k < 128 || k % 128) return {256, 256, 1, n, 0};
+  if (m <= kSkinnyM) return {0, 0, 1, 0, 0};
+  // the best tile and split of some columns: splits of 4 K units or more, no empty one, their
+  // shares within the workspace
+  const size_t room = mx_share_bytes(m, n, k, cus);
+  struct Pick {
+    int bm, bn, splits;
+    double t;
+  };
+  auto best = [&](int cols, bool small_only) {
+    static const int kTiles[4][3] = {{64, 128, 8}, {128, 128, 4}, {128, 256, 2}, {256, 256, 1}};
+    Pick b{256, 256, 1, 1e30};
+    for (int i = 0; i < (small_only ? 3 : 4); ++i)
+      for (int s = 1; s <= kTiles[i][2]; s *= 2) {
+        const int units = k / 128, kper = (units + s - 1) / s;
+        if (s > 1 && (units / s < 4 || (units + kper - 1) / kper != s || (size_t)s * m * cols * 4u > room))
+          continue;
+        const double t = mx_cost(m, cols, k, kTiles[i][0], kTiles[i][1], s, cus);
+        if (t < b.t) b = {kTiles[i][0], kTiles[i][1], s, t};
+      }
+    return b;
+  };
+  const Pick all = best(n, false);
+  const int cut = wave_cut(m, n, 256, cus);
+  if (cut > 0 && cut < n) {  // whole waves on 256 x 256 tiles and the rest on smaller ones
+    const Pick rest = best(n - cut, true);
+    if (mx_cost(m, cut, k, 256, 256, 1, cus) + rest.t < all.t)
+      return {rest.bm, rest.bn, rest.splits, cut, room};
+  }
+  if (all.bm == 256) return {256, 256, 1, n, room};
+  return {all.bm, all.bn, all.splits, 0, room};
+}
+
+}  // namespace hkx

@@ -13,8 +13,8 @@ static hipError_t launch(const TileArgs& a, bool f32_shares, dim3 grid, hipStrea
 }
 
 hipError_t launch_tile4_mx(const TileArgs& a, int bm, int bn, bool f32_shares, dim3 grid, hipStream_t s) {
-  if (bm == 64 && bn == 128) return tile4_two(a, grid) ? launch<64, 128, 2>(a, f32_shares, grid, s) : launch<64, 128, 1>(a, f32_shares, grid, s);
-  if (bm == 128 && bn == 128) return tile4_two(a, grid) ? launch<128, 128, 2>(a, f32_shares, grid, s) : launch<128, 128, 1>(a, f32_shares, grid, s);
+  if (bm == 64 && bn == 128) return tile4_two(grid.x * grid.y, a.cus) ? launch<64, 128, 2>(a, f32_shares, grid, s) : launch<64, 128, 1>(a, f32_shares, grid, s);
+  if (bm == 128 && bn == 128) return tile4_two(grid.x * grid.y, a.cus) ? launch<128, 128, 2>(a, f32_shares, grid, s) : launch<128, 128, 1>(a, f32_shares, grid, s);
   if (bm == 128 && bn == 256) return launch<128, 256, 1>(a, f32_shares, grid, s);
   return hipErrorInvalidValue;
 }
