@@ -109,7 +109,7 @@ hipError_t launch_reduce(const ReduceArgs& a, const HkxEpilogue& ep, bool progra
     return hipGetLastError();                                                                \
   }
 
-// (two workgroups a CU where the tile's stages allow it and the grid has more than one a CU)
+// (two workgroups a CU where tile4_two says so)
 #define HKX_TILE4_LAUNCHER(BM, BN)                                                           \
   template <bool FP8, int RES>                                                               \
   static hipError_t launch_res(const TileArgs& a, int mode, dim3 grid, hipStream_t s) {      \
@@ -127,7 +127,7 @@ hipError_t launch_reduce(const ReduceArgs& a, const HkxEpilogue& ep, bool progra
   template <>                                                                                \
   hipError_t launch_tile4<BM, BN>(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s) { \
     if constexpr (BN == 128) {                                                               \
-      if (tile4_two(grid.x * grid.y, a.cus)) return fp8 ? launch_res<true, 2>(a, mode, grid, s) : launch_res<false, 2>(a, mode, grid, s); \
+      if (tile4_two(BM, fp8, grid.x * grid.y, a.kt_split, a.cus)) return fp8 ? launch_res<true, 2>(a, mode, grid, s) : launch_res<false, 2>(a, mode, grid, s); \
     }                                                                                        \
     return fp8 ? launch_res<true, 1>(a, mode, grid, s) : launch_res<false, 1>(a, mode, grid, s); \
   }

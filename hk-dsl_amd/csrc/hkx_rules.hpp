@@ -46,12 +46,24 @@ inline bool pair_streams(int m, int n, int k, int cus) {
   return k <= 4096 || blocks <= cus || blocks > 2 * cus || (m <= 16 && blocks > cus * 7 / 4);
 }
 
-// Whether a grid of the 4-wave kernel's 128-column tiles runs its two-a-CU form: past one
-// workgroup a CU, where the second hides what a lone wave a SIMD waits for and fills the last
-// wave's idle CUs (700 x 4096 x 4096 on 64 x 128 tiles 44.5 -> 39.4 us, 2048 x 4096 x 4096 on
-// 128 x 128 ones 79.4 -> 72.1, 333 x 4096 x 14336 split 4 ways 79.2 -> 74.6). Up to one a CU
-// the one-a-CU form's deeper stages stay.
-inline bool tile4_two(unsigned wgs, int cus) { return wgs > (unsigned)cus; }
+// Whether a grid of the 4-wave kernel's 128-column tiles (bm rows, `units` 128-byte K stages a
+// workgroup) runs its two-a-CU form: past one workgroup a CU, where the second hides what a lone
+// wave a SIMD waits for and fills the last wave's idle CUs (700 x 4096 x 4096 on 64 x 128 tiles
+// 44.5 -> 39.4 us, 2048 x 4096 x 4096 on 128 x 128 ones 79.4 -> 72.1). Up to one a CU the
+// one-a-CU form's deeper stages stay.
+//
+// 128 x 128 tiles, whose two-a-CU form has two LDS stages for four, gain 1.05 (long K) to 1.5
+// (short) while both forms take the same waves of workgroups; where an odd wave leaves the last
+// pair a CU to half of them, a long K loses instead. Measured, bf16 and fp8, one a CU against two:
+// 520 to 720 workgroups (three waves) 0.82-0.99 from 16 stages (bf16 past 640: from 32, 1.02-1.05
+// at 16), 1.03-1.19 up to 8; 1040 to 1280 (five) 0.93-0.98 from 48, 1.01-1.15 up to 32; seven
+// and more 1.01-1.6. 64 x 128 tiles (three stages) gain 1.01-1.5 throughout.
+inline bool tile4_two(int bm, bool fp8, unsigned wgs, int units, int cus) {
+  if (wgs <= (unsigned)cus) return false;
+  const int waves = (int)((wgs + cus - 1) / cus);
+  const int most = fp8 || 2 * wgs <= 5u * cus ? 12 : 16;
+  return bm == 64 || !((waves == 3 && units > most) || (waves == 5 && units >= 48));
+}
 
 // How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles of the
 // 4-wave kernel, K split over workgroups into fp32 shares a second launch sums; or, for the

@@ -12,9 +12,15 @@ static hipError_t launch(const TileArgs& a, bool f32_shares, dim3 grid, hipStrea
   return hipGetLastError();
 }
 
+template <int BM>
+static hipError_t launch_res(const TileArgs& a, bool f32_shares, dim3 grid, hipStream_t s) {
+  return tile4_two(BM, true, grid.x * grid.y, a.kt_split, a.cus) ? launch<BM, 128, 2>(a, f32_shares, grid, s)
+                                                                 : launch<BM, 128, 1>(a, f32_shares, grid, s);
+}
+
 hipError_t launch_tile4_mx(const TileArgs& a, int bm, int bn, bool f32_shares, dim3 grid, hipStream_t s) {
-  if (bm == 64 && bn == 128) return tile4_two(grid.x * grid.y, a.cus) ? launch<64, 128, 2>(a, f32_shares, grid, s) : launch<64, 128, 1>(a, f32_shares, grid, s);
-  if (bm == 128 && bn == 128) return tile4_two(grid.x * grid.y, a.cus) ? launch<128, 128, 2>(a, f32_shares, grid, s) : launch<128, 128, 1>(a, f32_shares, grid, s);
+  if (bm == 64 && bn == 128) return launch_res<64>(a, f32_shares, grid, s);
+  if (bm == 128 && bn == 128) return launch_res<128>(a, f32_shares, grid, s);
   if (bm == 128 && bn == 256) return launch<128, 256, 1>(a, f32_shares, grid, s);
   return hipErrorInvalidValue;
 }

@@ -16,7 +16,7 @@ SHIM = """
 extern "C" {
 int skinny(int m, int n, int k) { return hkx::skinny_wins(m, n, k); }
 int streams(int m, int n, int k, int cus) { return hkx::pair_streams(m, n, k, cus); }
-int two(unsigned wgs, int cus) { return hkx::tile4_two(wgs, cus); }
+int two(int bm, int fp8, unsigned wgs, int units, int cus) { return hkx::tile4_two(bm, fp8, wgs, units, cus); }
 long long mx(int m, int n, int k, int cus, int* out) {
   const hkx::MxPlan p = hkx::mx_plan(m, n, k, cus);
   out[0] = p.bm; out[1] = p.bn; out[2] = p.splits; out[3] = p.cut;
@@ -48,3 +48,7 @@ def mx_plan(m, n, k, cus=CUS):
 
 def pair_streams(m, n, k, cus=CUS):
     return bool(lib().streams(m, n, k, cus))
+
+
+def tile4_two(bm, fp8, wgs, units, cus=CUS):
+    return bool(lib().two(bm, fp8, wgs, units, cus))

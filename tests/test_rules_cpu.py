@@ -17,3 +17,18 @@ def test_the_rules_are_the_librarys():
         for n in (64, 8192, 8196, 24576):
             for k in (128, 1792, 2048, 2176):
                 assert bool(rules.lib().skinny(m, n, k)) == gemm_cdna.decode8(m, n, k)
+
+
+def test_two_workgroups_a_cu_where_they_were_measured_faster():
+    """128 x 128 tiles of a long K stay one a CU where the second would run an odd last wave:
+    640 workgroups of 96 stages 165 us against 198, 520 of 96 151 against 167, 1280 of 64 0.92x;
+    the same grids with few stages, even waves and 64 x 128 tiles take two."""
+    for fp8 in (False, True):
+        for wgs, units in ((513, 16), (520, 32), (640, 32), (640, 96), (768, 64), (1100, 64), (1280, 48)):
+            assert not rules.tile4_two(128, fp8, wgs, units) and rules.tile4_two(64, fp8, wgs, units)
+        for wgs, units in ((257, 112), (300, 8), (512, 96), (520, 8), (700, 4), (1024, 96), (1100, 32), (1300, 64),
+                           (1700, 96), (2048, 64)):
+            assert rules.tile4_two(128, fp8, wgs, units)
+        assert rules.tile4_two(128, fp8, 720, 16) == (not fp8)
+        for bm in (64, 128):
+            assert not rules.tile4_two(bm, fp8, 256, 4) and rules.tile4_two(bm, fp8, 257, 4)
