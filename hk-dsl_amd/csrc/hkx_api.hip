@@ -888,7 +888,7 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
     t.tiles_m = (m + 255) / 256;
     t.tiles_n = (q.cut + 255) / 256;
     const dim3 g(std::min(t.tiles_m * t.tiles_n, cu_count()));
-    int rc = launched(hkx::launch_quad_mx(t, g, s), "mx GEMM");
+    int rc = launched(hkx::launch_quad_mx(t, false, g, s), "mx GEMM");
     if (rc || q.cut >= n) return rc;
     // the rest of N as a call of its own: W's rows and their scales, C's columns
     t.b = (const uint8_t*)b + (int64_t)q.cut * ldb;
@@ -909,7 +909,9 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   tw.split_stride = (int64_t)m * t.N;
   tw.c_dt = HKX_FP32;
   tw.kt_split = (k / 128 + q.splits - 1) / q.splits;
-  int rc = launched(hkx::launch_tile4_mx(tw, q.bm, q.bn, true, g, s), "mx GEMM (split over K)");
+  int rc = launched(q.bm == 256 ? hkx::launch_quad_mx(tw, true, g, s)
+                                : hkx::launch_tile4_mx(tw, q.bm, q.bn, true, g, s),
+                    "mx GEMM (split over K)");
   if (rc) return rc;
   hkx::ReduceArgs r{};
   r.ws = (const float*)ws;

@@ -53,8 +53,9 @@ hipError_t launch_quad(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStre
 // Its fp8 forms with e5m2 operands (a.ab_fmt 2-4, the dequant forms) and with an fp32 C
 // (kEpDeqAcc), by compiled form.
 hipError_t launch_quad_fmt(const TileArgs& a, int epf, dim3 grid, hipStream_t s);
-// Its MX form (fp8 operands, E8M0 block scales in a.sa / a.sb, bf16 C, one pass).
-hipError_t launch_quad_mx(const TileArgs& a, dim3 grid, hipStream_t s);
+// Its MX form (fp8 operands, E8M0 block scales in a.sa / a.sb): bf16 C in one pass, or fp32
+// shares of a K split (f32_shares, a.c the workspace, grid.y the splits).
+hipError_t launch_quad_mx(const TileArgs& a, bool f32_shares, dim3 grid, hipStream_t s);
 // The 4-wave tile kernel's MX form: 64 x 128, 128 x 128 or 128 x 256 tiles, bf16 C or fp32
 // shares of a K split (f32_shares, a.c the workspace, grid.y the splits).
 hipError_t launch_tile4_mx(const TileArgs& a, int bm, int bn, bool f32_shares, dim3 grid, hipStream_t s);

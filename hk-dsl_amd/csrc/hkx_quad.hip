@@ -134,9 +134,13 @@ hipError_t launch_quad128(const TileArgs& a, int mode, dim3 grid, hipStream_t s)
   return hipGetLastError();
 }
 
-hipError_t launch_quad_mx(const TileArgs& a, dim3 grid, hipStream_t s) {
-  if (quad_form(a, true, kStore16) != kEpNone || a.ep.form != HKX_EP_NONE) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((quad_kernel<HKX_ACT_NONE, kEpNone, false, true, true>), grid, dim3(512), 0, s, a);
+hipError_t launch_quad_mx(const TileArgs& a, bool f32_shares, dim3 grid, hipStream_t s) {
+  if (quad_form(a, true, f32_shares ? kStoreF32 : kStore16) != kEpNone || a.ep.form != HKX_EP_NONE)
+    return hipErrorInvalidValue;
+  if (f32_shares)
+    hipLaunchKernelGGL((quad_kernel<HKX_ACT_NONE, kEpNone, false, true, true, 256, true>), grid, dim3(512), 0, s, a);
+  else
+    hipLaunchKernelGGL((quad_kernel<HKX_ACT_NONE, kEpNone, false, true, true>), grid, dim3(512), 0, s, a);
   return hipGetLastError();
 }
 

@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
   static_assert(BM == 256 || (BM == 128 && !FP8 && !MX), "128-row tiles: bf16 only");
   // SHARE: K split over blockIdx.y, each split's fp32 sums stored as they are (a later pass
   // adds the splits in order and applies the epilogue)
-  static_assert(!SHARE || (BM == 256 && !PAIR && !MX && EPF == kEpNone && ACT == HKX_ACT_NONE),
+  static_assert(!SHARE || (BM == 256 && !PAIR && EPF == kEpNone && ACT == HKX_ACT_NONE),
                 "fp32 shares: 256-row tiles, unpaired, no epilogue");
   constexpr int NI = BM / 128;          // A halves of a tile
   constexpr int QPS = NI + 2;           // quarters a K-tile slot: the A halves, B0, B1
@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
       const uint32_t row = (uint32_t)((wave < 4 ? st.m0 : st.n0) + 64 * (wave & 3) + lane);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rsc, (__attribute__((address_space(3))) void*)(smem + SCO + (chunk % 3) * 8192 + wave * 1024), 16,
-          row * (wave < 4 ? p.sa_ld : p.sb_ld), __builtin_amdgcn_readfirstlane((uint32_t)st.t * 4u), 0, 0);
+          row * (wave < 4 ? p.sa_ld : p.sb_ld), __builtin_amdgcn_readfirstlane((uint32_t)(kt0 + st.t) * 4u), 0, 0);
     }
   };
 
@@ -322,8 +322,8 @@ __global__ void __launch_bounds__(512, 1) quad_kernel(const TileArgs p) {
     tile_at(lt, m0, n0);
     const uint8_t* ev = smem + EPV + (lt % 3) * 3072;  // cs, rs, ra
     if constexpr (SHARE) {
-      // the split's fp32 sums, 16 bytes a lane (16 x 16 fragments; the split form is never
-      // MX): lane (rf, q) holds row rf, columns 4 q + [0, 4) of each fragment
+      // the split's fp32 sums, 16 bytes a lane (16 x 16 fragments): lane (rf, q) holds row rf,
+      // columns 4 q + [0, 4) of each fragment
 #pragma unroll
       for (int i = 0; i < 2; ++i)
 #pragma unroll

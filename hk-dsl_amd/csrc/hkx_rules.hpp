@@ -65,10 +65,10 @@ inline bool tile4_two(int bm, bool fp8, unsigned wgs, int units, int cus) {
   return bm == 64 || !((waves == 3 && units > most) || (waves == 5 && units >= 48));
 }
 
-// How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles of the
-// 4-wave kernel, K split over workgroups into fp32 shares a second launch sums; or, for the
-// first `cut` columns, on whole waves of 256 x 256 quadrant tiles, the rest of N on the tiles
-// (cut = n: all of it).
+// How the MX GEMM runs a shape: on the 8-bit decode kernel (bm = 0); on bm x bn tiles (the
+// quadrant kernel's 256 x 256 or the 4-wave kernel's smaller ones), K split over workgroups into
+// fp32 shares a second launch sums; or, for the first `cut` columns, on whole waves of 256 x 256
+// tiles, the rest of N on the smaller ones (cut = n: all of it).
 struct MxPlan {
   int bm, bn, splits, cut;
   size_t ws_bytes;  // the workspace a caller passes (mx_share_bytes)
@@ -116,27 +116,41 @@ inline MxPlan mx_plan(int32_t m, int32_t n, int32_t k, int cus) {
     int bm, bn, splits;
     double t;
   };
+  const int units = k / 128;
+  auto splits_ok = [&](int s, int cols, int least) {
+    return units / s >= least && (units + (units + s - 1) / s - 1) / ((units + s - 1) / s) == s &&
+           (size_t)s * m * cols * 4u <= room;
+  };
   auto best = [&](int cols, bool small_only) {
     static const int kTiles[4][3] = {{64, 128, 8}, {128, 128, 4}, {128, 256, 2}, {256, 256, 1}};
     Pick b{256, 256, 1, 1e30};
     for (int i = 0; i < (small_only ? 3 : 4); ++i)
       for (int s = 1; s <= kTiles[i][2]; s *= 2) {
-        const int units = k / 128, kper = (units + s - 1) / s;
-        if (s > 1 && (units / s < 4 || (units + kper - 1) / kper != s || (size_t)s * m * cols * 4u > room))
-          continue;
+        if (s > 1 && !splits_ok(s, cols, 4)) continue;
         const double t = mx_cost(m, cols, k, kTiles[i][0], kTiles[i][1], s, cus);
         if (t < b.t) b = {kTiles[i][0], kTiles[i][1], s, t};
       }
     return b;
   };
-  const Pick all = best(n, false);
+  Pick all = best(n, false);
+  // 256 x 256 tiles split over K, one a CU, where they lead: by 3%, or by 10% where the tiles are
+  // no multiple of the 8 XCDs, whose raster then keeps no share of the operands an XCD (up to
+  // 1.2 times the estimate: 1280 x 1792 x 16384). Cold weights, against the smaller tiles: 1087 x
+  // 4096 x 14336 in three splits 110.6 -> 87.0 us, 900 x 5120 x 12288 in three 96.2 -> 79.2, 2100
+  // x 2048 x 16384 in three 119.7 -> 94.1.
+  const int64_t big = (int64_t)((m + 255) / 256) * ((n + 255) / 256);
+  const double lead = big % 8 ? 0.90 : 0.97;
+  for (int s = 2; s <= 8 && big * s <= cus; ++s) {
+    const double t = splits_ok(s, n, 8) ? mx_cost(m, n, k, 256, 256, s, cus) : 1e30;
+    if (t < (all.bm == 256 && all.splits > 1 ? all.t : lead * all.t)) all = {256, 256, s, t};
+  }
   const int cut = wave_cut(m, n, 256, cus);
   if (cut > 0 && cut < n) {  // whole waves on 256 x 256 tiles and the rest on smaller ones
     const Pick rest = best(n - cut, true);
     if (mx_cost(m, cut, k, 256, 256, 1, cus) + rest.t < all.t)
       return {rest.bm, rest.bn, rest.splits, cut, room};
   }
-  if (all.bm == 256) return {256, 256, 1, n, room};
+  if (all.bm == 256 && all.splits == 1) return {256, 256, 1, n, room};
   return {all.bm, all.bn, all.splits, 0, room};
 }
 

@@ -52,3 +52,29 @@ def pair_streams(m, n, k, cus=CUS):
 
 def tile4_two(bm, fp8, wgs, units, cus=CUS):
     return bool(lib().two(bm, fp8, wgs, units, cus))
+
+
+def mx_form(m, n, k, cus=CUS):
+    """The plan of an MX GEMM in words: its tiles (those of the columns past the whole waves of
+    256 x 256 ones, "cut+"), K splits, and whether its 128-column tiles run two a CU."""
+    p = mx_plan(m, n, k, cus)
+    if p.bm == 0:
+        return "decode"
+    if p.cut == n:
+        return "256x256"
+    wgs = -(-m // p.bm) * -(-(n - p.cut) // p.bn) * p.splits
+    two = p.bn == 128 and tile4_two(p.bm, True, wgs, -(-(k // 128) // p.splits), cus)
+    return ("cut+" if p.cut else "") + f"{p.bm}x{p.bn}" + f" k{p.splits}" * (p.splits > 1) + " two" * two
+
+
+#: Shapes that run each plan of the MX GEMM.
+MX_FORMS = [
+    ("64x128", 33, 8, 128), ("64x128 two", 261, 11328, 128), ("64x128 k2", 33, 136, 2048),
+    ("64x128 k4", 70, 264, 4224), ("64x128 k8", 33, 520, 8192),
+    ("128x128", 5480, 264, 128), ("128x128 two", 6933, 1048, 640), ("128x128 k2", 65, 9176, 3840),
+    ("128x128 k4", 4214, 8, 4096), ("128x256", 6670, 520, 256), ("128x256 k2", 266, 8432, 12928),
+    ("256x256", 260, 13080, 128), ("256x256 k2", 265, 11248, 14720), ("256x256 k3", 406, 9016, 6528),
+    ("256x256 k5", 6074, 264, 8320), ("256x256 k8", 4243, 144, 15232),
+    ("cut+64x128", 1025, 14576, 256), ("cut+64x128 two", 2447, 7984, 768),
+    ("cut+128x128", 1057, 15192, 512), ("cut+128x128 two", 5511, 4104, 2944),
+    ("cut+128x256", 1601, 11824, 1024)]

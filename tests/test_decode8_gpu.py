@@ -2,7 +2,7 @@
 its edges: one to 32 tokens, one row block, ragged last blocks of W, K of one 128-byte step
 up to several rounds of the workgroup's waves with every kind of remainder.
 
-Bounds: against the 64-bit value the error is half a bf16 unit, 2^-9 |ref|, plus what the fp8
+Bounds: against the 64-bit value the error is half a bf16 unit, up to 2^-8 |ref|, plus what the fp8
 MFMA drops: it keeps a K-step's products to about 2^-16 of their largest (the tile kernels'
 fp32 output, rounded nowhere else, is off by up to 1.3e-5 of sum |a b| at K = 128). The check
 allows 2^-8 |ref| + 2^-15 sum |a b|, element by element."""

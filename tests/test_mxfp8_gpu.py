@@ -7,6 +7,7 @@ quantization bit for bit against the oracle's AITER per_1x32 rule
 import pytest
 import torch
 
+import rules
 from hk.ops import mxfp8
 from oracle import gemm_oracle as O
 
@@ -156,4 +157,25 @@ def test_mx_tiles_splits_and_wave_cuts(m, n, k):
     mxfp8.gemm(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV), out=out[:m, :n])
     ref = O.mx_gemm(a, b, sa, sb)
     assert O.rel_to_max(out[:m, :n].cpu(), ref) < 5e-3
+    assert (out[m] == 7.0).all() and (out[:, n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("form,m,n,k", rules.MX_FORMS)
+def test_mx_gemm_on_every_plan(form, m, n, k):
+    """Each plan of the MX GEMM against the 64-bit product: half a unit of bf16, up to 2^-8 |ref|,
+    and what the scaled MFMA drops of products far below a K-step's largest: 2^-14 of sum |a b|
+    (2^-14.87 at most, the same on every plan, over 10^8 outputs); nothing stored past M and N."""
+    print(f"case mx {form} {m}x{n}x{k}", flush=True)
+    a, b, sa, sb = (t.to(DEV) for t in _operands(m, n, k, seed=m + n + k))
+    out = torch.full((m + 1, n + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    mxfp8.gemm(a, b, sa, sb, out=out[:m, :n])
+    torch.cuda.synchronize()
+
+    def dequant(x, s):
+        return x.double() * torch.exp2(s.double() - 127).repeat_interleave(32, 1)
+
+    af, bf = dequant(a, sa), dequant(b, sb)
+    ref, got = af @ bf.t(), out[:m, :n].double()
+    big = af.abs() @ bf.abs().t()
+    assert ((got - ref).abs() <= 2.0 ** -8 * ref.abs() + 2.0 ** -14 * big).all()
     assert (out[m] == 7.0).all() and (out[:, n:] == 7.0).all()

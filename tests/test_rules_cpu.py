@@ -32,3 +32,17 @@ def test_two_workgroups_a_cu_where_they_were_measured_faster():
         assert rules.tile4_two(128, fp8, 720, 16) == (not fp8)
         for bm in (64, 128):
             assert not rules.tile4_two(bm, fp8, 256, 4) and rules.tile4_two(bm, fp8, 257, 4)
+
+
+def test_every_mx_plan_has_a_shape_that_runs_it():
+    """The shapes the GPU tests run each plan with still take it."""
+    assert [(rules.mx_form(m, n, k), m, n, k) for _, m, n, k in rules.MX_FORMS] == rules.MX_FORMS
+
+
+def test_mx_splits_256_tiles_over_a_long_k():
+    """Where few 256 x 256 tiles have a long K each, the split form measured fastest: 1087 x 4096 x
+    14336 in three 80 us (smaller tiles 110), 900 x 5120 x 12288, 2100 x 2048 x 16384."""
+    for m, n, k in ((1087, 4096, 14336), (600, 4096, 14336), (900, 5120, 12288), (2100, 2048, 16384)):
+        p = rules.mx_plan(m, n, k)
+        tiles = -(-m // 256) * -(-n // 256)
+        assert p.bm == 256 and p.splits > 1 and tiles * p.splits <= 256 and k // 128 // p.splits >= 8
