@@ -18,9 +18,22 @@ constexpr int kSkinnyM = 32;
 // 27.0 -> 20.4, 1024 x 8192 at M = 32 10.2 -> 9.5, 8192 x 512 at M = 32 5.6 -> 5.5. Where K is
 // short and the row blocks more than two a CU, the tiles' one launch wins (12288 x 1024: 6.7
 // against 7.2; 32768 x 512: 6.5 against 9.2; 12288 x 2048 at M = 32: 8.6 against 9.3, at M = 16
-// 8.5 against 8.0), so those stay there. hk.ops.gemm_cdna.decode8 is the same rule.
+// 8.5 against 8.0), so those stay there. So does a long K: past K = 4096 each 16-row block of W
+// streams all of X again, at M = 32 twice W's bytes, and the more blocks a CU takes and the
+// longer K, the sooner the tiles lead (2100 shapes, the kernel's rate over the tiles'; 4096
+// columns are a block a CU of 256): at M 17 to 32 to 4096 columns 1.21-2.1 up to K = 14336 and
+// 0.77-1.05 past it, to 8192 columns 1.04-1.27 up to K = 7168 and 0.74-1.01 past it, beyond
+// 0.64-1.04; at M 13 to 16 0.92-1.01 past K = 7168 at 4608 to 6144 columns and from 14336; at M
+// 9 to 16 0.85-1.0 past 24576 columns. M <= 8 keeps the kernel (0.93-1.9), and so does M <= 16
+// at multiples of 4096 up to 16384, whose row stride slows the tiles (0.96-1.4). Up to K = 4096
+// only M 17 to 32 past 24576 columns loses (0.79-0.91; at K = 4096 1.03-1.4).
+// hk.ops.gemm_cdna.decode8 is the same rule.
 inline bool skinny_wins(int m, int n, int k) {
-  return m <= kSkinnyM && (n <= 8192 || k > 2048 || (k >= 1792 && m <= 16));
+  if (m > kSkinnyM || !(n <= 8192 || k > 2048 || (k >= 1792 && m <= 16))) return false;
+  if (k <= 4096) return m <= 16 || n <= 24576 || k > 3840;
+  if (m > 16) return n <= 4096 ? k <= 14336 : n <= 8192 && k <= 7168;
+  if (m <= 8 || (k % 4096 == 0 && k <= 16384)) return true;
+  return n <= 24576 && (m <= 12 || k <= 7168 || n <= 4096 || (n > 6144 && n <= 12288));
 }
 
 // The columns of N whose 256 x 256 tiles fill whole waves of one-a-CU workgroups at M's

@@ -267,9 +267,18 @@ def decode8(m: int, n: int, k: int) -> bool:
     """Whether a scaled_mm of e4m3 operands runs on the 8-bit decode kernel
     (csrc/hkx_skinny.hpp, which the library picks for HKX_KERNEL_AUTO by the same rule) rather
     than on `route`'s tiles: up to 32 rows, except where K is short and the row blocks are
-    more than two a CU (csrc/hkx_api.hip's auto_skinny has both sides' times), unless a user
-    record names a candidate."""
+    more than two a CU, or where K is long and the rows or the blocks are many (skinny_wins in
+    csrc/hkx_rules.hpp has both sides' times), unless a user record names a candidate."""
     if m > DECODE8_M or not (n <= 8192 or k > 2048 or (k >= 1792 and m <= 16)):
+        return False
+    if k <= 4096:
+        wins = m <= 16 or n <= 24576 or k > 3840
+    elif m > 16:
+        wins = k <= 14336 if n <= 4096 else n <= 8192 and k <= 7168
+    else:
+        wins = m <= 8 or (k % 4096 == 0 and k <= 16384) or n <= 24576 and (
+            m <= 12 or k <= 7168 or n <= 4096 or 6144 < n <= 12288)
+    if not wins:
         return False
     return not any(key in OVERRIDE and fits(OVERRIDE[key], m, n, k, True)
                    for key in ((m, n, k), "*"))

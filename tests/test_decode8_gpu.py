@@ -19,7 +19,8 @@ DEV = "cuda:0"
 E4 = torch.float8_e4m3fn
 SHAPES = [(4, 128), (16, 256), (20, 1152), (1004, 1280), (260, 2048), (64, 2176), (132, 4096),
           (24, 4224), (48, 5120), (36, 14336),
-          (8192 + 20, 1152), (16384, 4096), (24576 + 4, 2176)]  # several blocks a workgroup
+          (8192 + 20, 1152), (16384, 4096), (24576 + 4, 2176),  # several blocks a workgroup,
+          (16384 + 20, 4224)]                                   # X streamed with each
 
 
 def _fp8(rows, k, g):

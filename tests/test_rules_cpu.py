@@ -19,6 +19,23 @@ def test_the_rules_are_the_librarys():
                 assert bool(rules.lib().skinny(m, n, k)) == gemm_cdna.decode8(m, n, k)
 
 
+def test_the_tiles_keep_the_decode_sizes_they_are_faster_at():
+    """Many rows or row blocks over a long K: the 8-bit decode kernel streams X once a block there
+    and lost to the split tiles (32 x 5312 x 14336 28.7 us against 21.9, 32 x 14336 x 11648 49.9
+    against 36.5, 18 x 6144 x 13312 26.2 against 22.4, 15 x 5312 x 13312 21.5 against 20.2)."""
+    for m, n, k in ((32, 5312, 14336), (32, 14336, 11648), (18, 6144, 13312), (15, 5312, 13312),
+                    (17, 8192, 8320), (20, 10240, 4608), (32, 28672, 3072), (12, 28672, 5120), (24, 2048, 16384),
+                    (16, 4608, 20480)):
+        assert not gemm_cdna.decode8(m, n, k)
+    for m, n, k in ((32, 4096, 14336), (32, 8192, 7168), (16, 12288, 14336), (8, 28672, 14336), (16, 20480, 12288),
+                    (32, 28672, 4096), (32, 24576, 3072), (12, 5312, 13312)):
+        assert gemm_cdna.decode8(m, n, k)
+    for m in range(1, 34):  # both sides' rule, on either side of its lines
+        for n in (4096, 4100, 6144, 6148, 8192, 8196, 12288, 12292, 24576, 24580):
+            for k in (1664, 1792, 2048, 2176, 3840, 3968, 4096, 4224, 7168, 7296, 8192, 14336, 14464, 16384, 20480):
+                assert bool(rules.lib().skinny(m, n, k)) == gemm_cdna.decode8(m, n, k), (m, n, k)
+
+
 def test_two_workgroups_a_cu_where_they_were_measured_faster():
     """128 x 128 tiles of a long K stay one a CU where the second would run an odd last wave:
     640 workgroups of 96 stages 165 us against 198, 520 of 96 151 against 167, 1280 of 64 0.92x;
