@@ -46,17 +46,25 @@ inline int wave_cut(int m, int n, int outw, int cus) {
   return (n / outw / per) * per * outw;
 }
 
-// Whether a paired decode call the stream kernel can take also runs on it. Up to K = 4096
-// (X held in registers) it always does: 1.06-2.4x the blocked kernel at 1536 to 28672 rows of
-// W, M = 1 to 32. Past that X is streamed with every 16-row block, and where those blocks are
-// more than the CUs but at most two a CU, the blocked kernel's 32-row workgroups are one wave
-// and read X half as often: it stays there above M = 16 (8192 x 6144 at M = 24: 24.6 against
-// 27.6 us) or where the last blocks leave CUs idle (6144 x 5120 at M = 8: 16.5 against 17.4);
-// on either side the stream kernel wins (4096 x 8192 at M = 16: 24.3 -> 16.1 us, 12288 x 5120
-// at M = 16: 34.5 -> 26.6, 28672 x 8192 at M = 1: 95.3 -> 78.5).
+// Whether a paired decode call the stream kernel can take also runs on it: where its 16-row
+// blocks (8 columns of C) go up to one a CU always, 1.04-2.7x the blocked kernel (4096 x 8192 at
+// M = 16 24.3 -> 16.1 us, 28672 x 8192 at M = 1 95.3 -> 78.5). Past one a CU the blocked kernel's
+// 32-row workgroups are half as many waves, where the blocks' waves are even full ones. Measured at
+// 2000 shapes, K 1024 to 12288, the stream kernel's rate over the blocked one's:
+// * past one to two blocks a CU (one wave of workgroups): K = 1024 0.82-0.98; K = 2048 0.81-1.02
+//   from M = 9, up to M = 8 0.94-1.1 (1.0-1.1 past 3/2 a CU); K = 3072 0.91-1.02 up to M = 8 and at
+//   M 17 to 24, 1.0-1.12 at the others; K = 4096 0.99-1.47; past it X is streamed with every block,
+//   and only the last eighth of the range gains, 0.97-1.21 up to M = 8, 1.02-1.09 to M = 16 from
+//   K = 8192;
+// * past three to four and five to six: past K = 4096 0.87-1.0 at M 17 to 28 (four) or 26 (six), less
+//   so the more waves; 0.96-1.3 up to M = 16 and 1.0-1.2 past those;
+// * the others 1.0-1.7.
 inline bool pair_streams(int m, int n, int k, int cus) {
-  const int blocks = (n + 7) / 8;
-  return k <= 4096 || blocks <= cus || blocks > 2 * cus || (m <= 16 && blocks > cus * 7 / 4);
+  const int blocks = (n + 7) / 8, waves = (blocks + cus - 1) / cus;
+  if (waves != 2) return k <= 4096 || m <= 16 || waves % 2 || m > 32 - waves;
+  if (k < 3072) return k >= 2048 && m <= 8 && 2 * blocks > 3 * cus;
+  if (k < 4096) return m > 24 || (m > 8 && m <= 16);
+  return k == 4096 || (m <= 16 && 4 * blocks > 7 * cus && (m <= 8 || k >= 8192));
 }
 
 // Whether a grid of the 4-wave kernel's 128-column tiles (bm rows, `units` 128-byte K stages a

@@ -40,8 +40,11 @@ def test_whole_rows_and_stream_at_k_4096(m, i):
 
 @pytest.mark.parametrize("m,i,k", [(1, 8, 1024), (9, 2052, 1024), (3, 2060, 2048), (17, 20, 2048),
                                    (32, 2056, 4096), (1, 12, 5120), (16, 4104, 6144), (32, 36, 8192),
-                                   (24, 3072, 5120)])
+                                   (24, 3072, 5120), (9, 4100, 1024), (3, 3076, 2048), (17, 4100, 2048),
+                                   (9, 2060, 3072), (24, 4100, 5120), (20, 6148, 5120)])
 def test_stream_at_other_k(m, i, k):
+    """The stream form, and the blocked kernel where the rule leaves it the call: up to two blocks
+    a CU at a short K, three to four at M = 20."""
     _check(m, i, k)
 
 

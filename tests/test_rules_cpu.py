@@ -36,6 +36,21 @@ def test_the_tiles_keep_the_decode_sizes_they_are_faster_at():
                 assert bool(rules.lib().skinny(m, n, k)) == gemm_cdna.decode8(m, n, k), (m, n, k)
 
 
+def test_the_blocked_kernel_keeps_the_paired_decode_it_is_faster_at():
+    """Where its 32-row workgroups fill whole waves and the stream kernel's blocks twice as many:
+    at a short K past one block a CU (10 x 6576 x 1024 6.7 us against 5.4, 18 x 7536 x 2048 11.0
+    against 9.3), at a long one with many rows (17 x 21504 x 7168 79.6 against 70.7, 19 x 12496 x
+    5120 42.1 against 37.0)."""
+    for m, n2, k in ((10, 6576, 1024), (1, 8192, 1024), (18, 7536, 2048), (32, 4160, 2048), (4, 5760, 2048),
+                     (1, 5152, 3072), (20, 6000, 3072), (17, 21504, 7168), (19, 12496, 5120), (13, 8080, 5120),
+                     (24, 14496, 6144), (28, 16384, 8192), (26, 20800, 5120)):
+        assert not rules.pair_streams(m, n2 // 2, k), (m, n2, k)
+    for m, n2, k in ((10, 4096, 1024), (10, 8208, 1024), (32, 4096, 2048), (4, 7000, 2048), (12, 5152, 3072),
+                     (32, 6000, 3072), (16, 8192, 4096), (4, 8192, 5120), (16, 8192, 8192), (16, 14496, 6144),
+                     (17, 10000, 5120), (29, 16384, 8192), (27, 20800, 5120), (16, 24576, 4096), (32, 24576, 4096)):
+        assert rules.pair_streams(m, n2 // 2, k), (m, n2, k)
+
+
 def test_two_workgroups_a_cu_where_they_were_measured_faster():
     """128 x 128 tiles of a long K stay one a CU where the second would run an odd last wave:
     640 workgroups of 96 stages 165 us against 198, 520 of 96 151 against 167, 1280 of 64 0.92x;
