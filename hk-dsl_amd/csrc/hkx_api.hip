@@ -857,7 +857,7 @@ int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const ui
   t.sa_bytes = (uint32_t)((long long)m * sa_ld);
   t.sb_bytes = (uint32_t)((long long)n * sb_ld);
   const hipStream_t s = (hipStream_t)stream;
-  if (!q.bm) {  // the 8-bit decode kernel takes every call of M <= 32
+  if (!q.bm) {  // the 8-bit decode kernel
     hkx::SkinnyArgs d{};
     d.a = a;
     d.b = b;

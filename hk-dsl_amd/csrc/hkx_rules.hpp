@@ -95,6 +95,18 @@ struct MxPlan {
   size_t ws_bytes;  // the workspace a caller passes (mx_share_bytes)
 };
 
+// Whether the 8-bit decode kernel runs an MX call of M <= 32: always up to M = 16 (1.0-5.6x the 256
+// x 256 tiles); at M 17 to 32 where K is short enough that X, streamed again with every 16-row block
+// of W past K = 4096, does not cost more than the tiles' padding. Its rate over the tiles', weights
+// from memory, M = 17 and 32: 4096 columns (a block a CU) and less 1.11-2.5 and 0.94-2.4 up to K =
+// 8192, 0.96-1.13 and 0.78-0.94 past it; more columns 1.0-1.8 and 0.9-1.7 up to K = 4096, 0.76-1.14
+// and 0.63-0.95 past it (32 x 12800 x 6144 56 us against 39) and under K = 1024 past 8192 columns.
+inline bool mx_skinny(int m, int n, int k) {
+  if (m <= 16) return true;
+  if (m > kSkinnyM) return false;
+  return n <= 4096 ? k <= 8192 : n <= 16384 && k <= 4096 && (k >= 1024 || n <= 8192);
+}
+
 // A plan's estimated time in us: waves of one-a-CU workgroups, each a fixed part and a time a
 // 128-K unit by tile shape, or W's bytes at the rate these tiles stream them; a split adds its
 // sum's launch and the shares' round trip. Fitted to a sweep of every tile and split at 165
@@ -118,7 +130,6 @@ inline double mx_cost(int m, int n, int k, int bm, int bn, int splits, int cus) 
 // of all of C where 256 x 256 tiles fill less than half the CUs, none otherwise (or where a
 // share would span 4 GiB). The plan below stays within it.
 inline size_t mx_share_bytes(int32_t m, int32_t n, int32_t k, int cus) {
-  if (m <= kSkinnyM) return 0;
   const int tiles = ((m + 255) / 256) * ((n + 255) / 256);
   if (2 * tiles > cus || (long long)((m + 255) / 256) * 256 * n * 4 >= (1LL << 32)) return 0;
   const int s = std::min(std::min(cus / tiles, (k / 128) / 8), 8);
@@ -129,7 +140,7 @@ inline size_t mx_share_bytes(int32_t m, int32_t n, int32_t k, int cus) {
 
 inline MxPlan mx_plan(int32_t m, int32_t n, int32_t k, int cus) {
   if (m < 1 || n < 1 || k < 128 || k % 128) return {256, 256, 1, n, 0};
-  if (m <= kSkinnyM) return {0, 0, 1, 0, 0};
+  if (mx_skinny(m, n, k)) return {0, 0, 1, 0, 0};
   // the best tile and split of some columns: splits of 4 K units or more, no empty one, their
   // shares within the workspace
   const size_t room = mx_share_bytes(m, n, k, cus);

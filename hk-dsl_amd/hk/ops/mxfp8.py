@@ -3,15 +3,15 @@
 The reference's contract (python/hk/ops/mxfp8.py:1-110): A (M, K) and B (N, K) fp8 e4m3,
 K-contiguous (F.linear's layout); sa (M, K/32) and sb (N, K/32) their E8M0 scales, one byte
 a row and 32 columns (the OCP MX layout; a 32 x 32-block weight scale is its rows repeated,
-`expand_block_scales`). Up to 32 rows the product runs on the 8-bit decode kernel, above that
-on the 256 x 256 quadrant kernel's MX form, on the 4-wave kernel's 64 x 128 to 128 x 256 tiles,
-or on both (whole waves of the large tiles, the rest of N on smaller ones), as the library's
-cost of each plan says (csrc/hkx_api.hip, mx_plan). Every MFMA is gfx950's scaled one, each lane
-passing the E8M0 byte of its own fragment row and 32-K block; the tiles' scales reach LDS by the
-same DMA as the operands, 16 bytes a row every 4 K units of 128 (whole lines: a 4-byte load a
-row and half a unit doubled the L2 requests and cost 60%). K a multiple of 128, N of 8, any M.
-Where few tiles would fill the CUs, K is split over workgroups into fp32 shares (a cached
-workspace, `_native.workspace`) that a second pass sums in split order.
+`expand_block_scales`). Up to 16 rows, and up to 32 at a short K, the product runs on the 8-bit
+decode kernel, elsewhere on the 256 x 256 quadrant kernel's MX form, on the 4-wave kernel's 64 x
+128 to 128 x 256 tiles, or on both (whole waves of the large tiles, the rest of N on smaller
+ones), as the library's cost of each plan says (csrc/hkx_rules.hpp, mx_plan). Every MFMA is
+gfx950's scaled one, each lane passing the E8M0 byte of its own fragment row and 32-K block; the
+tiles' scales reach LDS by the same DMA as the operands, 16 bytes a row every 4 K units of 128
+(whole lines: a 4-byte load a row and half a unit doubled the L2 requests and cost 60%). K a
+multiple of 128, N of 8, any M. Where few tiles would fill the CUs, K is split over workgroups
+into fp32 shares (a cached workspace, `_native.workspace`) that a second pass sums in split order.
 
 `quant(x)` is the activation side (python/hk/ops/mxfp8.py:605-660): bf16 x to fp8 e4m3 and
 E8M0 scales by AITER's per_1x32 rule (python/hk/mx.py:17-31), in one launch, the scales in

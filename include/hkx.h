@@ -295,8 +295,9 @@ int hkx_scaled_mm(const void* a, int64_t lda, const void* b, int64_t ldb,
  * (N, K/32) E8M0 bytes (scale 2^(s - 127) for its row and 32 K), row strides lda, ldb,
  * ldc in elements and sa_ld, sb_ld in bytes. K a multiple of 128, N of 8; sa and sb
  * 4-byte aligned with sa_ld, sb_ld multiples of 4 and >= K/32; C's rows 16-byte aligned.
- * M any. Up to M = 32 the 8-bit decode kernel runs it in one pass; above that the plan of
- * tiles, K splits and columns of least estimated time. A split's fp32 shares go through ws
+ * M any. Up to M = 16, and up to 32 at a short K, the 8-bit decode kernel runs it in one
+ * pass; elsewhere the plan of tiles, K splits and columns of least estimated time. A split's
+ * fp32 shares go through ws
  * (hkx_mx_gemm_workspace() bytes where 256 x 256 tiles fill less than half the CUs and K is 2048
  * or more; HKX_ERR_WORKSPACE if smaller), summed in split order by a second pass. */
 int hkx_mx_gemm(const void* a, int64_t lda, const void* b, int64_t ldb, const uint8_t* sa,

@@ -77,4 +77,7 @@ MX_FORMS = [
     ("256x256 k5", 6074, 264, 8320), ("256x256 k8", 4243, 144, 15232),
     ("cut+64x128", 1025, 14576, 256), ("cut+64x128 two", 2447, 7984, 768),
     ("cut+128x128", 1057, 15192, 512), ("cut+128x128 two", 5511, 4104, 2944),
-    ("cut+128x256", 1601, 11824, 1024)]
+    ("cut+128x256", 1601, 11824, 1024),
+    # M <= 32 on the tiles
+    ("64x128", 20, 8200, 512), ("64x128 k2", 24, 12808, 6144), ("64x128 k4", 32, 4104, 4224),
+    ("64x128 k8", 17, 520, 8320)]

@@ -71,6 +71,15 @@ def test_every_mx_plan_has_a_shape_that_runs_it():
     assert [(rules.mx_form(m, n, k), m, n, k) for _, m, n, k in rules.MX_FORMS] == rules.MX_FORMS
 
 
+def test_mx_decode_sizes_on_the_tiles():
+    """M 17 to 32 over a long K and many columns, where the decode kernel lost: 32 x 12800 x 6144 56 us
+    against 39, 24 x 5312 x 14336 against 256 x 256 tiles 0.92x."""
+    for m, n, k in ((32, 12800, 6144), (17, 8192, 4224), (24, 5312, 14336), (32, 2304, 8320), (20, 12800, 512)):
+        assert rules.mx_form(m, n, k).startswith("64x128"), (m, n, k)
+    for m, n, k in ((16, 12800, 14336), (17, 4096, 8192), (32, 5120, 4096), (32, 8192, 128), (1, 16384, 512)):
+        assert rules.mx_form(m, n, k) == "decode", (m, n, k)
+
+
 def test_mx_splits_256_tiles_over_a_long_k():
     """Where few 256 x 256 tiles have a long K each, the split form measured fastest: 1087 x 4096 x
     14336 in three 80 us (smaller tiles 110), 900 x 5120 x 12288, 2100 x 2048 x 16384."""
