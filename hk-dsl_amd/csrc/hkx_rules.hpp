@@ -110,10 +110,12 @@ inline bool mx_skinny(int m, int n, int k) {
 // A plan's estimated time in us: waves of one-a-CU workgroups, each a fixed part and a time a
 // 128-K unit by tile shape, or W's bytes at the rate these tiles stream them; a split adds its
 // sum's launch and the shares' round trip. Fitted to a sweep of every tile and split at 165
-// shapes (M 33-6000, N 768-16384, K 512-14336, one box): its pick is 0.3% slower than the best
-// on average, 1.13x at worst (M = 1000, 1024 x 8192). Before, every call ran on 256 x 256
-// tiles: 5120 x 4096 at M = 256 30.7 -> 14.9 us, 4096 x 1280 at M = 512 22.4 -> 8.7, 12800 x
-// 6144 at M = 256 51.1 -> 40.4, 1024 x 8192 at M = 64 21.3 -> 10.0.
+// shapes (M 33-6000, N 768-16384, K 512-14336, one box, part of W cached), 128 x 128 tiles one a CU
+// then. With weights from memory the calls take 1.04-1.09 times it on 64 x 128 and 128 x 128 tiles
+// and their splits, 1.15-1.18 on 128 x 256 and on 256 x 256 ones, 0.96-1.03 on split 256 x 256 ones
+// (497 shapes, each within 0.86-1.32; two a CU 0.86 of it at best): mx_plan's margins. Before, every
+// call ran on 256 x 256 tiles: 5120 x 4096 at M = 256 30.7 -> 14.9 us, 4096 x 1280 at M = 512 22.4 ->
+// 8.7, 12800 x 6144 at M = 256 51.1 -> 40.4, 1024 x 8192 at M = 64 21.3 -> 10.0.
 inline double mx_cost(int m, int n, int k, int bm, int bn, int splits, int cus) {
   const double fixed = bm == 256 ? 6.3 : bm == 64 ? 4.3 : bn == 128 ? 5.9 : 7.5;
   const double unit = bm == 256 ? 1.53 : bm == 64 ? 0.47 : bn == 128 ? 0.56 : 0.90;
@@ -165,13 +167,21 @@ inline MxPlan mx_plan(int32_t m, int32_t n, int32_t k, int cus) {
     return b;
   };
   Pick all = best(n, false);
+  auto wide = [&]() { return all.bm == 128 && all.bn == 256; };
+  // 128 x 256 tiles, and whole waves with a rest (below), in place of 256 x 256 tiles where they lead
+  // by 5%: 4860 x 4944 x 2688 82.3 us for 78.5 by an estimate 4% less, 5435 x 3728 x 1280 44.9 for
+  // 41.1 by 3%
+  const double t256 = mx_cost(m, n, k, 256, 256, 1, cus);
+  if (wide() && all.splits == 1 && all.t > 0.95 * t256) all = {256, 256, 1, t256};
   // 256 x 256 tiles split over K, one a CU, where they lead: by 3%, or by 10% where the tiles are
   // no multiple of the 8 XCDs, whose raster then keeps no share of the operands an XCD (up to
   // 1.2 times the estimate: 1280 x 1792 x 16384). Cold weights, against the smaller tiles: 1087 x
   // 4096 x 14336 in three splits 110.6 -> 87.0 us, 900 x 5120 x 12288 in three 96.2 -> 79.2, 2100
-  // x 2048 x 16384 in three 119.7 -> 94.1.
+  // x 2048 x 16384 in three 119.7 -> 94.1. Against 128 x 256 tiles, whose calls take 1.15 times
+  // the estimate, already where they are less than 5% behind: 858 x 4688 x 6272 57.7 -> 53.7, 2131
+  // x 2272 x 7552 65.4 -> 61.2, 1158 x 4224 x 8320 74.2 -> 71.3.
   const int64_t big = (int64_t)((m + 255) / 256) * ((n + 255) / 256);
-  const double lead = big % 8 ? 0.90 : 0.97;
+  const double lead = wide() && all.splits == 1 ? 1.05 : big % 8 ? 0.90 : 0.97;
   for (int s = 2; s <= 8 && big * s <= cus; ++s) {
     const double t = splits_ok(s, n, 8) ? mx_cost(m, n, k, 256, 256, s, cus) : 1e30;
     if (t < (all.bm == 256 && all.splits > 1 ? all.t : lead * all.t)) all = {256, 256, s, t};
@@ -179,7 +189,7 @@ inline MxPlan mx_plan(int32_t m, int32_t n, int32_t k, int cus) {
   const int cut = wave_cut(m, n, 256, cus);
   if (cut > 0 && cut < n) {  // whole waves on 256 x 256 tiles and the rest on smaller ones
     const Pick rest = best(n - cut, true);
-    if (mx_cost(m, cut, k, 256, 256, 1, cus) + rest.t < all.t)
+    if (mx_cost(m, cut, k, 256, 256, 1, cus) + rest.t < std::min(all.t, 0.95 * t256))
       return {rest.bm, rest.bn, rest.splits, cut, room};
   }
   if (all.bm == 256 && all.splits == 1) return {256, 256, 1, n, room};

@@ -72,12 +72,12 @@ MX_FORMS = [
     ("64x128", 33, 8, 128), ("64x128 two", 261, 11328, 128), ("64x128 k2", 33, 136, 2048),
     ("64x128 k4", 70, 264, 4224), ("64x128 k8", 33, 520, 8192),
     ("128x128", 5480, 264, 128), ("128x128 two", 6933, 1048, 640), ("128x128 k2", 65, 9176, 3840),
-    ("128x128 k4", 4214, 8, 4096), ("128x256", 6670, 520, 256), ("128x256 k2", 266, 8432, 12928),
+    ("128x128 k4", 4214, 8, 4096), ("128x256", 2533, 1560, 384), ("128x256 k2", 266, 8432, 12928),
     ("256x256", 260, 13080, 128), ("256x256 k2", 265, 11248, 14720), ("256x256 k3", 406, 9016, 6528),
     ("256x256 k5", 6074, 264, 8320), ("256x256 k8", 4243, 144, 15232),
-    ("cut+64x128", 1025, 14576, 256), ("cut+64x128 two", 2447, 7984, 768),
-    ("cut+128x128", 1057, 15192, 512), ("cut+128x128 two", 5511, 4104, 2944),
-    ("cut+128x256", 1601, 11824, 1024),
+    ("cut+64x128", 903, 16496, 384), ("cut+64x128 two", 5413, 3472, 1280),
+    ("cut+128x128", 6436, 2568, 640), ("cut+128x128 two", 6543, 3336, 3200),
+    ("cut+128x256", 6541, 2824, 1536),
     # M <= 32 on the tiles
     ("64x128", 20, 8200, 512), ("64x128 k2", 24, 12808, 6144), ("64x128 k4", 32, 4104, 4224),
     ("64x128 k8", 17, 520, 8320)]

@@ -80,6 +80,18 @@ def test_mx_decode_sizes_on_the_tiles():
         assert rules.mx_form(m, n, k) == "decode", (m, n, k)
 
 
+def test_mx_keeps_256_tiles_where_smaller_ones_were_no_faster():
+    """An estimate a few percent lower was slower: 4860 x 4944 x 2688 82.3 us on 128 x 256 tiles, 78.5
+    on 256 x 256 ones; 5435 x 3728 x 1280 44.9 for 41.1 with whole waves and a rest; 858 x 4688 x 6272
+    57.7 for 53.7 split over K."""
+    for m, n, k in ((4860, 4944, 2688), (5435, 3728, 1280), (2278, 16384, 1280), (5087, 10088, 1024)):
+        assert rules.mx_form(m, n, k) == "256x256", (m, n, k)
+    for m, n, k in ((858, 4688, 6272), (2131, 2272, 7552), (1158, 4224, 8320)):
+        assert rules.mx_form(m, n, k) == "256x256 k3", (m, n, k)
+    for m, n, k in ((2876, 12800, 6144), (4096, 5120, 4096)):
+        assert rules.mx_form(m, n, k).startswith("cut+"), (m, n, k)
+
+
 def test_mx_splits_256_tiles_over_a_long_k():
     """Where few 256 x 256 tiles have a long K each, the split form measured fastest: 1087 x 4096 x
     14336 in three 80 us (smaller tiles 110), 900 x 5120 x 12288, 2100 x 2048 x 16384."""
