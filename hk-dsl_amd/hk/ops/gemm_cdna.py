@@ -201,7 +201,24 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
 
 
 def _less(name: str, than: str, m: int, n: int, k: int, fp8: bool = False) -> bool:
-    return _cost(name, m, n, k, fp8) <= 0.93 * _cost(than, m, n, k, fp8)
+    """Whether `name`'s cost is 7% or more under `than`'s; 64 x 128 tiles in place of 128 x 128 ones
+    need more in two places. Where their count is no multiple of the 8 XCDs the workgroups are dealt
+    to them in turn, and with 3, 5, 6 or 7 tile rows each XCD then reads all of A and W: with W from
+    memory they were slower from 0.70 of the other's cost up (440 x 2272 x 2880 split in two, 0.76,
+    24.1 us for 21.1; 151 x 2536 x 4224 in four, 0.75, 17.8 for 16.5; paired 410 x 3824 x 1792, 0.70, 18.3
+    for 15.8) and 1.14 to 1.8 times faster to 0.67, at other counts 1.05 to 1.5 times faster at the
+    same costs. And unsplit against 128 x 128 tiles split in two they were slower from 0.82 (fp8 2618 x
+    744 x 14208 45.4 us for 39.3; at other counts from 0.795, 254 x 7744 x 3072 paired 30.1 for 28.7) and
+    1.07 to 1.18 times faster below."""
+    lead = 0.93
+    if than.startswith("t128x128") and name.startswith("t64x128"):
+        rows = math.ceil(m / 64)
+        whole = rows * math.ceil(n / 128) % 8 == 0
+        if not whole and rows in (3, 5, 6, 7):
+            lead = 0.68
+        elif than == "t128x128k2" and name == "t64x128":
+            lead = 0.81 if whole else 0.79
+    return _cost(name, m, n, k, fp8) <= lead * _cost(than, m, n, k, fp8)
 
 
 def _steps(m: int, n: int, k: int, fp8: bool = False) -> str:

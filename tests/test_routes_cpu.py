@@ -244,6 +244,21 @@ def test_rule_keeps_the_cus_full_on_uncached_weights():
     assert {s: gemm_cdna.rule(*s) for s in best} == best
 
 
+def test_rule_keeps_128_row_tiles_where_64_row_ones_were_slower():
+    """W from memory: 440 x 2272 x 2880 on 128 x 128 tiles split in two 21.1 us, on 64 x 128 ones 24.1;
+    151 x 2536 x 4224 split in four 16.5 against 17.8; 410 x 3824 x 1792 unsplit 15.8 against 18.3; fp8
+    2618 x 744 x 14208 39.3 against 45.4."""
+    keep = {(440, 2272, 2880): "t128x128k2", (290, 3096, 3968): "t128x128k2", (404, 1784, 3392): "t128x128k2",
+            (405, 2528, 2496): "t128x128k2", (2320, 580, 3584): "t128x128k2", (151, 2536, 4224): "t128x128k4",
+            (436, 680, 12800): "t128x128k4", (133, 2224, 5888): "t128x128k4", (410, 3824, 1792): "t128x128"}
+    assert {s: gemm_cdna.rule(*s) for s in keep} == keep
+    assert {gemm_cdna.rule(*s, True) for s in ((2618, 744, 14208), (1655, 800, 10368), (1774, 592, 9088))} == {"t128x128k2"}
+    gain = {(1014, 1144, 2496): "t64x128", (581, 2296, 2176): "t64x128", (204, 2536, 3008): "t64x128k2",
+            (1478, 280, 3840): "t64x128k2", (541, 864, 2368): "t64x128k4", (183, 3760, 1280): "t64x128",
+            (437, 864, 2048): "t64x128k4"}
+    assert {s: gemm_cdna.rule(*s) for s in gain} == gain
+
+
 def test_a_shapes_route_is_worked_out_once(monkeypatch):
     """Calls that are not prepared ask the route every time: only the first evaluates the costs,
     and a user's record still answers at once."""
