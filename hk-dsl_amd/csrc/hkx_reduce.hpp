@@ -43,35 +43,21 @@ HKX_DEV f32x4 prog_load(const HkxOperand& o, int m, int n) {
   return ld4(o.ptr, o.dtype, (int64_t)m * o.ld + n);
 }
 
-// A program's registers of one row's four columns, in VGPRs. A number is wave-uniform at run
-// time: it picks by selects over the NR registers the program names (an indexed vector went to
-// scratch memory). A field that is no register number (a LOAD's operand) reads register 0.
-template <int NR>
+// A program's registers of a row's four columns: in LDS, a private 16-byte slot a thread and
+// register (a register's number is known at run time only: an indexed vector goes to scratch
+// memory, and selects over VGPRs cost 8 instructions a register and access).
+template <int NT>
 struct ProgRegs {
-  f32x4 r[NR];
-  HKX_DEV f32x4 get(int i) const {
-    f32x4 v = r[0];
-#pragma unroll
-    for (int k = 1; k < NR; ++k) {
-      const bool is = k == i;
-      v = f32x4{is ? r[k].x : v.x, is ? r[k].y : v.y, is ? r[k].z : v.z, is ? r[k].w : v.w};
-    }
-    return v;
-  }
-  HKX_DEV void set(int i, f32x4 v) {
-#pragma unroll
-    for (int k = 0; k < NR; ++k) {
-      const bool is = k == i;
-      r[k] = f32x4{is ? v.x : r[k].x, is ? v.y : r[k].y, is ? v.z : r[k].z, is ? v.w : r[k].w};
-    }
-  }
+  f32x4* r;  // register 0's slot
+  HKX_DEV f32x4 get(int i) const { return r[i * NT]; }
+  HKX_DEV void set(int i, f32x4 v) { r[i * NT] = v; }
 };
 
 // One instruction on a row's four columns (m, n .. n + 3).
-template <int NR>
-HKX_DEV f32x4 prog_op(const HkxEpilogue& ep, const HkxInstr& I, const ProgRegs<NR>& R, int m, int n, int M) {
+template <int NT>
+HKX_DEV f32x4 prog_op(const HkxEpilogue& ep, const HkxInstr& I, const ProgRegs<NT>& R, int m, int n, int M) {
   {
-    const f32x4 a = R.get(I.a);
+    const f32x4 a = R.get(I.op == HKX_OP_LOAD ? 0 : I.a);  // (a LOAD's a is an operand)
     const f32x4 b = R.get(I.b);
     f32x4 r;
     switch (I.op) {
@@ -199,40 +185,28 @@ __global__ void __launch_bounds__(256) reduce_kernel(const ReduceArgs p) {
   }
 }
 
-// The pass that runs an epilogue program on a sum (or a split's shares). Each thread takes four
-// columns of U rows (blockIdx.y U rows apart), so an instruction is decoded once for U rows and
-// U reads are in flight. It is bound by its memory (4 bytes read a value, 2 written): with the
-// registers in LDS, 64 KB a workgroup left two workgroups a CU and each instruction three LDS
-// round trips, and squared ReLU on 1024 x 12288 took 48 us; in VGPRs it takes 26.
-template <int NR, int U>
-__global__ void __launch_bounds__(256) program_kernel(const ReduceArgs p, const HkxEpilogue ep) {
-  const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
-  if (n >= p.N) return;
-  for (int m = blockIdx.y * U; m < p.M; m += gridDim.y * U) {
-    ProgRegs<NR> R[U];
-    int row[U];
-    f32x4 v[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      row[u] = min(m + u, p.M - 1);  // a row past the end repeats the last, and is not stored
-      v[u] = sum_splits(p.ws + (int64_t)row[u] * p.ws_ld + n, p.splits, p.split_stride);
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-#pragma unroll
-      for (int k = 1; k < NR; ++k) R[u].r[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      R[u].r[0] = v[u];
-    }
+// The pass that runs an epilogue program on a sum (or a split's shares), four columns a thread, with
+// the registers the program names in the launch's LDS (4 KB each). It is bound by its memory (4 bytes
+// read a value, 2 written) where workgroups enough fit a CU to hide the interpreter's chain of LDS
+// and scalar reads; all 16 registers, 64 KB a workgroup, left two a CU. Call times at K = 256, 16
+// registers -> those named: squared ReLU (2 registers) on 512 x 12288 43.3 -> 30.6 us, 11
+// instructions on 4 registers on 700 x 12288 79.9 -> 47.6, 27 on 6 on 512 x 12288 96.6 -> 59.6, a few
+// rows level. Registers in VGPRs, picked by selects, were slower throughout: 0.4 us at 2 registers
+// and few rows, 1.04 times at many, and past 3 registers up to 4.3 times (169 us for 39.4 at 6
+// registers on 512 x 6824); two rows a thread were no faster.
+template <int NT>
+__global__ void __launch_bounds__(NT) program_kernel(const ReduceArgs p, const HkxEpilogue ep) {
+  extern __shared__ f32x4 prog_lds[];
+  const int n = (blockIdx.x * NT + threadIdx.x) * 4;
+  if (n >= p.N) return;  // no barrier follows: each thread's registers are its own
+  ProgRegs<NT> R{prog_lds + threadIdx.x};
+  for (int m = blockIdx.y; m < p.M; m += gridDim.y) {
+    R.set(0, sum_splits(p.ws + (int64_t)m * p.ws_ld + n, p.splits, p.split_stride));
     for (int pc = 0; pc < ep.nins; ++pc) {
       const HkxInstr I = ep.ins[pc];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = prog_op<NR>(ep, I, R[u], row[u], n, p.M);
-#pragma unroll
-      for (int u = 0; u < U; ++u) R[u].set(I.dst, v[u]);
+      R.set(I.dst, prog_op(ep, I, R, m, n, p.M));
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (m + u < p.M) store4(p.c, p.c_dt, (int64_t)(m + u) * p.ldc + n, R[u].get(ep.out_reg));
+    store4(p.c, p.c_dt, (int64_t)m * p.ldc + n, R.get(ep.out_reg));
   }
 }
 
