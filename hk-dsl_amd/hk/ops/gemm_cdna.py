@@ -161,7 +161,7 @@ def _cost(name: str, m: int, n: int, k: int, fp8: bool = False) -> float:
 
 
 @functools.lru_cache(maxsize=8192)
-def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
+def rule(m: int, n: int, k: int, fp8: bool = False, generic: bool = False) -> str:
     """The route when no record or table entry names one: the decode kernel at M <= 32 (bf16);
     else `_steps`, and past 64 rows the tile and split of the least `_cost` where that is 7% or
     more under the steps'.
@@ -183,6 +183,13 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
     6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x 1024 on 64 x 128 ones 8.9 ->
     6.5).
 
+    `generic`: the call's epilogue is one that 256 x 256 tiles run on the ring kernel's generic form
+    (an fp16 or fp32 C, a scale). The cost is fitted to the quadrant kernel's bf16 forms and does not
+    know it: in place of 128 x 256 tiles 256 x 256 ones were up to 1.6 times slower (1248 x 6632 x
+    512 with GELU and an fp32 C 35.4 -> 55.9 us, 746 x 11144 x 7424 with bias and residual 207 -> 248,
+    1671 x 6656 x 256 with SiLU and an fp16 C 27.3 -> 33.0), so they are no candidate then (split
+    ones store plain sums, which the quadrant kernel takes).
+
     The answer depends on the arguments alone and is kept: the costs of a shape take the host
     15-30 us, and a scaled_mm call that is not a prepared one (out, an fp32 sum, a number for a
     scale) asks every time."""
@@ -193,6 +200,7 @@ def rule(m: int, n: int, k: int, fp8: bool = False) -> str:
         return steps
     kunits, least_units = (k // 128, 8) if fp8 else (k // 64, 4)
     out = ("q128",) if fp8 else () if m > 256 and k >= 12288 else ("t256k4", "t256k8")
+    out += ("t256",) * generic
     best = min((c for c, (_, least) in _RULE.items()
                 if c not in out and m >= least and (CANDIDATES[c].get("splits", 1) == 1
                                                     or kunits // CANDIDATES[c]["splits"] >= least_units)),
@@ -209,9 +217,12 @@ def _less(name: str, than: str, m: int, n: int, k: int, fp8: bool = False) -> bo
     for 15.8) and 1.14 to 1.8 times faster to 0.67, at other counts 1.05 to 1.5 times faster at the
     same costs. And unsplit against 128 x 128 tiles split in two they were slower from 0.82 (fp8 2618 x
     744 x 14208 45.4 us for 39.3; at other counts from 0.795, 254 x 7744 x 3072 paired 30.1 for 28.7) and
-    1.07 to 1.18 times faster below."""
+    1.07 to 1.18 times faster below; against 128 x 256 tiles at 0.88 (1728 x 4704 x 1472 with bias and
+    an fp32 C 56.5 for 51.7)."""
     lead = 0.93
-    if than.startswith("t128x128") and name.startswith("t64x128"):
+    if than in ("q128", "t128") and name == "t64x128":
+        lead = 0.81
+    elif than.startswith("t128x128") and name.startswith("t64x128"):
         rows = math.ceil(m / 64)
         whole = rows * math.ceil(n / 128) % 8 == 0
         if not whole and rows in (3, 5, 6, 7):
@@ -251,13 +262,14 @@ def _steps(m: int, n: int, k: int, fp8: bool = False) -> str:
     return f"t{bm}x128" + (f"k{splits}" if splits > 1 else "")
 
 
-def route(m: int, n: int, k: int, fp8: bool = False) -> str:
+def route(m: int, n: int, k: int, fp8: bool = False, generic: bool = False) -> str:
     """The candidate an M x N x K call runs: a user record, else the measured table's
     nearest M (log scale) for this N x K, else `rule` (gemm_cdna.py:969-999). Between two
     measured Ms, 5% or more from the nearer, the rule answers too, past 64 rows up to BETWEEN_M,
     where its cost is 7% or more under the nearest M's pick: there the tiles are few waves and
     that pick may leave a wave nearly empty (300 x 24576 x 4096 109.6 -> 83.2 us). A pick that
-    has no cost class stays (1300 x 24576 x 4096: its 225.5 us, the rule's 234.7)."""
+    has no cost class stays (1300 x 24576 x 4096: its 225.5 us, the rule's 234.7). `generic` as in
+    `rule`."""
     for key in ((m, n, k), "*"):
         if key in OVERRIDE and fits(OVERRIDE[key], m, n, k, fp8):
             return OVERRIDE[key]
@@ -268,12 +280,12 @@ def route(m: int, n: int, k: int, fp8: bool = False) -> str:
             best = min(ms, key=lambda x: abs(math.log(x) - math.log(m)))
             name = ent[str(best)]
             if 64 < m <= BETWEEN_M and abs(math.log(best / m)) >= 0.05 and name in _RULE:
-                other = rule(m, n, k)
+                other = rule(m, n, k, generic=generic)
                 if _less(other, name, m, n, k):
                     return other
             if fits(name, m, n, k, fp8):
                 return name
-    return rule(m, n, k, fp8)
+    return rule(m, n, k, fp8, generic)
 
 
 #: The most rows the 8-bit decode kernel takes.

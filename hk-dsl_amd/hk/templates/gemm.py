@@ -443,14 +443,14 @@ def _sched_record(schedule) -> Dict[str, Any]:
 
 
 def plan(m: int, n: int, k: int, arch: Optional[str] = None, *, schedule=None,
-         fp8: bool = False, epilogue_in_kernel: bool = True) -> List[Step]:
+         fp8: bool = False, epilogue_in_kernel: bool = True, generic: bool = False) -> List[Step]:
     """The launches gemm() makes for an M x N x K problem, in order, and the one that
     carries the epilogue (templates/gemm.py:506-547). Needs no GPU.
 
     Exactly one launch writes each column of C, and it runs the epilogue; a split-K
     plan's shares go to a scratch and a reduction runs the epilogue once on their sum
     -- as does the one-share plan of an epilogue outside the fused form
-    (`epilogue_in_kernel=False`)."""
+    (`epilogue_in_kernel=False`). `generic`: see hk.ops.gemm_cdna.rule."""
     from ..ops import gemm_cdna  # noqa: PLC0415
     from ..target import current_arch  # noqa: PLC0415
 
@@ -462,7 +462,7 @@ def plan(m: int, n: int, k: int, arch: Optional[str] = None, *, schedule=None,
         rec = _sched_record(schedule)
         name = rec.pop("name", "schedule")
     else:
-        name = gemm_cdna.route(m, n, k, fp8=fp8)
+        name = gemm_cdna.route(m, n, k, fp8=fp8, generic=generic)
         rec = dict(gemm_cdna.CANDIDATES[name])
     rec = gemm_cdna.resolve(rec, m, n, k, fp8=fp8)
     kernel = rec["kernel"]
@@ -703,6 +703,18 @@ def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operan
     return go(a, b, out, operands)
 
 
+def _generic(ep: Epilogue, operands: Dict[str, Any], out_dtype) -> bool:
+    """Whether 256 x 256 tiles run this epilogue on the ring kernel's generic form, several times
+    as slow an epilogue as the quadrant kernel's: a fused one that is not act(acc + bias + tile)
+    in bf16, or a C of another 16- or 32-bit type (an 8-bit C's is the same in both)."""
+    torch, c = _torch(), ep.compiled
+    if c.form != "fused" or out_dtype.itemsize == 1:
+        return False
+    return (out_dtype is not torch.bfloat16 or c.cmul != 1.0 or c.cadd != 0.0
+            or bool(c.col_scale or c.row_scale)
+            or any(operands[x].dtype is not torch.bfloat16 for x in (c.row_add, c.tile_add) if x))
+
+
 def _slow(a, b, epilogue, out, out_dtype, operands, schedule=None):
     """Check a call and make its launch: (go, C's shape, C's dtype)
     (templates/gemm.py:770-803)."""
@@ -737,7 +749,7 @@ def _slow(a, b, epilogue, out, out_dtype, operands, schedule=None):
             raise ValueError(f"hk.templates.gemm: operand {name} is on {operands[name].device}, "
                              f"A on {a.device}")
     steps = plan(m, cn if not paired else n, k, schedule=schedule,
-                 epilogue_in_kernel=ep.runs_in_kernel)
+                 epilogue_in_kernel=ep.runs_in_kernel, generic=_generic(ep, operands, tdt))
     if paired:
         for st in steps:
             st.cols = (0, cn)

@@ -259,6 +259,35 @@ def test_rule_keeps_128_row_tiles_where_64_row_ones_were_slower():
     assert {s: gemm_cdna.rule(*s) for s in gain} == gain
 
 
+def test_generic_epilogues_take_no_256_tile_for_its_cost():
+    """256 x 256 tiles run an fp16 or fp32 C's epilogue, or a scaled one, on the ring kernel's generic
+    form: 1248 x 6632 x 512 with GELU and an fp32 C 55.9 us there, 35.4 on 128 x 256 ones; 746 x 11144 x
+    7424 248 against 207."""
+    import torch
+
+    import hk
+
+    T = hk.templates.gemm
+    for s in ((1248, 6632, 512), (1177, 8248, 384), (1671, 6656, 256), (1728, 4704, 1472), (746, 11144, 7424)):
+        assert gemm_cdna.rule(*s) == "t256"
+        assert gemm_cdna.rule(*s, generic=True) == ("t256k2" if s[2] == 7424 else "q128")
+        assert gemm_cdna.route(*s, generic=True) == T.plan(*s, generic=True)[0].route
+    for s in ((2048, 12288, 4096), (4096, 8192, 512)):   # the steps' own large tiles stay
+        assert gemm_cdna.rule(*s, generic=True) == "t256"
+    assert gemm_cdna.rule(577, 8216, 7360, generic=True) == "t256k2"
+
+    def generic(fn, dtype=torch.bfloat16, **ops):
+        return T._generic(T.bind(fn, ops, 4, 8, dtype), ops, dtype)
+
+    b, r = torch.zeros(8).bfloat16(), torch.zeros(4, 8).bfloat16()
+    assert not generic(T.bias_gelu, bias=b) and not generic(T.bias_residual, bias=b, residual=r)
+    assert not generic(T.scale, torch.int8, scale=b.float()) and not generic(lambda acc, ctx: acc, torch.float32)
+    assert not generic(lambda acc, ctx: (acc + ctx.bias) * acc, torch.float32, bias=b)   # a program
+    assert generic(T.bias_gelu, torch.float32, bias=b) and generic(T.bias_silu, torch.float16, bias=b)
+    assert generic(T.scale, scale=b.float()) and generic(T.bias, bias=b.float())
+    assert generic(lambda acc, ctx: acc * 0.5 + ctx.bias, bias=b)
+
+
 def test_a_shapes_route_is_worked_out_once(monkeypatch):
     """Calls that are not prepared ask the route every time: only the first evaluates the costs,
     and a user's record still answers at once."""
