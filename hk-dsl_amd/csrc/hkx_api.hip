@@ -128,9 +128,10 @@ void auto_choose(const HkxGemmArgs* a, int* kernel, int* bm, int* bn, int* split
 hkx::Fused make_fused(const HkxEpilogue& ep);
 
 // Whether HKX_KERNEL_AUTO runs a call on the 8-bit decode kernel: fp8 e4m3, no epilogue or the
-// dequant form, and a shape skinny_wins names.
+// dequant form, no schedule or variant asked for, and a shape skinny_wins names.
 bool auto_skinny(const HkxGemmArgs* a) {
-  return a->kernel == HKX_KERNEL_AUTO && a->ab_dtype == HKX_FP8E4M3 &&
+  return a->kernel == HKX_KERNEL_AUTO && a->tile_schedule == HKX_TILE_AUTO && !a->variant &&
+         a->ab_dtype == HKX_FP8E4M3 &&
          hkx::skinny_wins(a->m, a->n, a->k) &&
          (a->ep.form == HKX_EP_NONE || a->ep.form == HKX_EP_FUSED) && hkx::skinny_ep_ok(make_fused(a->ep));
 }

@@ -201,3 +201,16 @@ def test_the_build_refuses_spills():
     remarks = ("x: remark: Function Name: k1\nx: remark:     ScratchSize [bytes/lane]: 0\n"
                "x: remark: Function Name: k2\nx: remark:     ScratchSize [bytes/lane]: 16\n")
     assert build._spills(remarks) == [("k2", 16)]
+
+
+def test_auto_refuses_what_no_kernel_has_at_decode_sizes_too():
+    """HKX_KERNEL_AUTO of fp8 operands at M <= 32 takes the 8-bit decode kernel; a variant or a schedule
+    that the tile it would pick otherwise does not have is refused as at any other M."""
+    for m in (16, 48):
+        kw = dict(m=m, ab_dtype=nat.FP8E4M3, kernel=nat.KERNEL_AUTO, tile_m=0, tile_n=0)
+        assert _check(_args(**kw)) == (nat.OK, "")
+        rc, msg = _check(_args(variant=64, **kw))
+        assert rc == nat.ERR_ARG and "variant" in msg
+        for sched in (nat.SCHEDULES["pp"], nat.SCHEDULES["ring"], 9):
+            rc, msg = _check(_args(tile_schedule=sched, **kw))
+            assert rc == nat.ERR_ARG, sched
