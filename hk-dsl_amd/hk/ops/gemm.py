@@ -125,7 +125,8 @@ def _run_ready(ready, a, b, scale_a, scale_b, bias):
         raise ValueError("scaled_mm: A and B need unit stride along K")
     import torch  # noqa: PLC0415
 
-    out = nat.empty(a, shape, torch.bfloat16)
+    out = (a.new_empty(shape, dtype=torch.bfloat16) if type(a) is torch.Tensor
+           else nat.empty(a, shape, torch.bfloat16))
     raw = bytearray(raw)
     _POINTERS.pack_into(raw, 0, a.data_ptr(), b.data_ptr(), out.data_ptr(), sa[0], sb[0], shape[1])
     _POINTER.pack_into(raw, _OPS, scale_a.data_ptr())

@@ -70,14 +70,17 @@ def gemm(a, b, sa, sb, out=None):
     n = b.shape[0]
     if k % 128 or n % 8:
         raise ValueError(f"mxfp8.gemm: K={k} a multiple of 128 and N={n} of 8")
-    if not a.is_cuda or b.device != a.device:
+    d = a.get_device()  # (-1 off the GPU; an int's comparison is half a device's 0.15 us)
+    if d < 0 or b.get_device() != d:
         raise ValueError("mxfp8.gemm: a and b are on one GPU")
-    _on(a.device, "mxfp8.gemm", sa=sa, sb=sb, out=out)
+    if sa.get_device() != d or sb.get_device() != d or (out is not None and out.get_device() != d):
+        _on(a.device, "mxfp8.gemm", sa=sa, sb=sb, out=out)
     a, b = _rows16(a), _rows16(b)
     sa = _scales(torch, sa, m, k, "sa")
     sb = _scales(torch, sb, n, k, "sb")
     if out is None:
-        out = nat.empty(a, (m, n), torch.bfloat16)
+        out = (a.new_empty((m, n), dtype=torch.bfloat16) if type(a) is torch.Tensor
+               else nat.empty(a, (m, n), torch.bfloat16))
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (m, n) or out.stride(1) != 1:
         raise ValueError(f"mxfp8.gemm: out is bf16 ({m}, {n}) with unit column stride")
     L = nat.lib()
@@ -109,8 +112,13 @@ def quant(x, out=None):
         _on(x.device, "mxfp8.quant", q=out[0], s=out[1])
     if x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16:
         x = x.contiguous()
-    q, s = out if out is not None else (
-        nat.empty(x, (m, k), torch.float8_e4m3fn), nat.empty(x, (m, k // 32), torch.uint8))
+    if out is not None:
+        q, s = out
+    elif type(x) is torch.Tensor:
+        q = x.new_empty((m, k), dtype=torch.float8_e4m3fn)
+        s = x.new_empty((m, k // 32), dtype=torch.uint8)
+    else:
+        q, s = nat.empty(x, (m, k), torch.float8_e4m3fn), nat.empty(x, (m, k // 32), torch.uint8)
     nat.check(nat.lib().hkx_mx_quant(x.data_ptr(), x.stride(0), q.data_ptr(), q.stride(0),
                                      s.data_ptr(), s.stride(0), m, k,
                                      nat.stream_of(x.device)))
