@@ -216,8 +216,8 @@ __global__ void __launch_bounds__(NW * 64) decode_kernel(const DecodeArgs p) {
 
 // The streaming decode GEMM: one workgroup a CU walks its share of the 16-row blocks of W
 // (a consecutive run of them), for M <= 32 (MF = 1 or 2 16-token fragments; two from
-// K = 2048 up), unpaired, no split, K a multiple of 1024: CPB chunks of 1024 a block
-// (CPB = 1..4), or, with CPB = 0, K / 1024 of them read at run time (K past 4096).
+// K = 2048 up), plain or paired (PAIR, below), no split, K a multiple of 1024: CPB chunks of
+// 1024 a block (CPB = 1..4), or, with CPB = 0, K / 1024 of them read at run time (K past 4096).
 //
 // * W goes HBM -> LDS by non-temporal buffer loads (`buffer_load_dwordx4 ... lds`, read
 //   once, kept out of the caches), each instruction 1 KB

@@ -39,11 +39,12 @@ bool ring_takes(const TileArgs& a, bool fp8, int mode);
 hipError_t launch_ring(const TileArgs& a, bool fp8, int mode, dim3 grid, hipStream_t s);
 hipError_t launch_ring_bf16(const TileArgs& a, int mode, int epf, int act, dim3 grid, hipStream_t s);
 hipError_t launch_ring_fp8(const TileArgs& a, int mode, int epf, int act, dim3 grid, hipStream_t s);
-// The quadrant ring kernel (hkx_quad.hpp): a 16-bit bf16 C, no split; bf16 operands with no
-// epilogue, a bias and an activation, a residual tile, or the paired silu * up form; fp8
-// operands with no epilogue or the dequant forms (row and column fp32 scales, a bf16 bias).
-// Vectors of unit stride, 16-byte aligned. Or, unpaired, a K split's fp32 shares (mode
-// kStoreF32, blockIdx.y the split). quad_takes says which calls.
+// The quadrant ring kernel (hkx_quad.hpp): a bf16 C, no split; bf16 operands with no epilogue, a
+// bias and an activation, a residual tile, or the paired silu * up form; fp8 operands with no
+// epilogue or the dequant forms (row and column fp32 scales, a bf16 bias). Vectors of unit stride,
+// 16-byte aligned. Or mode kStoreF32: unpaired, a K split's fp32 shares (blockIdx.y the split) or
+// one fp32 sum; of fp8 operands also the dequant scales with an fp32 tile added. quad_takes says
+// which calls.
 bool quad_takes(const TileArgs& a, bool fp8, int mode);
 // The quadrant kernel on 128 x 256 tiles (bf16, one phase a K-tile): the calls it takes, and
 // its launch (grid: one workgroup a CU at most).
@@ -70,11 +71,12 @@ hipError_t launch_skinny(SkinnyArgs a, bool mx, int cus, hipStream_t s);
 hipError_t launch_decode(const DecodeArgs& a, int waves, int fn, int mf, int mode, dim3 grid,
                          hipStream_t s);
 
-// The streaming decode kernel (stream_kernel): M <= 16, K a multiple of 1024 up to 32768,
-// no split, plain or paired (M 17-32 from K = 2048).
+// The streaming decode kernel (stream_kernel): M <= 16, or 17-32 from K = 2048, K a multiple of
+// 1024 up to 32768, no split, plain or paired.
 bool stream_takes(const DecodeArgs& a, int splits);
 hipError_t launch_stream(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s);
-// the whole-row decode kernel (K = 4096, M <= 4, N <= 32768), for calls stream_takes accepts
+// the whole-row decode kernel (K = 4096, M <= 4; N <= 32768, at M <= 2 any W under 2 GiB; paired: the
+// same rows of W, at M = 4 up to 8192), for calls stream_takes accepts
 bool rows_takes(const DecodeArgs& a, bool pair);
 hipError_t launch_rows(const DecodeArgs& a, bool pair, dim3 grid, hipStream_t s);
 // the per-wave whole-row decode kernel (K = 1024 with M <= 3, K = 2048 with M <= 2), for calls

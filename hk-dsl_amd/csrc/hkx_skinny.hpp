@@ -1,4 +1,4 @@
-// The 8-bit decode GEMM: C (M <= 32, N) = epilogue(X . W^T), X and W fp8 e4m3, plain (scaled_mm's
+// The 8-bit decode GEMM (hkx_rules.hpp has its rules): C (M <= 32, N) = epilogue(X . W^T), X and W fp8 e4m3, plain (scaled_mm's
 // dequant form) or MX (E8M0 block scales), W read once.
 //
 // At these sizes (2-100 MB of W) the time is latency and HBM, so a workgroup is short and all it

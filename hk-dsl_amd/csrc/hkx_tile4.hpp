@@ -16,7 +16,8 @@
 //   one barrier and spread under the next iteration's k-steps; with three stages they have
 //   one iteration more to land (a wave a SIMD has nothing else to hide their latency with).
 //   RES = 2 is the form of which two workgroups fit a CU (128-column tiles in half the LDS: two
-//   stages at 128 x 128, three at 64 x 128), for grids of more than one a CU.
+//   stages at 128 x 128, three at 64 x 128), for most grids of more than one a CU (tile4_two in
+//   hkx_rules.hpp).
 // * Fragment reads are software-pipelined one k-step ahead (two register sets), and the
 //   reads of the next stage's first k-step are issued under the last k-step's MFMAs.
 // * MFMA: v_mfma_f32_32x32x16_bf16 / v_mfma_f32_32x32x64_f8f6f4 (fp8 e4m3), B's fragment

@@ -149,7 +149,7 @@ def scaled_mm(a, b, scale_a, scale_b, *, bias=None, out=None, accumulate: bool =
 
     * A (M, K) and B (N, K), float8_e4m3fn or float8_e5m2, either pairing (a mixed pair is
       a training backward's gradient against a weight); e4m3 x e4m3 runs on every tile
-      kernel, a pair with e5m2 on the 256 x 256 ring kernel;
+      kernel, a pair with e5m2 on 256 x 256 ring tiles;
     * scale_a one value or one a row of A ((M,) or (M, 1)), scale_b one value or one a row
       of B ((N,) or (1, N)), taken to A's GPU if they are elsewhere; bias (N,);
     * an fp32 `out` (M, N) takes the product unrounded, and with `accumulate=True` it is

@@ -178,10 +178,10 @@ def rule(m: int, n: int, k: int, fp8: bool = False, generic: bool = False) -> st
     1.34 times the steps' rate), so bf16 takes them past 256 rows from K = 12288. Past 64 rows
     the cost still gains there (100 x 20480 x 5120 79.8 -> 59.0, 160 x 8192 x 8192 63.4 -> 43.9).
 
-    fp8 takes the cost from K = 1024 (fitted to 279 shapes of scaled_mm with bias, M 33-4096: the
-    steps were 6.6% slower than the best on average and 1.66x at worst, both together 1%: 1300 x
-    6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x 1024 on 64 x 128 ones 8.9 ->
-    6.5).
+    fp8 takes the cost from K = 1024 (fitted to 279 shapes of scaled_mm with bias, M 33-4096, part of
+    W cached: 1300 x 6144 x 4096 on 256 x 256 tiles 64.4 -> 42.8 us, 900 x 1024 x 1024 on 64 x 128 ones
+    8.9 -> 6.5). With W from memory, 619 other shapes past 64 rows: 1.12 times the steps' rate on
+    average, 0.95 at the least, as much as one kernel's times differ between two processes.
 
     `generic`: the call's epilogue is one that 256 x 256 tiles run on the ring kernel's generic form
     (an fp16 or fp32 C, a scale). The cost is fitted to the quadrant kernel's bf16 forms and does not

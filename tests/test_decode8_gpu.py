@@ -1,5 +1,5 @@
-"""The 8-bit decode kernel (scaled_mm and the MX GEMM at M <= 32) against 64-bit products, at
-its edges: one to 32 tokens, one row block, ragged last blocks of W, K of one 128-byte step
+"""The 8-bit decode kernel (scaled_mm and the MX GEMM at M <= 32, but for long K at 17 and more rows
+and many columns) against 64-bit products, at its edges: one to 32 tokens, one row block, ragged last blocks of W, K of one 128-byte step
 up to several rounds of the workgroup's waves with every kind of remainder.
 
 Bounds: against the 64-bit value the error is half a bf16 unit, up to 2^-8 |ref|, plus what the fp8

@@ -34,11 +34,11 @@ def _operands(m, n, k, seed, block_weight_scales=False):
                                        (4096, 4352, 1152, True), (64, 512, 4224, False),
                                        (16, 1792, 5120, True)])
 def test_mx_gemm_matches_the_scaled_product(m, n, k, blk):
-    """Whole and partial chunks of 8 half-stages of scales (K = 1152: 18 half-stages, its last
-    chunk two), the shortest K (128: a two-half-stage chunk a tile, two tiles a workgroup at
-    4096 x 4352), ragged M; K split over workgroups where the tiles are few (2 splits at
-    2100 x 2048 x 2048, 5 at 16 x 1792 x 5120, 4 of 9, 9, 9 and 6 k-tiles at 64 x 512 x
-    4224), each split's scales read from its own first K block."""
+    """Whole and partial chunks of 4 K units of scales (K = 1152: 9 units, its last chunk one), the
+    shortest K (128: one unit a tile, two 256 x 256 tiles a workgroup at 4096 x 4352), ragged M;
+    the decode kernel (M = 1 and 16), 64 x 128 and 128 x 256 tiles, whole waves of 256 x 256 tiles
+    with a rest (4096 x 4352 x 1152); K split over workgroups (4 of 9, 9, 9 and 6 units at 64 x 512
+    x 4224), each split's scales read from its own first K block."""
     a, b, sa, sb = _operands(m, n, k, seed=m + n + k, block_weight_scales=blk)
     print(f"case mx_gemm {m}x{n}x{k}", flush=True)
     out = mxfp8.gemm(a.to(DEV), b.to(DEV), sa.to(DEV), sb.to(DEV))
@@ -148,9 +148,10 @@ def test_mx_quant_every_code_and_the_special_values():
                                    (512, 4096, 1280), (40, 1024, 8192), (700, 1032, 4224), (1000, 5128, 1152),
                                    (1500, 2304, 2176), (2300, 7688, 640), (4100, 5128, 384)])
 def test_mx_tiles_splits_and_wave_cuts(m, n, k):
-    """The 4-wave tiles' MX form at the plans the shapes pick: one tile and one K unit, ragged
-    rows and columns, unit counts of every remainder by 4 (a scale chunk), K splits, and whole
-    waves of 256 x 256 tiles with the rest of N on smaller ones (the last two)."""
+    """The MX forms at the plans the shapes pick: one 64 x 128 tile and one K unit, ragged rows and
+    columns, unit counts of every remainder by 4 (a scale chunk), K splits of 64 x 128 tiles, 128 x
+    128 and 128 x 256 ones, whole waves of 256 x 256 tiles with the rest of N on 64 x 128 ones (2300
+    x 7688), and 256 x 256 tiles alone (4100 x 5128)."""
     a, b, sa, sb = _operands(m, n, k, seed=m + n + k, block_weight_scales=False)
     out = torch.full((m + 1, n + 8), 7.0, dtype=torch.bfloat16, device=DEV)
     print(f"case mx tiles {m}x{n}x{k}", flush=True)
