@@ -52,16 +52,18 @@ inline int wave_cut(int m, int n, int outw, int cus) {
 // 32-row workgroups are half as many waves, where the blocks' waves are even full ones. Measured at
 // 2000 shapes, K 1024 to 12288, the stream kernel's rate over the blocked one's:
 // * past one to two blocks a CU (one wave of workgroups): K = 1024 0.82-0.98; K = 2048 0.81-1.02
-//   from M = 9, up to M = 8 0.94-1.1 (1.0-1.1 past 3/2 a CU); K = 3072 0.91-1.02 up to M = 8 and at
-//   M 17 to 24, 1.0-1.12 at the others; K = 4096 0.99-1.47; past it X is streamed with every block,
-//   and only the last eighth of the range gains, 0.97-1.21 up to M = 8, 1.02-1.09 to M = 16 from
-//   K = 8192;
+//   from M = 9, up to M = 8 0.94-1.02, 1.0-1.1 past 3/2 a CU; K = 3072 0.91-1.02 up to M = 8 and at M 17
+//   to 24, 1.0-1.12 at the others; just past one a CU the blocked kernel's workgroups leave half the
+//   CUs idle, and up to M = 8 both K gain 1.05-1.2 (260 and 265 blocks); K = 4096 0.99-1.47; past it X is
+//   streamed with every block, and only the last eighth of the range gains, 0.97-1.21 up to M = 8,
+//   1.02-1.09 to M = 16 from K = 8192;
 // * past three to four and five to six: past K = 4096 0.87-1.0 at M 17 to 28 (four) or 26 (six), less
 //   so the more waves; 0.96-1.3 up to M = 16 and 1.0-1.2 past those;
 // * the others 1.0-1.7.
 inline bool pair_streams(int m, int n, int k, int cus) {
   const int blocks = (n + 7) / 8, waves = (blocks + cus - 1) / cus;
   if (waves != 2) return k <= 4096 || m <= 16 || waves % 2 || m > 32 - waves;
+  if (m <= 8 && k >= 2048 && k < 4096 && 16 * blocks <= 17 * cus) return true;
   if (k < 3072) return k >= 2048 && m <= 8 && 2 * blocks > 3 * cus;
   if (k < 4096) return m > 24 || (m > 8 && m <= 16);
   return k == 4096 || (m <= 16 && 4 * blocks > 7 * cus && (m <= 8 || k >= 8192));

@@ -45,7 +45,7 @@ def test_the_blocked_kernel_keeps_the_paired_decode_it_is_faster_at():
                      (1, 5152, 3072), (20, 6000, 3072), (17, 21504, 7168), (19, 12496, 5120), (13, 8080, 5120),
                      (24, 14496, 6144), (28, 16384, 8192), (26, 20800, 5120)):
         assert not rules.pair_streams(m, n2 // 2, k), (m, n2, k)
-    for m, n2, k in ((10, 4096, 1024), (10, 8208, 1024), (32, 4096, 2048), (4, 7000, 2048), (12, 5152, 3072),
+    for m, n2, k in ((10, 4096, 1024), (10, 8208, 1024), (4, 4160, 2048), (8, 4160, 3072), (32, 4096, 2048), (4, 7000, 2048), (12, 5152, 3072),
                      (32, 6000, 3072), (16, 8192, 4096), (4, 8192, 5120), (16, 8192, 8192), (16, 14496, 6144),
                      (17, 10000, 5120), (29, 16384, 8192), (27, 20800, 5120), (16, 24576, 4096), (32, 24576, 4096)):
         assert rules.pair_streams(m, n2 // 2, k), (m, n2, k)
