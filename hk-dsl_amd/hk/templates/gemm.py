@@ -660,6 +660,7 @@ class _Launch:
 #: device is part of it: a hit makes no check, and a host tensor's address is not one the
 #: kernels may read.
 _LAUNCH: Dict[Tuple, Any] = {}
+_TENSOR = None  # torch.Tensor, once a call was made ready
 
 
 def _sig(item):
@@ -698,8 +699,8 @@ def _gemm(a, b, epilogue=None, out=None, out_dtype=None, schedule=None, **operan
     except TypeError:  # an unhashable operand
         got = _slow(a, b, epilogue, out, out_dtype, operands, schedule)
     go, shape, dtype = got
-    if out is None:
-        out = nat.empty(a, shape, dtype)
+    if out is None:  # (in place where A is a plain tensor: 0.1 us of the call's 7)
+        out = a.new_empty(shape, dtype=dtype) if type(a) is _TENSOR else nat.empty(a, shape, dtype)
     return go(a, b, out, operands)
 
 
@@ -718,7 +719,9 @@ def _generic(ep: Epilogue, operands: Dict[str, Any], out_dtype) -> bool:
 def _slow(a, b, epilogue, out, out_dtype, operands, schedule=None):
     """Check a call and make its launch: (go, C's shape, C's dtype)
     (templates/gemm.py:770-803)."""
+    global _TENSOR
     torch = _torch()
+    _TENSOR = torch.Tensor
     if a.dim() != 2 or b.dim() != 2:
         raise ValueError(f"hk.templates.gemm: want A (M, K) and B (N, K), got "
                          f"{tuple(a.shape)} and {tuple(b.shape)}")
